@@ -1,0 +1,66 @@
+"""The aggregation's tiles and the group filter's staged members, bit for
+bit against the oracle at the sizes where they can go wrong: frames of one
+pixel more and less than the 32 x 16 tiles, tiles that meet several crops
+of a tiled reference grid or none, three-channel members whose planes are
+not whole cache lines (k = 5, 6, 7) in one lane batch or several, and the
+unpadded members of the no-allocation scratch."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from vbm3d_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def _bits(a):
+    return np.ascontiguousarray(a, np.float32).view(np.uint32)
+
+
+def _check(V, oracle, ctx, W, H, F, ch, k2, N, nb, sigma=20.0):
+    _, noisy = synth.noisy_clip(W, H, F, ch, sigma, 41)
+    p1, p2 = V.initialize_parameters_1(sigma, N=N), V.initialize_parameters_2(sigma, k=k2, N=N)
+    basic, final = V.denoise(noisy, sigma, True, nb, p1, p2, ctx)
+    ob, of, _ = oracle.run_vbm3d(sigma, noisy, p1, p2, True, nb)
+    np.testing.assert_array_equal(_bits(basic), _bits(ob))
+    np.testing.assert_array_equal(_bits(final), _bits(of))
+
+
+@pytest.mark.parametrize("W,H", [(32, 16), (33, 17), (31, 15), (65, 47)])
+@pytest.mark.parametrize("ch", [1, 3])
+def test_tile_edges(oracle, gpu_ctx, W, H, ch):
+    import vbm3d_amd as V
+    _check(V, oracle, gpu_ctx, W, H, 3, ch, 7, 8, 1)
+
+
+@pytest.mark.parametrize("k2,N", [(4, 8), (5, 8), (6, 16), (7, 1), (7, 16), (8, 16)])
+def test_staged_members(oracle, gpu_ctx, k2, N):
+    import vbm3d_amd as V
+    _check(V, oracle, gpu_ctx, 50, 38, 5, 3, k2, N, 1)
+
+
+@pytest.mark.parametrize("nb", [2, 16, 32])
+def test_crops_of_a_tile(oracle, gpu_ctx, nb):
+    import vbm3d_amd as V
+    _check(V, oracle, gpu_ctx, 330, 190, 2, 3 if nb == 16 else 1, 7, 8, nb)
+
+
+def test_unpadded_members(oracle):
+    import torch
+    import vbm3d_amd as V
+    sigma = 20.0
+    _, noisy = synth.noisy_clip(45, 37, 5, 3, sigma, 42)
+    p1, p2 = V.initialize_parameters_1(sigma), V.initialize_parameters_2(sigma)
+    z = torch.from_numpy(noisy).to("cuda:0")
+    b, f = torch.empty_like(z), torch.empty_like(z)
+    F, ch, H, W = noisy.shape
+    fn = V.lib().vbm3d_run_device_noalloc
+    fn.argtypes = [C.c_float, C.c_void_p, C.c_void_p, C.c_void_p] + [C.c_uint] * 4 + [
+        C.POINTER(V.Parameters), C.POINTER(V.Parameters), C.c_int, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p]
+    torch.cuda.synchronize()
+    assert fn(sigma, z.data_ptr(), None, None, W, H, F, ch, C.byref(p1), C.byref(p2), 1, 1, b.data_ptr(),
+              f.data_ptr(), None) == 0
+    ob, of, _ = oracle.run_vbm3d(sigma, noisy, p1, p2, True, 1)
+    np.testing.assert_array_equal(_bits(b.cpu().numpy()), _bits(ob))
+    np.testing.assert_array_equal(_bits(f.cpu().numpy()), _bits(of))

@@ -533,8 +533,10 @@ int run_step(vbm3d_ctx* ctx, const StepIO& io, hipStream_t s) {
     // the general path's members span kt frames, so the ring keeps kt - 1
     // more frames of reference patches for the aggregation
     const size_t mpos_words = gen && kt > 1 ? (size_t)N * kt : 0;
-    const size_t per_frame = g_arena ? (size_t)nrf * (C * N * K2t + N + 1 + C + mpos_words) * sizeof(float)
-                                     : (size_t)nrf * C * N * K2t * sizeof(float);
+    // the scratch array holds members unpadded, so that it takes the same clips
+    const unsigned ms = gen ? C * K2t : est_words(K, C, !g_arena);
+    const size_t per_frame = g_arena ? (size_t)nrf * (N * ms + N + 1 + C + mpos_words) * sizeof(float)
+                                     : (size_t)nrf * N * ms * sizeof(float);
     const size_t budget = ring_budget(ctx, ctx->est.cap + ctx->idx.cap + ctx->nsx.cap + ctx->wgt.cap);
     size_t cap_frames = std::max<size_t>(1, budget / std::max<size_t>(per_frame, 1));
     unsigned S = (unsigned)std::max<long>(1, (long)cap_frames - 2 * (long)p.Nf - (long)(kt - 1));
@@ -543,12 +545,12 @@ int run_step(vbm3d_ctx* ctx, const StepIO& io, hipStream_t s) {
     unsigned ring = std::min<unsigned>(Fr, S + 2 * p.Nf + (kt - 1));
     if (S >= Fr) { S = Fr; ring = Fr; }
     const size_t slots = (size_t)ring * nrf;
-    // slot * kMaxN + n and the `est` plane index slot * C * N + n are 32-bit
+    // slot * kMaxN + n and the `est` member index slot * N + n are 32-bit
     if ((slots * kMaxN * 3) >> 32) return fail(VBM3D_ERR_UNSUPPORTED, "too many reference patches in flight");
 
     HIP_TRY(ensure(ctx->idx, slots * N * 4));
     HIP_TRY(ensure(ctx->nsx, slots * 4));
-    HIP_TRY(ensure(ctx->est, slots * C * N * K2t * 4));
+    HIP_TRY(ensure(ctx->est, slots * N * ms * 4));
     HIP_TRY(ensure(ctx->wgt, slots * C * 4));
     if (mpos_words) HIP_TRY(ensure(ctx->mpos, slots * mpos_words * 4));
     HIP_TRY(hipMemcpyAsync(ctx->tabs.p, &tabs, sizeof tabs, hipMemcpyHostToDevice, s));
@@ -596,6 +598,7 @@ int run_step(vbm3d_ctx* ctx, const StepIO& io, hipStream_t s) {
     for (int c = 0; c < 3; c++) fa.sig[c] = sig[c];
     fa.tabs = (const Tabs*)ctx->tabs.p;
     fa.est = (float*)ctx->est.p;
+    fa.ms = (int)ms;
     fa.wgt = (float*)ctx->wgt.p;
     fa.gy = io.gy;
     fa.den = io.den;
@@ -610,7 +613,7 @@ int run_step(vbm3d_ctx* ctx, const StepIO& io, hipStream_t s) {
     ag.crop_meta = (const int*)ctx->meta.p;
     ag.grid_pos = (const uint16_t*)ctx->gpos.p;
     ag.idx = bm.idx_out; ag.nsx = bm.nsx_out;
-    ag.est = fa.est; ag.wgt = fa.wgt; ag.tabs = fa.tabs;
+    ag.est = fa.est; ag.ms = (int)ms; ag.wgt = fa.wgt; ag.tabs = fa.tabs;
     ag.R = member_reach(p, io.maxflow, io.W, io.H);
     member_reach_steps(p, io.maxflow, io.W, io.H, &ag.R0, &ag.Rs);
     if (!gen) {
@@ -857,7 +860,7 @@ size_t blob_put(std::vector<char>& blob, const void* p, size_t n) {
 struct Member {
     int clip;
     const vbm3d_params* p;
-    unsigned K, C, N, nrf, Fr, ring = 0, maxflow = 0;
+    unsigned K, C, N, nrf, Fr, ms = 0, ring = 0, maxflow = 0;
     size_t per_frame = 0;  // ring bytes per frame of reference patches
     size_t refxy = 0, meta = 0, gpos = 0, tab = 0;
     int ncrop = 0;
@@ -939,7 +942,8 @@ int plan_batch(vbm3d_ctx* ctx, const vbm3d_clip* clips, int n, int nb, const vbm
                     for (unsigned x : g.cols[q]) h_refxy.push_back(x | (y << 16));
             }
             m.nrf = (unsigned)(h_refxy.size() - m.refxy);
-            m.per_frame = (size_t)m.nrf * (m.C * m.N * m.K * m.K * 4 + m.N * 4 + 4 + m.C * 4);
+            m.ms = est_words(m.K, m.C, true);
+            m.per_frame = (size_t)m.nrf * (m.N * m.ms * 4 + m.N * 4 + 4 + m.C * 4);
             Tabs t;
             fill_tabs(t, m.K);
             m.tab = h_tabs.size();
@@ -986,12 +990,13 @@ int plan_batch(vbm3d_ctx* ctx, const vbm3d_clip* clips, int n, int nb, const vbm
                 m.ring = ring_of(m, S);
                 m.slot_base = sb;
                 m.idx_base = ib;
+                eb = (eb + 31) & ~(size_t)31;  // padded members start on cache lines
                 m.est_base = eb;
                 m.wgt_base = wb;
                 const size_t slots = (size_t)m.ring * m.nrf;
                 sb += slots;
                 ib += slots * m.N;
-                eb += slots * m.C * m.N * m.K * m.K;
+                eb += slots * m.N * m.ms;
                 wb += slots * m.C;
             }
             if (((size_t)sb * kMaxN * 3) >> 32) return fail(VBM3D_ERR_UNSUPPORTED, "too many reference patches in flight");
@@ -1084,6 +1089,7 @@ int plan_batch(vbm3d_ctx* ctx, const vbm3d_clip* clips, int n, int nb, const vbm
                         for (int k = 0; k < 3; k++) fa.sig[k] = sig[k];
                         fa.tabs = d_tabs + m.tab;
                         fa.est = d_est + m.est_base;
+                        fa.ms = (int)m.ms;
                         fa.wgt = d_wgt + m.wgt_base;
                         fa.gy = nullptr; fa.den = nullptr;
                         fa.dW = bm.dW; fa.dWHC = bm.dWHC;
@@ -1113,6 +1119,7 @@ int plan_batch(vbm3d_ctx* ctx, const vbm3d_clip* clips, int n, int nb, const vbm
                         ag.idx = d_idx + m.idx_base;
                         ag.nsx = d_nsx + m.slot_base;
                         ag.est = d_est + m.est_base;
+                        ag.ms = (int)m.ms;
                         ag.wgt = d_wgt + m.wgt_base;
                         ag.tabs = d_tabs + m.tab;
                         ag.R = member_reach(p, m.maxflow, c.W, c.H);

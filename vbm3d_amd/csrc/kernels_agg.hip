@@ -40,28 +40,45 @@ __device__ __forceinline__ int lower_bound_u16(const uint16_t* a, int n, int v) 
 // list, and each wavefront then accumulates, for its 8x8 block, the
 // members that overlap the block in list order: every output sample sees
 // its contributions in exactly the reference's order.
+//
+// What bounds it: with three channels the cache lines of `est` its gathers
+// touch, with one channel instruction issue.  An entry used to be decoded
+// on the scalar unit, 27 scalar and 28 vector instructions; decoded by one
+// lane for 64 entries at once and taken through readlane it costs about 10
+// and 23 (14 with one channel).  Scanning a tile's chunks into one list
+// before any sum leaves the scan's registers out of the sums and one
+// barrier per chunk.  Measured, step 2 and step 1: 30 RGB frames 960x540
+// 3.67 -> 2.94 and 1.10 -> 1.00 ms (the first with the padded members of
+// est_words, 3.59 without); 10 grey frames 176x144 97 -> 57 and 34 -> 23
+// us; 32 grey frames 640x360 1.52 -> 1.00 ms.  With three channels 3, 6 or
+// 8 entries in flight are slower than 4 (3.07, 3.41, 3.04 ms), with one
+// channel 12 or 16 within noise of 8.
 // ONE: the grid is a single crop (nb = 1); the per-crop sums are then the
 // totals, and no crop-order merge is kept live across the scan.
 template <int C, bool RAW, int NM, bool ONE, class A>
 __device__ __forceinline__ void agg_tile(const A& a, const int bx, const int by, const unsigned bz, const int nl) {
-    typedef const __attribute__((address_space(4))) float cfloat;
     constexpr int TX = kAggTileX, TY = kAggTileY, NT = kAggThreads;
     constexpr int QS = 8;             // a wavefront's block edge
     constexpr int NWV = NT / 64, WX = TX / QS;
+    constexpr int U = C == 1 ? 8 : 4;  // entries whose loads are in flight together
     static_assert(TX % QS == 0 && TY % QS == 0 && NT % 64 == 0, "tile of 8x8 blocks");
-    // the ordered list of one NT-patch chunk (at most nl >= N members
-    // each): entry = {position x | y << 16, slot * kMaxN + n}, one 8-byte
-    // LDS read per entry
+    static_assert(TX + kMaxK - 1 <= 64 && TY + kMaxK - 1 <= 32 && NT * kMaxN <= 65536, "list entry fields");
+    // the ordered list of members that overlap the tile: {member n (4
+    // bits), its column + K - 1 and row + K - 1 in the tile (6, 5 bits);
+    // slot}.  It holds what one NT-patch chunk can bring (nl >= N members
+    // each), in practice the whole tile's members.
     extern __shared__ uint2 agg_lists[];
     uint2* L_e = agg_lists;
+    const int cap = NT * nl;
+    __shared__ uint16_t s_pick[NWV][128];  // per wavefront: entries overlapping its block, not yet summed
     __shared__ float s_kai[kMaxWin * kMaxWin * 4];
-    __shared__ int s_w[NWV];
+    __shared__ int s_w[2][NWV];
     const int tid = threadIdx.x;
     const int lane = tid & 63, wv = tid >> 6;
     const int x0 = bx * TX, y0 = by * TY;
     const unsigned to = a.t_begin + bz;
-    const int qx0 = x0 + (wv % WX) * QS, qy0 = y0 + (wv / WX) * QS;  // this wave's block
-    const int px = qx0 + (lane & (QS - 1)), py = qy0 + lane / QS;
+    const int qx0 = (wv % WX) * QS, qy0 = (wv / WX) * QS;  // this wave's block in the tile
+    const int px = x0 + qx0 + (lane & (QS - 1)), py = y0 + qy0 + lane / QS;
     const bool inside = px < (int)a.W && py < (int)a.H;
     const int K = a.K, K2 = K * K, N = a.N;
     const unsigned W = a.W, wh = a.wh, whc = a.whc;
@@ -76,6 +93,16 @@ __device__ __forceinline__ void agg_tile(const A& a, const int bx, const int by,
     const unsigned tbase = to * whc;
     const Div32 dW = {a.divW.m, a.divW.s1, a.divW.s2};
     const unsigned rmin = (unsigned)max(0, y0 - K + 1) * W, rmax = (unsigned)min((int)a.H, y0 + TY) * W;
+    // packed pairs of 16 bits (x low, y high): the lane's pixel in list
+    // entry coordinates, the patch's last sample, and the bytes of a
+    // sample's column and row
+    typedef short short2v __attribute__((ext_vector_type(2)));
+    typedef unsigned short ushort2v __attribute__((ext_vector_type(2)));
+    const short2v lpos = {(short)(qx0 + (lane & (QS - 1)) + K - 1), (short)(qy0 + lane / QS + K - 1)};
+    const short2v kmax = {(short)(K - 1), (short)(K - 1)}, zero = {0, 0};
+    typedef const __attribute__((address_space(1))) char gchar;
+    typedef const __attribute__((address_space(1))) float gfloat;
+    const ushort2v kstr = {4, (unsigned short)(4 * K)};
 
     // per frame of a crop's box: {first index, columns, first row, first
     // column} of the grid patches whose members can reach the tile, and the
@@ -85,7 +112,37 @@ __device__ __forceinline__ void agg_tile(const A& a, const int bx, const int by,
     __shared__ Div32 s_div[2 * kGenMaxNf + 1];
     __shared__ int s_total;
 
-    for (int ci = 0; ci < (ONE ? 1 : a.ncrop); ci++) {
+    // The crops that hold a patch whose members can reach the tile, from
+    // the widest box (frame distance Nf): a tile meets one crop, at the
+    // seams up to four, and a crop without patches adds nothing.  (16 grey
+    // frames 1280x720 on 16 crops, visiting only these: step 2 and step 1
+    // 2.52 -> 1.54 and 1.65 -> 0.98 ms with the rest of this kernel.)
+    uint32_t crops = 1u;
+    if (!ONE) {
+        __shared__ int s_any[2 * kMaxCrops];
+        const int Rk = (int)min((long)a.R, (long)a.R0 + (long)a.Nf * a.Rs);
+        for (int q = tid; q < 2 * a.ncrop; q += NT) {
+            const int ci = q >> 1, col = q & 1;
+            int lo, hi;
+            if (a.boxtab) {
+                const int4 v = a.boxtab[((size_t)ci * (a.nty + a.ntx) + (col ? a.nty + bx : by)) * (a.Nf + 1) + a.Nf];
+                lo = v.x;
+                hi = v.y;
+            } else {
+                const int* meta = a.crop_meta + ci * 5;
+                const uint16_t* g = a.grid_pos + meta[3 + col];
+                const int b0 = (col ? x0 : y0) - Rk - (K - 1), b1 = (col ? x0 + TX : y0 + TY) + Rk;
+                lo = lower_bound_u16(g, meta[1 + col], b0);
+                hi = lower_bound_u16(g, meta[1 + col], b1);
+            }
+            s_any[q] = hi > lo;
+        }
+        __syncthreads();
+        crops = (uint32_t)__ballot(lane < a.ncrop && s_any[2 * (lane & (kMaxCrops - 1))] && s_any[2 * (lane & (kMaxCrops - 1)) + 1]);
+    }
+
+    for (; crops; crops &= crops - 1) {
+        const int ci = ONE ? 0 : __builtin_ctz(crops);
         const int* meta = a.crop_meta + ci * 5;
         const int off = meta[0], nrows = meta[1], ncols = meta[2];
         const uint16_t* rows = a.grid_pos + meta[3];
@@ -155,17 +212,16 @@ __device__ __forceinline__ void agg_tile(const A& a, const int bx, const int by,
 #pragma unroll
         for (int c = 0; c < C; c++) pn[c] = pd[c] = 0.f;
 
-        // The scan data of a chunk (slot, group size, member indices, up
-        // to NM >= N of them) is loaded one chunk ahead: the loads for chunk
-        // cb + NT fly while chunk cb is accumulated.
-        uint32_t slot_n = 0, mi_n[NM];
-        int ns_n = 0;
+        // The scan data of a chunk: slot, group size, member indices (up to
+        // NM >= N of them).
+        uint32_t slot = 0, mi[NM];
+        int ns = 0;
         auto fetch = [&](long cb) {
             const unsigned e = (unsigned)(cb + tid);
-            slot_n = 0;
-            ns_n = 0;
+            slot = 0;
+            ns = 0;
 #pragma unroll
-            for (int n = 0; n < NM; n++) mi_n[n] = 0u;
+            for (int n = 0; n < NM; n++) mi[n] = 0u;
             if (e < total) {
                 // the frame whose box holds index e: the last one starting
                 // at or before it (empty boxes start where the next does)
@@ -178,135 +234,155 @@ __device__ __forceinline__ void agg_tile(const A& a, const int bx, const int by,
                 const unsigned rest = e - (unsigned)bx.x;
                 const unsigned ii = div32(rest, dq), jj = rest - ii * (unsigned)bx.y;
                 const unsigned tr = trlo + q;
-                slot_n = (tr % a.ring) * a.nrf + off + (bx.z + ii) * ncols + (bx.w + jj);
-                ns_n = (int)a.nsx[slot_n];
-                const uint32_t* mem = a.idx + (size_t)slot_n * N;
+                slot = (tr % a.ring) * a.nrf + off + (bx.z + ii) * ncols + (bx.w + jj);
+                ns = (int)a.nsx[slot];
+                const uint32_t* mem = a.idx + (size_t)slot * N;
 #pragma unroll
-                for (int n = 0; n < NM; n++) mi_n[n] = n < N ? mem[n] : 0u;
+                for (int n = 0; n < NM; n++) mi[n] = n < N ? mem[n] : 0u;
             }
         };
-        if (total > 0) fetch(0);
-        for (long cb = 0; cb < total; cb += NT) {
-            const uint32_t slot = slot_n;
-            const int ns = ns_n;
-            uint32_t mi[NM];
+        // Sums the first `cnt` <= 64 entries of this wavefront's pick list,
+        // in order.  Lane q decodes entry q -- position, est address,
+        // weights -- for all of them at once; the entries then go one after
+        // the other through readlane into scalar registers, so that an
+        // entry costs neither scalar decoding nor a dependent load.
+        const uint64_t cstr = (uint64_t)(unsigned)(K2 * 4);  // bytes from one channel's plane to the next
+        auto sum_picks = [&](int cnt) {
+            const uint2 ent = L_e[s_pick[wv][lane < cnt ? lane : 0]];
+            float ew[RAW ? 1 : C];
+            if (!RAW)
 #pragma unroll
-            for (int n = 0; n < NM; n++) mi[n] = mi_n[n];
-            uint32_t hits = 0;
+                for (int c = 0; c < C; c++) ew[c] = a.wgt[(size_t)ent.y * C + c];
+            const uint32_t epos = ((ent.x >> 4) & 63u) | ((ent.x >> 10) << 16);
+            // the member index slot * N + n fits 32 bits (the host refuses
+            // larger rings)
+            const uint32_t pl = ent.y * (unsigned)N + (ent.x & 15u);
+            const uint64_t eb = (uint64_t)a.est + (uint64_t)pl * (unsigned)(a.ms * 4);
+            const uint32_t elo = (uint32_t)eb, ehi = (uint32_t)(eb >> 32);
+            for (int j0 = 0; j0 < cnt; j0 += U) {
+                // U entries at a time: every load is issued before the first
+                // sum.  Straight-line loads: an absent entry repeats the
+                // last one, a lane outside a patch reads the patch's sample
+                // nearest to it (within the rows and columns the patch's own
+                // lanes read, so no extra cache line); only the sums below
+                // are masked
+                float ev[U][C], kai[U];
+                bool on[U];
 #pragma unroll
-            for (int n = 0; n < NM; n++) {
-                if (n >= ns) break;
-                const unsigned r = mi[n] - tbase;
-                if (r < rmin || r >= rmax) continue;
-                const int qy = (int)div32(r, dW), qx = (int)(r - (unsigned)qy * W);
-                if (qx <= x0 + TX - 1 && qx + K - 1 >= x0) hits |= 1u << n;
-            }
-            // ordered compaction: exclusive block scan of the hit counts
-            const int cnt = __popc(hits);
-            int x = cnt;
+                for (int u = 0; u < U; u++) {
+                    const int j = min(j0 + u, cnt - 1);
+                    const uint32_t pos = __builtin_amdgcn_readlane(epos, j);
+                    const uint64_t b = (uint64_t)(uint32_t)__builtin_amdgcn_readlane(elo, j) |
+                                       ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(ehi, j) << 32);
+                    const short2v d = lpos - __builtin_bit_cast(short2v, pos);
+                    const short2v cl = __builtin_elementwise_min(__builtin_elementwise_max(d, zero), kmax);
+                    on[u] = (j0 + u < cnt) & (__builtin_bit_cast(uint32_t, d) == __builtin_bit_cast(uint32_t, cl));
+                    const uint32_t ko = __builtin_amdgcn_udot2(__builtin_bit_cast(ushort2v, cl), kstr, 0u, false);
+                    kai[u] = *(const float*)((const char*)s_kai + ko);
 #pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int y = __shfl_up(x, o, 64);
-                if (lane >= o) x += y;
-            }
-            if (lane == 63) s_w[wv] = x;
-            __syncthreads();
-            int base = 0, tot = 0;
-#pragma unroll 1
-            for (int q = 0; q < NWV; q++) {
-                const int sq = s_w[q];
-                base += q < wv ? sq : 0;
-                tot += sq;
-            }
-            int o = base + x - cnt;
-#pragma unroll
-            for (int n = 0; n < NM; n++)
-                if ((hits >> n) & 1u) {
-                    const unsigned r = mi[n] - tbase;
-                    const unsigned qy = div32(r, dW), qx = r - qy * W;
-                    L_e[o] = make_uint2(qx | (qy << 16), slot * kMaxN + n);
-                    o++;
+                    for (int c = 0; c < C; c++) ev[u][c] = *(const gfloat*)((const gchar*)(b + c * cstr) + ko);
                 }
-            __syncthreads();
-            if (cb + NT < total) fetch(cb + NT);
-            // this wave: the list entries overlapping its 8x8 block, in order
-            for (int j0 = 0; j0 < tot; j0 += 64) {
-                bool ov = false;
-                if (j0 + lane < tot) {
-                    const uint32_t pos = L_e[j0 + lane].x;
-                    const int ex = (int)(pos & 0xFFFFu), ey = (int)(pos >> 16);
-                    ov = ex <= qx0 + QS - 1 && ex + K - 1 >= qx0 && ey <= qy0 + QS - 1 && ey + K - 1 >= qy0;
-                }
-                uint64_t m = __ballot(ov);
-                while (m) {
-                    // up to 4 entries at a time: every load is issued before
-                    // the first sum, and the sums then run in list order.
-                    // The entry is the same for every lane: its position,
-                    // slot and member are decoded on the scalar unit, its
-                    // weights arrive through scalar loads.
-                    constexpr int U = 4;
-                    int jj[U];
+                // keeps the loads above from being sunk to their sums
+                asm volatile("" ::: "memory");
 #pragma unroll
-                    for (int u = 0; u < U; u++) {
-                        jj[u] = m ? j0 + (int)__builtin_ctzll(m) : -1;
-                        m &= m - 1;
-                    }
-                    // straight-line loads: an absent entry repeats the
-                    // first one, a lane outside a patch reads the patch's
-                    // sample nearest to it (within the rows and columns the
-                    // patch's own lanes read, so no extra cache line); only
-                    // the sums below are masked
-                    float ev[U][C], kai[U], w[U][C];
-                    bool on[U];
-#pragma unroll
-                    for (int u = 0; u < U; u++) {
-                        const int jv = jj[u] >= 0 ? jj[u] : jj[0];
-                        const uint2 ent = L_e[jv];
-                        const uint32_t pos = __builtin_amdgcn_readfirstlane(ent.x);
-                        const uint32_t sn = __builtin_amdgcn_readfirstlane(ent.y);
-                        const uint32_t sl = sn / kMaxN, n = sn % kMaxN;
-                        const cfloat* wb = (const cfloat*)(a.wgt + (size_t)sl * C);
-#pragma unroll
-                        for (int c = 0; c < C; c++) w[u][c] = RAW ? 0.f : wb[c];
-                        const int dx = px - (int)(pos & 0xFFFFu), dy = py - (int)(pos >> 16);
-                        on[u] = (jj[u] >= 0) & inside & ((unsigned)dx < (unsigned)K) & ((unsigned)dy < (unsigned)K);
-                        // clamp to [0, K-1] in one instruction per axis
-                        int cx, cy;
-                        asm("v_med3_i32 %0, %1, 0, %2" : "=v"(cx) : "v"(dx), "s"(K - 1));
-                        asm("v_med3_i32 %0, %1, 0, %2" : "=v"(cy) : "v"(dy), "s"(K - 1));
-                        const unsigned kk = __umul24((unsigned)cy, (unsigned)K) + (unsigned)cx;
-                        kai[u] = s_kai[kk];
-                        // wave-uniform base, 32-bit lane byte offset; the
-                        // plane index slot * C * N + n fits 32 bits (the
-                        // host refuses larger rings)
-                        const unsigned pl = sl * (unsigned)(C * N) + n;
-                        const char* eb = (const char*)a.est + (size_t)pl * (unsigned)(K2 * 4);
+                for (int u = 0; u < U; u++) {
+                    float w[RAW ? 1 : C];
+                    if (!RAW)
 #pragma unroll
                         for (int c = 0; c < C; c++)
-                            ev[u][c] = *(const float*)(eb + (size_t)c * N * K2 * 4 + kk * 4u);
-                    }
-                    // keeps the loads above from being sunk to their sums
-                    // (the weights' scalar loads included)
+                            w[c] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ew[c]), min(j0 + u, cnt - 1)));
+                    if (!on[u]) continue;
 #pragma unroll
-                    for (int u = 0; u < U; u++)
-#pragma unroll
-                        for (int c = 0; c < C; c++) asm volatile("" ::"s"(w[u][c]));
-                    asm volatile("" ::: "memory");
-#pragma unroll
-                    for (int u = 0; u < U; u++) {
-                        if (!on[u]) continue;
-#pragma unroll
-                        for (int c = 0; c < C; c++) {
-                            if (RAW) {
-                                pn[c] = pn[c] + ev[u][c];
-                            } else {
-                                const float kw = kai[u] * w[u][c];
-                                pn[c] = pn[c] + kw * ev[u][c];
-                                pd[c] = pd[c] + kw;
-                            }
+                    for (int c = 0; c < C; c++) {
+                        if (RAW) {
+                            pn[c] = pn[c] + ev[u][c];
+                        } else {
+                            const float kw = kai[u] * w[c];
+                            pn[c] = pn[c] + kw * ev[u][c];
+                            pd[c] = pd[c] + kw;
                         }
                     }
                 }
+            }
+        };
+        long cb = 0;
+        while (cb < total) {
+            // Scan: chunks are appended to the list until they are all in
+            // or the next one does not fit (it is scanned again after the
+            // sums below; an empty list takes any chunk).  The loads of
+            // chunk cb + NT fly while chunk cb is listed.
+            int len = 0;
+            fetch(cb);
+            while (cb < total) {
+                uint32_t hits = 0;
+#pragma unroll
+                for (int n = 0; n < NM; n++) {
+                    if (n >= ns) break;
+                    const unsigned r = mi[n] - tbase;
+                    if (r < rmin || r >= rmax) continue;
+                    const int qy = (int)div32(r, dW), qx = (int)(r - (unsigned)qy * W);
+                    if (qx <= x0 + TX - 1 && qx + K - 1 >= x0) hits |= 1u << n;
+                }
+                // ordered compaction: exclusive block scan of the hit counts
+                const int cnt = __popc(hits);
+                int x = cnt;
+#pragma unroll
+                for (int o = 1; o < 64; o <<= 1) {
+                    const int y = __shfl_up(x, o, 64);
+                    if (lane >= o) x += y;
+                }
+                const int par = (int)(cb / NT) & 1;  // alternate, so that one barrier a chunk is enough
+                if (lane == 63) s_w[par][wv] = x;
+                __syncthreads();
+                int base = 0, tot = 0;
+#pragma unroll 1
+                for (int q = 0; q < NWV; q++) {
+                    const int sq = s_w[par][q];
+                    base += q < wv ? sq : 0;
+                    tot += sq;
+                }
+                if (len + tot > cap) break;  // workgroup-uniform
+                const uint32_t sl = slot;
+                uint32_t m2[NM];
+#pragma unroll
+                for (int n = 0; n < NM; n++) m2[n] = mi[n];
+                cb += NT;
+                if (cb < total) fetch(cb);
+                int o = len + base + x - cnt;
+#pragma unroll
+                for (int n = 0; n < NM; n++)
+                    if ((hits >> n) & 1u) {
+                        const unsigned r = m2[n] - tbase;
+                        const unsigned qy = div32(r, dW), qx = r - qy * W;
+                        L_e[o] = make_uint2((unsigned)n | ((qx + K - 1 - x0) << 4) | ((qy + K - 1 - y0) << 10), sl);
+                        o++;
+                    }
+                len += tot;
+            }
+            __syncthreads();
+            // Sums: this wave takes the list entries overlapping its 8x8
+            // block, in order, 64 at a time.
+            int np = 0, j0 = 0;
+            for (;;) {
+                while (np < 64 && j0 < len) {
+                    bool ov = false;
+                    if (j0 + lane < len) {
+                        const uint32_t ent = L_e[j0 + lane].x;
+                        // block-relative corner + K - 1 in [0, QS + K - 2]
+                        const unsigned ex = ((ent >> 4) & 63u) - (unsigned)qx0, ey = (ent >> 10) - (unsigned)qy0;
+                        ov = ex <= (unsigned)(QS + K - 2) && ey <= (unsigned)(QS + K - 2);
+                    }
+                    const uint64_t m = __ballot(ov);
+                    if (ov) s_pick[wv][np + lanes_below(m, lane)] = (uint16_t)(j0 + lane);
+                    np += __popcll(m);
+                    j0 += 64;
+                }
+                if (np == 0) break;
+                wave_sync();
+                sum_picks(min(np, 64));
+                if (np > 64) s_pick[wv][lane] = s_pick[wv][64 + lane];
+                np = max(np - 64, 0);
+                wave_sync();
             }
             __syncthreads();
         }
@@ -332,13 +408,12 @@ __device__ __forceinline__ void agg_tile(const A& a, const int bx, const int by,
     }
 }
 
-// Occupancy floor of 8 waves per SIMD (64 registers, two of them spilled):
-// the kernel waits on memory more than it computes, and measured faster
-// than at its unconstrained 7 waves.
-template <int C, bool RAW, int NM>
+// Occupancy floor of 8 waves per SIMD (64 registers): the kernel waits on
+// memory more than it computes (6 waves with twice the entries in flight:
+// 3.04 against 2.94 ms).
+template <int C, bool RAW, int NM, bool ONE>
 __global__ __launch_bounds__(kAggThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_aggregate(AArgs a) {
-    if (a.ncrop == 1) agg_tile<C, RAW, NM, true>(a, blockIdx.x, blockIdx.y, blockIdx.z, a.N);
-    else agg_tile<C, RAW, NM, false>(a, blockIdx.x, blockIdx.y, blockIdx.z, a.N);
+    agg_tile<C, RAW, NM, ONE>(a, blockIdx.x, blockIdx.y, blockIdx.z, a.N);
 }
 
 // Batched form with one workgroup per tile: workgroup b takes item b, so
@@ -494,16 +569,22 @@ hipError_t launch_aggregate(int C, const AArgs& a, unsigned frames, hipStream_t 
     if (frames == 0) return hipSuccess;
     dim3 grid((a.W + kAggTileX - 1) / kAggTileX, (a.H + kAggTileY - 1) / kAggTileY, frames);
     if (a.N < 1 || a.N > kMaxN) return hipErrorInvalidValue;
-    const size_t lds = (size_t)kAggThreads * a.N * sizeof(uint2);  // the chunk's ordered list
+    const size_t lds = (size_t)kAggThreads * a.N * sizeof(uint2);  // the tile's ordered list
     const dim3 blk(kAggThreads);
     // members held in registers by the scan: 8, or 16 for N = 16
-#define VB_AGG(NM)                                                                         \
-    if (a.raw) {                                                                           \
-        if (C == 1) hipLaunchKernelGGL((k_aggregate<1, true, NM>), grid, blk, lds, s, a);  \
-        else hipLaunchKernelGGL((k_aggregate<3, true, NM>), grid, blk, lds, s, a);         \
-    } else {                                                                               \
-        if (C == 1) hipLaunchKernelGGL((k_aggregate<1, false, NM>), grid, blk, lds, s, a); \
-        else hipLaunchKernelGGL((k_aggregate<3, false, NM>), grid, blk, lds, s, a);        \
+#define VB_AGG1(NM, ONE)                                                                        \
+    if (a.raw) {                                                                                \
+        if (C == 1) hipLaunchKernelGGL((k_aggregate<1, true, NM, ONE>), grid, blk, lds, s, a);  \
+        else hipLaunchKernelGGL((k_aggregate<3, true, NM, ONE>), grid, blk, lds, s, a);         \
+    } else {                                                                                    \
+        if (C == 1) hipLaunchKernelGGL((k_aggregate<1, false, NM, ONE>), grid, blk, lds, s, a); \
+        else hipLaunchKernelGGL((k_aggregate<3, false, NM, ONE>), grid, blk, lds, s, a);        \
+    }
+#define VB_AGG(NM)               \
+    if (a.ncrop == 1) {          \
+        VB_AGG1(NM, true)        \
+    } else {                     \
+        VB_AGG1(NM, false)       \
     }
     if (a.N <= 8) {
         VB_AGG(8)
@@ -511,6 +592,7 @@ hipError_t launch_aggregate(int C, const AArgs& a, unsigned frames, hipStream_t 
         VB_AGG(16)
     }
 #undef VB_AGG
+#undef VB_AGG1
     return hipGetLastError();
 }
 

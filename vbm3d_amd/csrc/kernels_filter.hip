@@ -122,11 +122,21 @@ __device__ __forceinline__ float wiener_sum(const float* vc) {
 // Per-wavefront LDS layout of k_filter (4-byte words): transposes, zg,
 // eg, then one v^2 buffer per channel, each region 16-byte aligned.
 __host__ __device__ constexpr int round4(int v) { return (v + 3) & ~3; }
+// Whether the filtered members of a group leave through one staged copy
+// (filter_one): three channels whose planes are not whole cache lines.
+__host__ __device__ constexpr bool stage_est(int K, int C, int step) { return step == 2 && C == 3 && (K * K) % 32 != 0; }
+// Words from one staged member to the next: the padded member, and 4 more
+// so that the members' stores fall in different LDS banks.
+__host__ __device__ constexpr int stage_pitch(int K, int C) { return (C * K * K + 31) / 32 * 32 + 4; }
+// Words before the v^2 buffers: transposes, zg and eg, over which the
+// staged members go.
+__host__ __device__ constexpr int filter_front(int K, int C, int N, int step) {
+    const int w = round4((64 / K) * xstride(K)) + (step == 2 ? 2 : 1) * round4(N * K * K);
+    const int st = stage_est(K, C, step) ? (N < 64 / K ? N : 64 / K) * stage_pitch(K, C) : 0;
+    return w > st ? w : st;
+}
 __host__ __device__ inline int filter_lds_words(int K, int C, int N, int step) {
-    const int pb = 64 / K;
-    int w = round4(pb * xstride(K)) + round4(N * K * K);
-    if (step == 2) w += round4(N * K * K) + C * round4(K * K * N);
-    return w;
+    return filter_front(K, C, N, step) + (step == 2 ? C * round4(K * K * N) : 0);
 }
 
 // Channel sigma without a dynamically indexed array (a private array
@@ -145,7 +155,7 @@ __device__ __forceinline__ void filter_one(const A& a, const long r, float* X, c
     const int gw = round4(a.N * K2);               // group buffer words
     float* zg = X + round4(PB * XS);               // [N][K2]
     float* eg = zg + gw;                           // [N][K2] (step 2)
-    float* v2 = eg + gw;                           // [C][gw] (step 2)
+    float* v2 = X + filter_front(K, C, a.N, STEP);  // [C][gw] (step 2)
     const unsigned t = (unsigned)(r / a.nrf), i = (unsigned)(r - (long)t * a.nrf);
     const unsigned slot = __builtin_amdgcn_readfirstlane((t % a.ring) * a.nrf + i);
     const unsigned W = a.W, wh = a.wh, whc = a.whc;
@@ -162,6 +172,13 @@ __device__ __forceinline__ void filter_one(const A& a, const long r, float* X, c
     const float dct_out = a.tabs->dct_out;
     const int nl = lane / K, rr = lane - nl * K;    // batch patch, row / column index
     const bool lact = lane < PB * K;
+    // Staged members: the outputs of channels 0 and 1 stay in registers until
+    // the group's members go out together, each padded to whole cache lines
+    // (a member in one lane batch; the unpadded ring of the scratch array
+    // takes the plain stores).
+    constexpr bool STG = stage_est(K, C, STEP);
+    const bool stg = STG && nsx <= PB && a.ms == stage_pitch(K, C) - 4;
+    float held[STG ? C - 1 : 1][K];
     float wsel = 0.f;  // step 1: lane c ends with channel c's weight
     // mb0: offset of row rr of member nl, the lane's row in the first lane
     // batch (its index is read whether or not the member exists, so that
@@ -268,8 +285,12 @@ __device__ __forceinline__ void filter_one(const A& a, const long r, float* X, c
         //      A member's outputs replace its coefficients in LDS (pass 1
         //      of its batch has read them all), and the group's planes then
         //      leave in contiguous 256-byte stores.
+        //      Three channels of 7x7 planes are not whole cache lines: there
+        //      the members are staged (held, stage_est) and leave in 16-byte
+        //      stores of whole lines, so that the aggregation reads 5 lines
+        //      per member instead of the 7.5 of separate planes.
         float* est = STEP == 2 ? eg : zg;
-        float* dstg = a.est + (((size_t)slot * C + c) * a.N) * K2;
+        float* dstg = a.est + (size_t)slot * (unsigned)(a.N * a.ms) + c * K2;
         for (int nb0 = 0; nb0 < nsx; nb0 += PB) {
             const int n = nb0 + nl;
             const bool act = lact && n < nsx;
@@ -311,13 +332,48 @@ __device__ __forceinline__ void filter_one(const A& a, const long r, float* X, c
                 } else {
                     float y[K];
                     dct_inv_pass<K>(col, y, TI);
+                    if (stg) {
+                        if (c == C - 1) {
+                            // X and the group buffers are no longer read
+                            // (one lane batch: col is in registers)
+                            wave_sync();
 #pragma unroll
-                    for (int u = 0; u < K; u++) est[n * K2 + u * K + rr] = dct_out * y[u];
+                            for (int u = 0; u < K; u++) {
+                                float* m = X + n * stage_pitch(K, C) + u * K + rr;
+#pragma unroll
+                                for (int h = 0; h < C - 1; h++) m[h * K2] = held[STG ? h : 0][u];
+                                m[(C - 1) * K2] = dct_out * y[u];
+                            }
+                        } else {
+#pragma unroll
+                            for (int u = 0; u < K; u++) {
+                                const float o = dct_out * y[u];
+                                if (c == 0) held[0][u] = o;
+                                else held[STG ? 1 : 0][u] = o;
+                            }
+                        }
+                    } else {
+#pragma unroll
+                        for (int u = 0; u < K; u++) est[n * K2 + u * K + rr] = dct_out * y[u];
+                    }
                 }
             }
             wave_sync();
         }
-        for (int j = lane; j < nsx * K2; j += 64) dstg[j] = est[j];
+        if (stg) {
+            if (c < C - 1) continue;
+            constexpr int M4 = (stage_pitch(K, C) - 4) / 4;  // 16-byte pieces of a member
+            float4* g4 = (float4*)(a.est + (size_t)slot * (unsigned)(a.N * a.ms));
+            for (int j = lane; j < nsx * M4; j += 64) {
+                const int n = j / M4;
+                g4[j] = *(const float4*)(X + n * stage_pitch(K, C) + 4 * (j - n * M4));
+            }
+            continue;
+        }
+        for (int j = lane; j < nsx * K2; j += 64) {
+            const int n = j / K2;
+            dstg[n * a.ms + (j - n * K2)] = est[j];
+        }
         wave_sync();  // read before the next channel's transforms refill it
     }
     if (STEP == 2) {
@@ -592,12 +648,12 @@ __global__ __launch_bounds__(256) void k_filter_adjoint(FArgs a) {
         acc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(acc), 0));
         const float s2 = a.sig[c] * a.sig[c];
         const float wg = had ? (acc > 0.0f ? 1.0f / (s2 * acc) : 1.0f) : 1.f / (s2 * acc);
-        float* dst = a.est + (((size_t)slot * C + c) * a.N) * K2;
+        float* dst = a.est + (size_t)slot * (unsigned)(a.N * a.ms) + c * K2;
         for (int n = 0; n < nsx; n++) {
             if (act) P[lane] = zg[n * K2 + lane];
             wave_sync();
             const float y = adj_fwd2d_T<K>(P, Tm, lane, bior, T);
-            if (act) dst[(size_t)n * K2 + lane] = wg * y;
+            if (act) dst[n * a.ms + lane] = wg * y;
         }
         wave_sync();
     }
