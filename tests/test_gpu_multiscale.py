@@ -157,3 +157,20 @@ def test_pyramid_command_lines(gpu_ctx, tmp_path):
     r = subprocess.run([os.path.join(bindir, "decompose"), str(tmp_path / "in.tiff")], capture_output=True, text=True,
                        timeout=60)
     assert r.returncode != 0 and "Usage" in r.stderr
+
+
+def test_multiscale_frames_in_several_batches(gpu_ctx):
+    """More frames than one batch of the pyramid's workspace holds: the
+    frames on both sides of the seam have the levels and the recomposition
+    that the single-image entries give (to the tolerance of another
+    summation order)."""
+    import vbm3d_amd as V
+    from vbm3d_amd import synth
+    F, W, H = 21, 1024, 1023
+    _, noisy = synth.noisy_clip(W, H, F, 1, 20.0, 51)
+    out, nlev, dlev = V.multiscale_denoise(noisy, 20.0, levels=2, return_levels=True, ctx=gpu_ctx)
+    for t in (0, 17, 18, 19, 20):
+        for g, o in zip(nlev, V.pyr_decompose(noisy[t], 2, ctx=gpu_ctx)):
+            np.testing.assert_allclose(g[t], o, rtol=0, atol=1e-3)
+        np.testing.assert_allclose(out[t], V.pyr_recompose([d[t] for d in dlev], factor=0.7, ctx=gpu_ctx), rtol=0,
+                                   atol=1e-3)

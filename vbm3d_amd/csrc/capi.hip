@@ -412,6 +412,7 @@ struct vbm3d_ctx {
     DevBuf tabsg, mpos;  // general path: tables, members' slice corners
     DevBuf tv;           // TV-L1 flow workspace (flow.hip)
     DevBuf pyr;          // pyramid workspace (pyramid.hip)
+    DevBuf msbuf;        // multiscale denoising: the video and its levels
     rocblas_handle blas = nullptr;  // the pyramid's DCT products
     size_t est_budget = 0;  // bytes for the per-patch rings; 0 = from free device memory
     unsigned chunk_frames = 0;  // per-clip path: frames per chunk; 0 = from the budget
@@ -1353,6 +1354,11 @@ hipError_t ctx_pyr_workspace(vbm3d_ctx* c, size_t bytes, void** p) {
     *p = c->pyr.p;
     return e;
 }
+hipError_t ctx_multiscale_buffer(vbm3d_ctx* c, size_t bytes, void** p) {
+    const hipError_t e = ensure(c->msbuf, bytes);
+    *p = c->msbuf.p;
+    return e;
+}
 rocblas_handle ctx_blas(vbm3d_ctx* c) {
     if (!c->blas) {
         if (rocblas_create_handle(&c->blas) != rocblas_status_success) {
@@ -1392,7 +1398,7 @@ void vbm3d_destroy(vbm3d_ctx* c) {
                       &c->idx, &c->nsx, &c->nsim, &c->dist, &c->est, &c->wgt, &c->tabs,
                       &c->refxy, &c->meta, &c->gpos, &c->rlist, &c->scal, &c->stats, &c->counts,
                       &c->b_idx, &c->b_nsx, &c->b_est, &c->b_wgt, &c->b_refxy, &c->b_meta, &c->b_gpos,
-                      &c->b_tabs, &c->b_plan, &c->b_cnt, &c->b_save, &c->tabsg, &c->mpos, &c->tv, &c->pyr,
+                      &c->b_tabs, &c->b_plan, &c->b_cnt, &c->b_save, &c->tabsg, &c->mpos, &c->tv, &c->pyr, &c->msbuf,
                       &c->boxtab})
         if (b->p) (void)hipFree(b->p);
     if (c->b_exec) (void)hipGraphExecDestroy(c->b_exec);

@@ -9,7 +9,9 @@
 // REDFT01) matrix -- in FP64 through rocBLAS's strided-batched DGEMM on
 // the matrix cores, then one rounding to float: the transform's exact
 // value to within double rounding (the reference's FFTW float transform
-// differs from it in the last bits).  The Gaussian and Lanczos pyramids
+// differs from it in the last bits).  The matrices are formed on the GPU
+// and the planes of many frames go through each product together.  The
+// Gaussian and Lanczos pyramids
 // are separable convolutions, one thread per output sample, in the
 // reference's float order: bit for bit its results.
 #include <hip/hip_runtime.h>
@@ -30,6 +32,7 @@ namespace vb {
 hipStream_t ctx_stream(vbm3d_ctx* c);
 int ctx_device(vbm3d_ctx* c);
 hipError_t ctx_pyr_workspace(vbm3d_ctx* c, size_t bytes, void** p);
+hipError_t ctx_multiscale_buffer(vbm3d_ctx* c, size_t bytes, void** p);
 rocblas_handle ctx_blas(vbm3d_ctx* c);
 int ctx_fail(int code, const std::string& msg);
 }  // namespace vb
@@ -39,6 +42,7 @@ namespace {
 
 constexpr int BX = 64, BY = 4;
 constexpr int kMaxPyrTaps = 32;
+constexpr size_t kPyrBatchBytes = (size_t)1 << 30;  // workspace bound of a batch of frames
 
 struct PTaps {
     float k[kMaxPyrTaps];
@@ -51,27 +55,40 @@ dim3 g2(int cols, int rows, int ch) {
 }
 
 // ---- element kernels
-__global__ void k_to_double(const float* __restrict__ in, double* out, long n) {
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
-        out[i] = (double)in[i];
+// The top-left rows x cols block of each sr x sc plane, as doubles
+// (decompose.cpp:44-52 where the block is smaller than the plane)
+__global__ void k_to_double(const float* __restrict__ in, int sr, int sc, double* out, int rows, int cols) {
+    const int q = blockIdx.x * BX + threadIdx.x, r = blockIdx.y * BY + threadIdx.y;
+    const size_t c = blockIdx.z;
+    if (q >= cols || r >= rows) return;
+    out[(c * rows + r) * cols + q] = (double)in[(c * sr + r) * sc + q];
 }
 
 // float(Y) / (4 rows cols) for the forward DCT (multiscaler.cpp:52-56),
-// float(Y) for the inverse
-__global__ void k_from_double(const double* __restrict__ in, float* out, long n, float div, int apply) {
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        const float v = (float)in[i];
-        out[i] = apply ? v / div : v;
-    }
+// float(Y) for the inverse, of the top-left h x w block of rows x cols
+// planes, into dr x dc planes (recompose.cpp:50-56 where these are larger)
+__global__ void k_from_double(const double* __restrict__ in, int rows, int cols, float* out, int dr, int dc, int h,
+                              int w, float div, int apply) {
+    const int q = blockIdx.x * BX + threadIdx.x, r = blockIdx.y * BY + threadIdx.y;
+    const size_t c = blockIdx.z;
+    if (q >= w || r >= h) return;
+    const float v = (float)in[(c * rows + r) * cols + q];
+    out[(c * dr + r) * dc + q] = apply ? v / div : v;
 }
 
-// copy the top-left h x w block of a rows x cols plane into an h x w
-// plane (decompose.cpp:44-52), or back (recompose.cpp:50-56, only j <
-// lim_r, k < lim_c)
-__global__ void k_block(const float* __restrict__ src, int sr, int sc, float* dst, int dr, int dc, int h, int w) {
-    const int q = blockIdx.x * BX + threadIdx.x, r = blockIdx.y * BY + threadIdx.y, c = blockIdx.z;
-    if (q >= w || r >= h) return;
-    dst[((size_t)c * dr + r) * dc + q] = src[((size_t)c * sr + r) * sc + q];
+// REDFT10 (inverse = 0: 2 cos(pi k (2n+1) / 2N)) or REDFT01 (1 for n = 0,
+// else 2 cos(pi n (2k+1) / 2N)) as a row-major N x N table [k][n].  The
+// argument is reduced in integers, so that cospi sees it in [0, 2).
+// Filled here, a table takes microseconds; the host's cosines took most of
+// a call (4 RGB frames 640x360 in 3 levels: 86.9 ms per call, 4.3 ms of
+// them in kernels).
+__global__ void k_dct_table(double* a, int N, int inverse) {
+    const int n = blockIdx.x * BX + threadIdx.x, k = blockIdx.y * BY + threadIdx.y;
+    if (n >= N || k >= N) return;
+    const unsigned long long m = inverse ? (unsigned long long)n * (2u * (unsigned)k + 1u)
+                                         : (unsigned long long)k * (2u * (unsigned)n + 1u);
+    const double c = cospi((double)(m % (4ull * (unsigned)N)) / (2.0 * N));
+    a[(size_t)k * N + n] = inverse && n == 0 ? 1.0 : 2.0 * c;
 }
 
 __global__ void k_fill_zero(float* p, long n) {
@@ -225,49 +242,45 @@ struct Pyr {
     }
 };
 
-// REDFT10 (inverse = false: 2 cos(pi k (2n+1) / 2N)) or REDFT01 (1 for
-// n = 0, else 2 cos(pi n (2k+1) / 2N)) as a row-major N x N table [k][n]
-std::vector<double> dct_table(int N, bool inverse) {
-    std::vector<double> a((size_t)N * N);
-    for (int k = 0; k < N; k++)
-        for (int n = 0; n < N; n++)
-            a[(size_t)k * N + n] = inverse ? (n == 0 ? 1.0 : 2.0 * std::cos(M_PI * n * (2.0 * k + 1.0) / (2.0 * N)))
-                                           : 2.0 * std::cos(M_PI * k * (2.0 * n + 1.0) / (2.0 * N));
-    return a;
-}
-
-// In-place 2D DCT (REDFT10, / 4 rows cols) or inverse (REDFT01) of `ch`
-// planes (multiscaler.cpp:21-98) with two strided-batched DGEMMs.
+// 2D DCT (REDFT10, / 4 rows cols) or inverse (REDFT01) of the top-left
+// rows x cols block of `np` planes of sr x sc (multiscaler.cpp:21-98) with
+// two strided-batched DGEMMs; the top-left h x w block of the result goes
+// into planes of dr x dc.  src and dst may be the same planes.
 // Column-major view: a row-major rows x cols plane is the cols x rows
 // matrix P^T; T^T = A_C P^T, then Y^T = T^T A_R^T.
-int dct2(Pyr& P, float* img, int rows, int cols, int ch, bool inverse) {
-    const size_t n = (size_t)ch * rows * cols;
+int dct2(Pyr& P, const float* src, int sr, int sc, float* dst, int dr, int dc, int h, int w, int rows, int cols, int np,
+         bool inverse) {
+    const size_t n = (size_t)np * rows * cols;
     const size_t mark = P.used;
     double* x = P.take<double>(n);
     double* t = P.take<double>(n);
     double* ar = P.take<double>((size_t)rows * rows);
     double* ac = P.take<double>((size_t)cols * cols);
     if (!x || !t || !ar || !ac) return ctx_fail(VBM3D_ERR_NOMEM, "pyramid workspace too small");
-    const std::vector<double> hr = dct_table(rows, inverse), hc = dct_table(cols, inverse);
-    PYR_TRY(hipMemcpyAsync(ar, hr.data(), hr.size() * 8, hipMemcpyHostToDevice, P.s));
-    PYR_TRY(hipMemcpyAsync(ac, hc.data(), hc.size() * 8, hipMemcpyHostToDevice, P.s));
-    hipLaunchKernelGGL(k_to_double, dim3(1024), dim3(256), 0, P.s, img, x, (long)n);
+    const dim3 b(BX, BY);
+    hipLaunchKernelGGL(k_dct_table, g2(rows, rows, 1), b, 0, P.s, ar, rows, inverse ? 1 : 0);
+    hipLaunchKernelGGL(k_dct_table, g2(cols, cols, 1), b, 0, P.s, ac, cols, inverse ? 1 : 0);
+    hipLaunchKernelGGL(k_to_double, g2(cols, rows, np), b, 0, P.s, src, sr, sc, x, rows, cols);
     PYR_TRY(hipGetLastError());
-    rocblas_handle h = ctx_blas(P.ctx);
+    rocblas_handle hd = ctx_blas(P.ctx);
     const double one = 1.0, zero = 0.0;
     const rocblas_stride st = (rocblas_stride)rows * cols;
     // T^T (cols x rows) = A_C (row-major table = col-major A_C^T, transposed) * P^T
-    BLAS_TRY(rocblas_dgemm_strided_batched(h, rocblas_operation_transpose, rocblas_operation_none, cols, rows, cols,
-                                           &one, ac, cols, 0, x, cols, st, &zero, t, cols, st, ch));
+    BLAS_TRY(rocblas_dgemm_strided_batched(hd, rocblas_operation_transpose, rocblas_operation_none, cols, rows, cols,
+                                           &one, ac, cols, 0, x, cols, st, &zero, t, cols, st, np));
     // Y^T (cols x rows) = T^T * A_R^T (the row-major table read column-major)
-    BLAS_TRY(rocblas_dgemm_strided_batched(h, rocblas_operation_none, rocblas_operation_none, cols, rows, rows, &one,
-                                           t, cols, st, ar, rows, 0, &zero, x, cols, st, ch));
-    hipLaunchKernelGGL(k_from_double, dim3(1024), dim3(256), 0, P.s, x, img, (long)n, (float)(4 * rows * cols),
-                       inverse ? 0 : 1);
+    BLAS_TRY(rocblas_dgemm_strided_batched(hd, rocblas_operation_none, rocblas_operation_none, cols, rows, rows, &one,
+                                           t, cols, st, ar, rows, 0, &zero, x, cols, st, np));
+    hipLaunchKernelGGL(k_from_double, g2(w, h, np), b, 0, P.s, x, rows, cols, dst, dr, dc, h, w,
+                       (float)(4 * rows * cols), inverse ? 0 : 1);
     PYR_TRY(hipGetLastError());
-    PYR_TRY(hipStreamSynchronize(P.s));  // the host tables above are freed on return
     P.used = mark;
     return VBM3D_OK;
+}
+
+// The whole planes, in place.
+int dct2(Pyr& P, float* img, int rows, int cols, int np, bool inverse) {
+    return dct2(P, img, rows, cols, img, rows, cols, rows, cols, rows, cols, np, inverse);
 }
 
 int conv_clamped(Pyr& P, float* img, float* tmp, int rows, int cols, int ch, const PTaps& t) {
@@ -357,9 +370,25 @@ int check_image(int rows, int cols, int ch, int levels, int type) {
     return VBM3D_OK;
 }
 
-// decompose.cpp:17-106 on device planes: `out` holds the levels one after
-// the other.
-int decompose_dev(Pyr& P, const float* img, int rows, int cols, int ch, int levels, int type, float* out) {
+// The levels' planes, stored one level after the other: level i of `np`
+// planes in total, of which `at` come before the ones at hand.
+template <class T>
+std::vector<T*> level_ptrs(T* base, int rows, int cols, int np, int levels, int at) {
+    std::vector<int> lr, lc;
+    level_sizes(rows, cols, levels, lr, lc);
+    std::vector<T*> p(levels);
+    for (int i = 0; i < levels; i++) {
+        const size_t sz = (size_t)lr[i] * lc[i];
+        p[i] = base + sz * at;
+        base += sz * np;
+    }
+    return p;
+}
+
+// decompose.cpp:17-106 on `ch` device planes (the channels of one or more
+// frames); out[i]: the planes of level i.
+int decompose_dev(Pyr& P, const float* img, int rows, int cols, int ch, int levels, int type,
+                  const std::vector<float*>& out) {
     std::vector<int> lr, lc;
     level_sizes(rows, cols, levels, lr, lc);
     const size_t n = (size_t)ch * rows * cols, mark = P.used;
@@ -367,58 +396,34 @@ int decompose_dev(Pyr& P, const float* img, int rows, int cols, int ch, int leve
     if (type == 0) {
         float* d = P.take<float>(n);
         if (!d) return ctx_fail(VBM3D_ERR_NOMEM, "pyramid workspace too small");
-        PYR_TRY(hipMemcpyAsync(d, img, n * 4, hipMemcpyDeviceToDevice, P.s));
-        if ((rc = dct2(P, d, rows, cols, ch, false))) return rc;
-        float* o = out;
-        for (int i = 0; i < levels; i++) {
-            hipLaunchKernelGGL(k_block, g2(lc[i], lr[i], ch), dim3(BX, BY), 0, P.s, d, rows, cols, o, lr[i], lc[i],
-                               lr[i], lc[i]);
-            PYR_TRY(hipGetLastError());
-            if ((rc = dct2(P, o, lr[i], lc[i], ch, true))) return rc;
-            o += (size_t)ch * lr[i] * lc[i];
-        }
+        if ((rc = dct2(P, img, rows, cols, d, rows, cols, rows, cols, rows, cols, ch, false))) return rc;
+        for (int i = 0; i < levels; i++)
+            if ((rc = dct2(P, d, rows, cols, out[i], lr[i], lc[i], lr[i], lc[i], lr[i], lc[i], ch, true))) return rc;
         P.used = mark;
         return VBM3D_OK;
     }
-    PYR_TRY(hipMemcpyAsync(out, img, n * 4, hipMemcpyDeviceToDevice, P.s));
-    float* prev = out;
-    for (int i = 1; i < levels; i++) {
-        float* cur = prev + (size_t)ch * lr[i - 1] * lc[i - 1];
-        if ((rc = down(P, prev, cur, lr[i - 1], lc[i - 1], ch, type == 2))) return rc;
-        prev = cur;
-    }
+    PYR_TRY(hipMemcpyAsync(out[0], img, n * 4, hipMemcpyDeviceToDevice, P.s));
+    for (int i = 1; i < levels; i++)
+        if ((rc = down(P, out[i - 1], out[i], lr[i - 1], lc[i - 1], ch, type == 2))) return rc;
     return VBM3D_OK;
 }
 
-// recompose.cpp:17-125 on device planes.
-int recompose_dev(Pyr& P, const float* lev, int rows, int cols, int ch, int levels, int type, float factor, float* out) {
+// recompose.cpp:17-125 on `ch` device planes; lev[i]: the planes of level i.
+int recompose_dev(Pyr& P, const std::vector<const float*>& lev, int rows, int cols, int ch, int levels, int type,
+                  float factor, float* out) {
     std::vector<int> lr, lc;
     level_sizes(rows, cols, levels, lr, lc);
-    std::vector<size_t> off(levels);
-    size_t o = 0;
-    for (int i = 0; i < levels; i++) {
-        off[i] = o;
-        o += (size_t)ch * lr[i] * lc[i];
-    }
     const size_t mark = P.used;
     int rc;
     if (type == 0) {
-        PYR_TRY(hipMemcpyAsync(out, lev, (size_t)ch * rows * cols * 4, hipMemcpyDeviceToDevice, P.s));
-        if ((rc = dct2(P, out, rows, cols, ch, false))) return rc;
-        float* im = P.take<float>((size_t)ch * rows * cols);
-        if (!im) return ctx_fail(VBM3D_ERR_NOMEM, "pyramid workspace too small");
+        if ((rc = dct2(P, lev[0], rows, cols, out, rows, cols, rows, cols, rows, cols, ch, false))) return rc;
         for (int i = 1; i < levels; i++) {
             const int h = lr[i], w = lc[i];
-            PYR_TRY(hipMemcpyAsync(im, lev + off[i], (size_t)ch * h * w * 4, hipMemcpyDeviceToDevice, P.s));
-            if ((rc = dct2(P, im, h, w, ch, false))) return rc;
             // the copied block: j < h * factor, k < w * factor (float bounds)
             int bh = 0, bw = 0;
             while (bh < h && (float)bh < h * factor) bh++;
             while (bw < w && (float)bw < w * factor) bw++;
-            if (bh > 0 && bw > 0) {
-                hipLaunchKernelGGL(k_block, g2(bw, bh, ch), dim3(BX, BY), 0, P.s, im, h, w, out, rows, cols, bh, bw);
-                PYR_TRY(hipGetLastError());
-            }
+            if (bh > 0 && bw > 0 && (rc = dct2(P, lev[i], h, w, out, rows, cols, bh, bw, h, w, ch, false))) return rc;
         }
         if ((rc = dct2(P, out, rows, cols, ch, true))) return rc;
         P.used = mark;
@@ -429,11 +434,11 @@ int recompose_dev(Pyr& P, const float* lev, int rows, int cols, int ch, int leve
     float* nxt = P.take<float>((size_t)ch * rows * cols);
     float* small = P.take<float>((size_t)ch * rows * cols);
     if (!cur || !nxt || !small) return ctx_fail(VBM3D_ERR_NOMEM, "pyramid workspace too small");
-    PYR_TRY(hipMemcpyAsync(cur, lev + off[levels - 1], (size_t)ch * lr[levels - 1] * lc[levels - 1] * 4,
+    PYR_TRY(hipMemcpyAsync(cur, lev[levels - 1], (size_t)ch * lr[levels - 1] * lc[levels - 1] * 4,
                            hipMemcpyDeviceToDevice, P.s));
     for (int i = levels - 2; i >= 0; --i) {
         const int h = lr[i], w = lc[i], h2 = lr[i + 1], w2 = lc[i + 1];
-        const float* image = lev + off[i];
+        const float* image = lev[i];
         if ((rc = down(P, image, small, h, w, ch, lz))) return rc;
         const long n2 = (long)ch * h2 * w2;
         hipLaunchKernelGGL(k_axpy, dim3(256), dim3(256), 0, P.s, cur, small, n2, -1.f);
@@ -515,7 +520,7 @@ int vbm3d_pyr_decompose(vbm3d_ctx* ctx, const float* img, int rows, int cols, in
     float* dout = D.get(nl);
     if (!di || !dout) return ctx_fail(VBM3D_ERR_NOMEM, "device allocation failed");
     PYR_TRY(hipMemcpyAsync(di, img, n * 4, hipMemcpyHostToDevice, P.s));
-    if ((rc = decompose_dev(P, di, rows, cols, ch, levels, type, dout))) return rc;
+    if ((rc = decompose_dev(P, di, rows, cols, ch, levels, type, level_ptrs(dout, rows, cols, ch, levels, 0)))) return rc;
     PYR_TRY(hipMemcpyAsync(out, dout, nl * 4, hipMemcpyDeviceToHost, P.s));
     PYR_TRY(hipStreamSynchronize(P.s));
     return VBM3D_OK;
@@ -534,7 +539,8 @@ int vbm3d_pyr_recompose(vbm3d_ctx* ctx, const float* levels_in, int rows, int co
     float* dout = D.get(n);
     if (!dl || !dout) return ctx_fail(VBM3D_ERR_NOMEM, "device allocation failed");
     PYR_TRY(hipMemcpyAsync(dl, levels_in, nl * 4, hipMemcpyHostToDevice, P.s));
-    if ((rc = recompose_dev(P, dl, rows, cols, ch, levels, type, factor, dout))) return rc;
+    if ((rc = recompose_dev(P, level_ptrs((const float*)dl, rows, cols, ch, levels, 0), rows, cols, ch, levels, type,
+                           factor, dout))) return rc;
     PYR_TRY(hipMemcpyAsync(out, dout, n * 4, hipMemcpyDeviceToHost, P.s));
     PYR_TRY(hipStreamSynchronize(P.s));
     return VBM3D_OK;
@@ -561,11 +567,10 @@ int vbm3d_pyr_merge_coarse(vbm3d_ctx* ctx, const float* fine, int rows, int cols
     if (!df || !dc) return ctx_fail(VBM3D_ERR_NOMEM, "device allocation failed");
     PYR_TRY(hipMemcpyAsync(df, fine, n * 4, hipMemcpyHostToDevice, P.s));
     PYR_TRY(hipMemcpyAsync(dc, coarse, nc * 4, hipMemcpyHostToDevice, P.s));
-    if ((rc = dct2(P, df, rows, cols, ch, false)) || (rc = dct2(P, dc, crows, ccols, ch, false))) return rc;
-    if (bh > 0 && bw > 0) {
-        hipLaunchKernelGGL(k_block, g2(bw, bh, ch), dim3(BX, BY), 0, P.s, dc, crows, ccols, df, rows, cols, bh, bw);
-        PYR_TRY(hipGetLastError());
-    }
+    if ((rc = dct2(P, df, rows, cols, ch, false))) return rc;
+    if (bh > 0 && bw > 0 &&
+        (rc = dct2(P, dc, crows, ccols, df, rows, cols, bh, bw, crows, ccols, ch, false)))
+        return rc;
     if ((rc = dct2(P, df, rows, cols, ch, true))) return rc;
     PYR_TRY(hipMemcpyAsync(out, df, n * 4, hipMemcpyDeviceToHost, P.s));
     PYR_TRY(hipStreamSynchronize(P.s));
@@ -580,18 +585,22 @@ int vbm3d_multiscale_denoise(vbm3d_ctx* ctx, float sigma, const float* noisy, un
     if (rc) return rc;
     if (!noisy || !denoised || F == 0) return ctx_fail(VBM3D_ERR_ARG, "null buffer or empty video");
     if (!(sigma > 0.f)) return ctx_fail(VBM3D_ERR_ARG, "sigma must be positive");
+    // frames that go through the pyramid together: as many as a workspace of
+    // kPyrBatchBytes holds (planes are a grid dimension: at most 65535)
+    const size_t frame_bytes = pyr_bytes((int)H, (int)W, (int)C);
+    const int batch = (int)std::max<size_t>(
+        1, std::min<size_t>(std::min<size_t>(F, 65535 / C), kPyrBatchBytes / std::max<size_t>(frame_bytes, 1)));
     Pyr P;
-    if ((rc = pyr_open(ctx, P, pyr_bytes((int)H, (int)W, (int)C)))) return rc;
+    if ((rc = pyr_open(ctx, P, pyr_bytes((int)H, (int)W, (int)C * batch)))) return rc;
     std::vector<int> lr, lc;
     level_sizes((int)H, (int)W, levels, lr, lc);
     const size_t fw = (size_t)C * H * W, flev = level_words((int)H, (int)W, (int)C, levels);
-    Dev D;
-    float* dn = D.get(fw * F);
-    float* dlev = D.get(flev * F);   // per level: [F][C][h][w], level after level
-    float* dden = D.get(flev * F);
-    float* dbas = D.get(fw * F);
-    float* dfr = D.get(flev);
-    if (!dn || !dlev || !dden || !dbas || !dfr) return ctx_fail(VBM3D_ERR_NOMEM, "device allocation failed");
+    // the video, its levels (noisy and denoised: per level [F][C][h][w],
+    // level after level) and a basic estimate
+    void* base = nullptr;
+    if (ctx_multiscale_buffer(ctx, (2 * fw + 2 * flev) * F * 4, &base) != hipSuccess)
+        return ctx_fail(VBM3D_ERR_NOMEM, "device allocation failed");
+    float *dn = (float*)base, *dbas = dn + fw * F, *dlev = dbas + fw * F, *dden = dlev + flev * F;
     std::vector<size_t> loff(levels);
     size_t o = 0;
     for (int i = 0; i < levels; i++) {
@@ -599,15 +608,12 @@ int vbm3d_multiscale_denoise(vbm3d_ctx* ctx, float sigma, const float* noisy, un
         o += (size_t)C * lr[i] * lc[i] * F;
     }
     PYR_TRY(hipMemcpyAsync(dn, noisy, fw * F * 4, hipMemcpyHostToDevice, P.s));
-    // 1. every frame into its levels (decompose per frame)
-    for (unsigned t = 0; t < F; t++) {
-        if ((rc = decompose_dev(P, dn + fw * t, (int)H, (int)W, (int)C, levels, type, dfr))) return rc;
-        size_t fo = 0;
-        for (int i = 0; i < levels; i++) {
-            const size_t ls = (size_t)C * lr[i] * lc[i];
-            PYR_TRY(hipMemcpyAsync(dlev + loff[i] + ls * t, dfr + fo, ls * 4, hipMemcpyDeviceToDevice, P.s));
-            fo += ls;
-        }
+    // 1. every frame into its levels
+    for (unsigned t = 0; t < F; t += (unsigned)batch) {
+        const int nf = (int)std::min<unsigned>((unsigned)batch, F - t);
+        if ((rc = decompose_dev(P, dn + fw * t, (int)H, (int)W, (int)C * nf, levels, type,
+                                level_ptrs(dlev, (int)H, (int)W, (int)(C * F), levels, (int)(C * t)))))
+            return rc;
     }
     if (noisy_levels) {
         PYR_TRY(hipMemcpyAsync(noisy_levels, dlev, flev * F * 4, hipMemcpyDeviceToHost, P.s));
@@ -632,14 +638,11 @@ int vbm3d_multiscale_denoise(vbm3d_ctx* ctx, float sigma, const float* noisy, un
         PYR_TRY(hipMemcpyAsync(denoised_levels, dden, flev * F * 4, hipMemcpyDeviceToHost, P.s));
     }
     // 3. every frame recomposed from its denoised levels
-    for (unsigned t = 0; t < F; t++) {
-        size_t fo = 0;
-        for (int i = 0; i < levels; i++) {
-            const size_t ls = (size_t)C * lr[i] * lc[i];
-            PYR_TRY(hipMemcpyAsync(dfr + fo, dden + loff[i] + ls * t, ls * 4, hipMemcpyDeviceToDevice, P.s));
-            fo += ls;
-        }
-        if ((rc = recompose_dev(P, dfr, (int)H, (int)W, (int)C, levels, type, factor, dn + fw * t))) return rc;
+    for (unsigned t = 0; t < F; t += (unsigned)batch) {
+        const int nf = (int)std::min<unsigned>((unsigned)batch, F - t);
+        if ((rc = recompose_dev(P, level_ptrs((const float*)dden, (int)H, (int)W, (int)(C * F), levels, (int)(C * t)),
+                                (int)H, (int)W, (int)C * nf, levels, type, factor, dn + fw * t)))
+            return rc;
     }
     PYR_TRY(hipMemcpyAsync(denoised, dn, fw * F * 4, hipMemcpyDeviceToHost, P.s));
     PYR_TRY(hipStreamSynchronize(P.s));
