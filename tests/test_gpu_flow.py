@@ -61,6 +61,31 @@ def test_flow_matches_oracle(gpu_ctx, case):
     assert bits_equal(u, ou) and bits_equal(v, ov), (np.abs(u - ou).max(), np.abs(v - ov).max())
 
 
+# region sizes of the iteration kernel: one region, one pixel more than the
+# inside of a region, the smallest image, and levels of more regions than the
+# in-launch stopping test takes (large regions; with its own launch)
+STEP_SIZES = {
+    "12x11": (12, 11, {"nscales": 1, "warps": 2}),
+    "26x10": (26, 10, {"nscales": 1}),
+    "27x11": (27, 11, {"nscales": 1}),
+    "53x20": (53, 20, {"nscales": 1, "warps": 2}),
+    "313x256": (313, 256, {"nscales": 2, "warps": 2}),
+    "503x401": (503, 401, {"nscales": 2, "warps": 2}),
+    "eps0-503x401": (503, 401, {"nscales": 1, "warps": 1, "epsilon": 0.0}),
+}
+
+
+@pytest.mark.parametrize("case", list(STEP_SIZES), ids=list(STEP_SIZES))
+def test_flow_region_edges(gpu_ctx, case):
+    from oracle import tvl1 as T
+    w, h, kw = STEP_SIZES[case]
+    I0, I1 = pair(w, h, 11)
+    u, v, it = gpu_flow(I0, I1, gpu_ctx, **kw)
+    ou, ov, oit = T.flow(I0, I1, **kw)
+    np.testing.assert_array_equal(it, oit)
+    assert bits_equal(u, ou) and bits_equal(v, ov)
+
+
 def test_golden_flows(gpu_ctx):
     g = np.load(GOLDEN)
     for n in sorted({k.split("/")[0] for k in g.files}):

@@ -15,15 +15,16 @@
 // iteration when the two sums straddle epsilon^2.
 //
 // The iterations never return to the host one by one: a control word in
-// device memory (active, iteration count) is updated by a one-workgroup
-// kernel after each iteration, every iteration kernel exits at once when
-// the word says the warp has converged, and the host launches iterations
-// in batches and reads the word between batches.
+// device memory says where a level stands, every launch reads it, does what
+// comes next and leaves the word for the launch after it, and the host
+// enqueues launches and looks at the word now and then.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "vbm3d_hip.h"
@@ -52,11 +53,22 @@ struct Taps {
     int size;
 };
 
+// The flow's state planes of one side of the ping-pong.
+struct FlowState {
+    float *u1, *u2, *p11, *p12, *p21, *p22;
+};
+
+// Where a level stands; every launch of k_level_step reads one word and
+// leaves the next launch's.
+enum { kWarp, kStart, kRun, kDone };
 struct FlowCtl {
-    int active;   // 1 while the current warp iterates
-    int iter;     // iterations done in the current warp
-    float error;  // last mean squared change
-    unsigned done;  // blocks of k_iter_dual_ctl finished in this iteration
+    int phase;  // kWarp: set up `warp`; kStart: its first iterations; kRun: test
+                // the last launch's iterations, then go on; kDone: level solved
+    int warp;   // warp at hand
+    int iter;   // its iterations so far (those not yet tested included)
+    int steps;  // kRun: iterations of the last launch
+    int cur;    // which state holds the flow and the dual field
+    int stop;   // large levels: k_level_test's result for those iterations
 };
 
 __device__ __forceinline__ int clampi(int x, int n, bool& out) {
@@ -193,20 +205,44 @@ __global__ void k_gauss_cols(const float* __restrict__ in, float* out, int nx, i
 
 // ---- bicubic resampling of a level (zoom.c:44-117): output (j1, i1)
 // samples the input at (j1 / fx, i1 / fy); flows are then multiplied by
-// `scale` (the 1 / zfactor of tvl1flow_lib.c:453-457) when apply.
+// `scale` (the 1 / zfactor of tvl1flow_lib.c:453-457).
 __global__ void k_resample(const float* __restrict__ in, float* out, int nx, int ny, int nxx, int nyy, float fx,
-                           float fy, float scale, int apply) {
+                           float fy) {
     const int j1 = blockIdx.x * BX + threadIdx.x, i1 = blockIdx.y * BY + threadIdx.y;
     if (j1 >= nxx || i1 >= nyy) return;
     const float i2 = (float)i1 / fy, j2 = (float)j1 / fx;
     Nbhd n;
     (void)nbhd(j2, i2, nx, ny, n);
-    const float g = interp(in, nx, n);
-    out[(size_t)i1 * nxx + j1] = apply ? g * scale : g;
+    out[(size_t)i1 * nxx + j1] = interp(in, nx, n);
+}
+
+// Both components of a flow: from `a` or, at a solved level (ctl not null),
+// from the state that holds it
+__global__ void k_upsample(const FlowCtl* __restrict__ ctl, FlowState s0, FlowState s1, float* o1, float* o2, int nx,
+                           int ny, int nxx, int nyy, float fx, float fy, float scale) {
+    const int j1 = blockIdx.x * BX + threadIdx.x, i1 = blockIdx.y * BY + threadIdx.y;
+    if (j1 >= nxx || i1 >= nyy) return;
+    const FlowState& s = ctl && ctl->cur ? s1 : s0;
+    const float i2 = (float)i1 / fy, j2 = (float)j1 / fx;
+    Nbhd n;
+    (void)nbhd(j2, i2, nx, ny, n);
+    o1[(size_t)i1 * nxx + j1] = interp(s.u1, nx, n) * scale;
+    o2[(size_t)i1 * nxx + j1] = interp(s.u2, nx, n) * scale;
+}
+
+// The solved flow of the finest level
+__global__ void k_flow_out(const FlowCtl* __restrict__ ctl, FlowState s0, FlowState s1, float* u, float* v, long n) {
+    const FlowState& s = ctl->cur ? s1 : s0;
+    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
+        u[i] = s.u1[i];
+        v[i] = s.u2[i];
+    }
 }
 
 // ---- centred gradient with one-sided edges (mask.c:144-214)
-__global__ void k_cgrad(const float* __restrict__ in, float* dx, float* dy, int nx, int ny) {
+// and the control word of a new level
+__global__ void k_cgrad(const float* __restrict__ in, float* dx, float* dy, int nx, int ny, FlowCtl* ctl) {
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0 && threadIdx.y == 0) *ctl = FlowCtl{kWarp, 0, 0, 0, 0, 0};
     const int j = blockIdx.x * BX + threadIdx.x, i = blockIdx.y * BY + threadIdx.y;
     if (j >= nx || i >= ny) return;
     const size_t k = (size_t)i * nx + j;
@@ -216,16 +252,15 @@ __global__ void k_cgrad(const float* __restrict__ in, float* dx, float* dy, int 
     dy[k] = (float)(0.5 * (double)(in[id] - in[iu]));
 }
 
-// ---- one warp's set-up (tvl1flow_lib.c:150-166): the target image and
+// ---- one warp's set-up at a pixel (tvl1flow_lib.c:150-166): the target image and
 // its derivatives at the flow-displaced positions (zero outside), |grad|^2
 // and the constant part of the linearised residual.
-__global__ void k_warp(const float* __restrict__ I0, const float* __restrict__ I1, const float* __restrict__ I1x,
-                       const float* __restrict__ I1y, const float* __restrict__ u1, const float* __restrict__ u2,
-                       float* wx, float* wy, float* grad, float* rho_c, int nx, int ny) {
-    const int j = blockIdx.x * BX + threadIdx.x, i = blockIdx.y * BY + threadIdx.y;
-    if (j >= nx || i >= ny) return;
+__device__ __forceinline__ void warp_px(const float* __restrict__ I0, const float* __restrict__ I1,
+                                        const float* __restrict__ I1x, const float* __restrict__ I1y, float u1,
+                                        float u2, float* wx, float* wy, float* grad, float* rho_c, int i, int j,
+                                        int nx, int ny) {
     const size_t p = (size_t)i * nx + j;
-    const float uu = (float)j + u1[p], vv = (float)i + u2[p];
+    const float uu = (float)j + u1, vv = (float)i + u2;
     Nbhd n;
     float w = 0.f, gx = 0.f, gy = 0.f;
     if (nbhd(uu, vv, nx, ny, n)) {
@@ -237,38 +272,50 @@ __global__ void k_warp(const float* __restrict__ I0, const float* __restrict__ I
     wx[p] = gx;
     wy[p] = gy;
     grad[p] = Ix2 + Iy2;
-    rho_c[p] = w - gx * u1[p] - gy * u2[p] - I0[p];
+    rho_c[p] = w - gx * u1 - gy * u2 - I0[p];
 }
+
+// ---- the primal-dual iterations (tvl1flow_lib.c:168-252)
+//
+// What one iteration does at a pixel is a stencil of radius 1 on the flow
+// (u1, u2) and the dual field (p11, p12, p21, p22): the primal step needs
+// the dual field at the left and upper neighbours, the dual step the new
+// flow at the right and lower ones.  Run one launch per step, an iteration
+// was three launches and 88 bytes of traffic per pixel.  Here a workgroup
+// takes an RX x RY region into LDS and runs T iterations on it; the outer
+// T pixels of the region go stale, one ring per iteration, and only the
+// inside is written, to the other state of a ping-pong.  The stopping test
+// needs the mean squared change of every iteration: each launch leaves its
+// iterations' sums per workgroup, the next launch adds them up (every
+// workgroup the same sums in the same order) and knows whether the warp
+// had converged inside the last launch.  If it had, and not at its last
+// iteration, that launch ran too far: the iterations up to the stopping
+// one are run again from the state it started from, which the ping-pong
+// still holds.  So the flow and the iteration counts are those of the
+// one-by-one form.  What bounds it: instruction issue on large levels (two
+// double-precision roots and five divisions per pixel and iteration),
+// the latency of the chain load, test, iterations, store on small ones.
+// Measured: a 1920x1080 pair 18.6 -> 7.5 ms, a 317x241 pair 8.7 -> 2.7 ms.
 
 // Backward-difference divergence with the reference's edge cases
-// (mask.c:39-90).
-__device__ __forceinline__ float div_at(const float* __restrict__ v1, const float* __restrict__ v2, int i, int j,
-                                        int nx, int ny) {
-    const size_t p = (size_t)i * nx + j;
-    const bool L = j == 0, R = j == nx - 1, T = i == 0, B = i == ny - 1;
-    if (!L && !R && !T && !B) return (v1[p] - v1[p - 1]) + (v2[p] - v2[p - nx]);
-    if (T && L) return v1[0] + v2[0];
-    if (T && R) return -v1[nx - 2] + v2[nx - 1];
-    if (B && L) return v1[p] - v2[p - nx];
-    if (B && R) return -v1[p - 1] - v2[p - nx];
-    if (T) return v1[p] - v1[p - 1] + v2[p];
-    if (B) return v1[p] - v1[p - 1] - v2[p - nx];
-    if (L) return v1[p] + v2[p] - v2[p - nx];
-    return -v1[p - 1] + v2[p] - v2[p - nx];
+// (mask.c:39-90) at a pixel that is first / last in its row (L, R) and
+// column (T, B), from the two components, the left neighbour of the first
+// and the upper neighbour of the second.
+template <bool EDGE>
+__device__ __forceinline__ float div_px(float v1, float v1l, float v2, float v2u, unsigned edge) {
+    if (!EDGE || edge == 0) return (v1 - v1l) + (v2 - v2u);
+    const bool L = edge & 1, R = edge & 2, T = edge & 4, B = edge & 8;
+    const float h = L ? v1 : (R ? -v1l : v1 - v1l);
+    if (T) return h + v2;
+    if (B) return h - v2u;
+    return h + v2 - v2u;
 }
 
-// ---- iteration, part 1 (tvl1flow_lib.c:170-231) at pixel (i, j):
-// thresholding towards the data term, divergence of the dual field, primal
-// update in place; returns the squared change of the flow.
-__device__ __forceinline__ double primal_px(float* u1, float* u2, const float* __restrict__ wx,
-                                            const float* __restrict__ wy, const float* __restrict__ grad,
-                                            const float* __restrict__ rho_c, const float* __restrict__ p11,
-                                            const float* __restrict__ p12, const float* __restrict__ p21,
-                                            const float* __restrict__ p22, int i, int j, int nx, int ny, float l_t,
-                                            float theta) {
-    const size_t p = (size_t)i * nx + j;
-    const float a = u1[p], b = u2[p], gx = wx[p], gy = wy[p], g = grad[p];
-    const float rho = rho_c[p] + (gx * a + gy * b);
+// Thresholding towards the data term (tvl1flow_lib.c:170-212): the
+// auxiliary flow at a pixel.
+__device__ __forceinline__ void threshold_px(float a, float b, float gx, float gy, float g, float rc, float l_t,
+                                             float& v1, float& v2) {
+    const float rho = rc + (gx * a + gy * b);
     float d1, d2;
     if (rho < -l_t * g) {
         d1 = l_t * gx;
@@ -283,203 +330,249 @@ __device__ __forceinline__ double primal_px(float* u1, float* u2, const float* _
         d1 = fi * gx;
         d2 = fi * gy;
     }
-    const float v1 = a + d1, v2 = b + d2;
-    const float n1 = v1 + theta * div_at(p11, p12, i, j, nx, ny);
-    const float n2 = v2 + theta * div_at(p21, p22, i, j, nx, ny);
-    u1[p] = n1;
-    u2[p] = n2;
-    return (double)((n1 - a) * (n1 - a) + (n2 - b) * (n2 - b));
+    v1 = a + d1;
+    v2 = b + d2;
 }
 
-// ---- iteration, part 2 (tvl1flow_lib.c:233-252) at pixel (i, j):
-// forward gradient of the new flow and the projected dual update.
-__device__ __forceinline__ void dual_px(const float* __restrict__ u1, const float* __restrict__ u2, float* p11,
-                                        float* p12, float* p21, float* p22, int i, int j, int nx, int ny,
-                                        float taut) {
-    const size_t p = (size_t)i * nx + j;
-    const float u1x = j < nx - 1 ? u1[p + 1] - u1[p] : 0.f, u1y = i < ny - 1 ? u1[p + nx] - u1[p] : 0.f;
-    const float u2x = j < nx - 1 ? u2[p + 1] - u2[p] : 0.f, u2y = i < ny - 1 ? u2[p + nx] - u2[p] : 0.f;
-    // |grad| in double: the squares of floats are exact, one rounding of
-    // their sum and one of the root; as a float this is the C library's
-    // hypot of the two values
-    const float g1 = (float)sqrt((double)u1x * (double)u1x + (double)u1y * (double)u1y);
-    const float g2 = (float)sqrt((double)u2x * (double)u2x + (double)u2y * (double)u2y);
-    const float ng1 = (float)(1.0 + (double)(taut * g1)), ng2 = (float)(1.0 + (double)(taut * g2));
-    p11[p] = (p11[p] + taut * u1x) / ng1;
-    p12[p] = (p12[p] + taut * u1y) / ng1;
-    p21[p] = (p21[p] + taut * u2x) / ng2;
-    p22[p] = (p22[p] + taut * u2y) / ng2;
+// The projected dual update of one flow component (tvl1flow_lib.c:233-252)
+// from its forward gradient.  |grad| is taken in double: the squares of
+// floats are exact, so one rounding of their sum and one of the root; as a
+// float this is the C library's hypot.  The sum 1.0 + taut |grad| in double,
+// rounded to float, is the float sum: it is exact in double wherever it
+// differs from 1.
+__device__ __forceinline__ void dual_px(float& pa, float& pb, float ux, float uy, float taut) {
+    const float g = (float)sqrt(__builtin_fma((double)ux, (double)ux, (double)uy * (double)uy));
+    const float ng = 1.0f + taut * g;
+    pa = (pa + taut * ux) / ng;
+    pb = (pb + taut * uy) / ng;
 }
 
-// Part 1 over the level; each workgroup (64 x 4 pixels) leaves its sum of
-// squared changes in a fixed order: every row of 64 by a wavefront's
-// butterfly, then the four rows in order.
-__global__ void k_iter_primal(const FlowCtl* __restrict__ ctl, float* u1, float* u2, const float* __restrict__ wx,
-                              const float* __restrict__ wy, const float* __restrict__ grad,
-                              const float* __restrict__ rho_c, const float* __restrict__ p11,
-                              const float* __restrict__ p12, const float* __restrict__ p21,
-                              const float* __restrict__ p22, double* part, int nx, int ny, float l_t, float theta) {
-    if (!ctl->active) return;  // uniform
-    const int j = blockIdx.x * BX + threadIdx.x, i = blockIdx.y * BY + threadIdx.y;
-    double e = 0.0;
-    if (j < nx && i < ny) e = primal_px(u1, u2, wx, wy, grad, rho_c, p11, p12, p21, p22, i, j, nx, ny, l_t, theta);
-    for (int o = 32; o >= 1; o >>= 1) e += __shfl_xor(e, o, 64);
-    __shared__ double s[BX * BY / 64];
-    const int t = threadIdx.y * BX + threadIdx.x;
-    if ((t & 63) == 0) s[t >> 6] = e;
-    __syncthreads();
-    if (t == 0) {
-        double acc = 0.0;
-        for (int q = 0; q < BX * BY / 64; q++) acc += s[q];
-        part[blockIdx.y * gridDim.x + blockIdx.x] = acc;
-    }
+// Sum over a wavefront in a fixed order on the DPP network (quad swaps,
+// half-row and row mirrors, the row-15 and lane-31 broadcasts): lane 63
+// holds it.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+    const long long b = __builtin_bit_cast(long long, v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xF, false);
+    return v + __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double wave_sum(double v) {
+    v = dpp_add<0xB1, 0xF>(v);
+    v = dpp_add<0x4E, 0xF>(v);
+    v = dpp_add<0x141, 0xF>(v);
+    v = dpp_add<0x140, 0xF>(v);
+    v = dpp_add<0x142, 0xA>(v);
+    return dpp_add<0x143, 0xC>(v);
 }
 
-// Part 2 over the level.
-__global__ void k_iter_dual(const FlowCtl* __restrict__ ctl, const float* __restrict__ u1,
-                            const float* __restrict__ u2, float* p11, float* p12, float* p21, float* p22, int nx,
-                            int ny, float taut) {
-    if (!ctl->active) return;  // uniform
-    const int j = blockIdx.x * BX + threadIdx.x, i = blockIdx.y * BY + threadIdx.y;
-    if (j >= nx || i >= ny) return;
-    dual_px(u1, u2, p11, p12, p21, p22, i, j, nx, ny, taut);
-}
+struct LevelArgs {
+    FlowCtl* ctl;     // [2], by launch parity
+    double* part;     // [2][T][blocks] sums of squared changes
+    FlowState st[2];
+    const float *I0, *I1, *I1x, *I1y;
+    const float *u1, *u2;  // the level's initial flow
+    float *wx, *wy, *grad, *rho;
+    int nx, ny, nwarps;
+    float l_t, theta, taut, size, eps2;
+    int* counts;  // iterations of each warp
+};
 
-// ---- iteration, part 3: the mean squared change and the stopping test
-// (tvl1flow_lib.c:159, 228): one workgroup sums the partials in a fixed
-// order.
-__global__ void k_iter_ctl(FlowCtl* ctl, const double* __restrict__ part, int nparts, float size, float eps2) {
-    if (!ctl->active) return;  // uniform
+// Whether `steps` <= T iterations ending at iteration `iter`, with sums in
+// part [step][nblk], hold the warp's last one: its index, or -1.  The
+// wavefronts of a workgroup of NT threads share the steps; each sum is
+// formed in a fixed order.  s: NT / 64 doubles.  Every thread gets it.
+template <int NT, int T>
+__device__ int stop_step(const LevelArgs& a, const double* __restrict__ part, int nblk, int steps, int iter, double* s) {
+    constexpr int WPS = NT / 64 / T;  // wavefronts per step
+    static_assert(WPS >= 1, "a wavefront per step");
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, k = w / WPS;
     double acc = 0.0;
-    for (int q = threadIdx.x; q < nparts; q += blockDim.x) acc += part[q];
-    for (int o = 32; o >= 1; o >>= 1) acc += __shfl_xor(acc, o, 64);
-    __shared__ double s[16];
-    if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = acc;
+    if (k < steps)
+        for (int q = (w - k * WPS) * 64 + lane; q < nblk; q += WPS * 64) acc += part[(size_t)k * nblk + q];
+    acc = wave_sum(acc);
+    if (lane == 63) s[w] = acc;
     __syncthreads();
-    if (threadIdx.x == 0) {
+    for (int q = 0; q < steps; q++) {
         double t = 0.0;
-        for (int q = 0; q < (int)(blockDim.x >> 6); q++) t += s[q];
+        for (int r = 0; r < WPS; r++) t += s[q * WPS + r];
         float err = (float)t;
-        err /= size;
-        ctl->error = err;
-        ctl->iter += 1;
-        ctl->active = (err > eps2 && ctl->iter < kMaxIter) ? 1 : 0;
+        err /= a.size;
+        if (!(err > a.eps2) || iter - steps + q + 1 >= kMaxIter) return q;
     }
+    return -1;
 }
 
-__global__ void k_ctl_start(FlowCtl* ctl) {
-    ctl->active = 1;
-    ctl->iter = 0;
-    ctl->error = INFINITY;
-    ctl->done = 0;
+// The test as a launch of its own, for levels of more than kTestBlocks
+// workgroups: there every workgroup of the next launch adding up all sums
+// reads more than the level itself (3,672 workgroups at 1920x1080: 323 MB a
+// launch).
+constexpr int kTestBlocks = 256;
+template <int T>
+__global__ __launch_bounds__(1024) void k_level_test(LevelArgs a, int par, int nblk) {
+    __shared__ double s_sum[16];
+    const FlowCtl c = a.ctl[par];
+    if (c.phase != kRun) return;
+    const int k = stop_step<1024, T>(a, a.part + (size_t)(par ^ 1) * T * nblk, nblk, c.steps, c.iter, s_sum);
+    if (threadIdx.x == 0) a.ctl[par].stop = k;
 }
 
-// Parts 2 and 3 in one launch, for levels of at most kFuseBlocks blocks:
-// the dual update, then the workgroup that finishes last (one atomic per
-// workgroup on the control word) sums the partials and runs the stopping
-// test exactly as k_iter_ctl does (256 threads, the same order), so the
-// flow and the iteration count are unchanged.  No workgroup waits for
-// another.
-constexpr int kFuseBlocks = 1024;
-__global__ void k_iter_dual_ctl(FlowCtl* ctl, const float* __restrict__ u1, const float* __restrict__ u2,
-                                float* p11, float* p12, float* p21, float* p22, int nx, int ny, float taut,
-                                const double* __restrict__ part, int nparts, float size, float eps2) {
-    if (!ctl->active) return;  // uniform
-    const int j = blockIdx.x * BX + threadIdx.x, i = blockIdx.y * BY + threadIdx.y;
-    if (j < nx && i < ny) dual_px(u1, u2, p11, p12, p21, p22, i, j, nx, ny, taut);
-    const int t = threadIdx.y * BX + threadIdx.x;
-    __shared__ int s_last;
-    __syncthreads();
-    if (t == 0) s_last = atomicAdd(&ctl->done, 1u) == gridDim.x * gridDim.y - 1;
-    __syncthreads();
-    if (!s_last) return;
-    double acc = 0.0;
-    for (int q = t; q < nparts; q += BX * BY) acc += part[q];
-    for (int o = 32; o >= 1; o >>= 1) acc += __shfl_xor(acc, o, 64);
-    __shared__ double s[BX * BY / 64];
-    if ((t & 63) == 0) s[t >> 6] = acc;
-    __syncthreads();
-    if (t == 0) {
-        double tt = 0.0;
-        for (int q = 0; q < BX * BY / 64; q++) tt += s[q];
-        float err = (float)tt;
-        err /= size;
-        ctl->error = err;
-        ctl->iter += 1;
-        ctl->active = (err > eps2 && ctl->iter < kMaxIter) ? 1 : 0;
-        ctl->done = 0;
+template <int RX, int RY, int NT, int T>
+__global__ __launch_bounds__(NT) void k_level_step(LevelArgs a, int par) {
+    constexpr int PX = RX * RY / NT, UX = RX - 2 * T, UY = RY - 2 * T;
+    static_assert(RX * RY % NT == 0 && UX > 0 && UY > 0, "whole pixels per thread");
+    __shared__ float s_u1[RX * RY], s_u2[RX * RY], s_p11[RX * RY], s_p12[RX * RY], s_p21[RX * RY], s_p22[RX * RY];
+    __shared__ double s_sum[NT / 64], s_err[T][NT / 64];
+    const int t = threadIdx.x;
+    const int nblk = gridDim.x * gridDim.y, blk = blockIdx.y * gridDim.x + blockIdx.x;
+    const FlowCtl c = a.ctl[par];
+    FlowCtl next = c;
+    int steps = 0, src = c.cur;  // iterations to run, from state src into the other
+    bool setup = false;          // or set the warp up
+    if (c.phase == kWarp) {
+        setup = true;
+        next.phase = kStart;
+    } else if (c.phase == kRun) {
+        const int k = nblk > kTestBlocks
+                          ? c.stop
+                          : stop_step<NT, T>(a, a.part + (size_t)(par ^ 1) * T * nblk, nblk, c.steps, c.iter, s_sum);
+        if (k >= 0) {
+            if (blk == 0 && t == 0) a.counts[c.warp] = c.iter - c.steps + k + 1;
+            next.warp = c.warp + 1;
+            next.phase = next.warp == a.nwarps ? kDone : kWarp;
+            if (k + 1 < c.steps) {
+                steps = k + 1;  // again, up to the stopping iteration
+                src = c.cur ^ 1;
+            } else if (next.phase == kWarp) {
+                setup = true;
+                next.phase = kStart;
+            }
+        }
     }
-}
-
-// Every iteration of one warp on a level of at most kSmallPx pixels (and
-// kSmallBlocks blocks of 64 x 4), in one workgroup of 1024 threads: the
-// same per-pixel updates as k_iter_primal and k_iter_dual, and the stopping
-// test's sums in their order (a row of 64 pixels by a wavefront's
-// butterfly, the four rows of a block in order, then the blocks' sums as
-// k_iter_ctl adds them), so the flow and the iteration count are those of
-// the three-launch form.  It replaces up to 3 x 300 launches and the host's
-// reads of the control word; the count goes to *count.
-constexpr int kSmallPx = 16384, kSmallBlocks = 256;
-__global__ __launch_bounds__(1024) void k_iter_small(FlowCtl* ctl, float* u1, float* u2, const float* __restrict__ wx,
-                                                     const float* __restrict__ wy, const float* __restrict__ grad,
-                                                     const float* __restrict__ rho_c, float* p11, float* p12,
-                                                     float* p21, float* p22, int nx, int ny, float l_t, float theta,
-                                                     float taut, float size, float eps2, int* count) {
-    __shared__ double s_row[kSmallBlocks * BY];
-    __shared__ double s_blk[kSmallBlocks];
-    __shared__ double s_w[4];
-    __shared__ int s_active, s_iter;
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int gx = (nx + BX - 1) / BX, gy = (ny + BY - 1) / BY, nblk = gx * gy;
-    if (t == 0) {
-        s_active = ctl->active;
-        s_iter = ctl->iter;
+    if (c.phase == kStart || next.phase == kRun) {
+        next.iter = c.phase == kStart ? 0 : c.iter;
+        next.steps = steps = min(T, kMaxIter - next.iter);
+        next.iter += steps;
+        next.phase = kRun;
+        next.cur = src ^ 1;
     }
-    for (;;) {
-        __syncthreads();  // the previous iteration's dual updates and control word
-        if (!s_active) break;  // workgroup-uniform
-        // primal, one row of 64 pixels (block b, row r) per wavefront step
-        for (int vr = w; vr < nblk * BY; vr += 16) {
-            const int b = vr / BY, r = vr - b * BY;
-            const int j = (b % gx) * BX + lane, i = (b / gx) * BY + r;
+    if (blk == 0 && t == 0) a.ctl[par ^ 1] = next;
+    const int nx = a.nx, ny = a.ny;
+    const int x0 = (int)blockIdx.x * UX - T, y0 = (int)blockIdx.y * UY - T;  // the region's corner
+    if (setup) {
+        // the flow displaces from state `cur`; the level's first warp takes
+        // its initial flow and a zero dual field into state 0
+        const FlowState& st = a.st[c.cur];
+        const bool first = next.warp == 0;
+        for (int q = t; q < UX * UY; q += NT) {
+            const int j = x0 + T + q % UX, i = y0 + T + q / UX;
+            if (j >= nx || i >= ny) continue;
+            const size_t p = (size_t)i * nx + j;
+            const float u = first ? a.u1[p] : st.u1[p], v = first ? a.u2[p] : st.u2[p];
+            if (first) {
+                st.u1[p] = u;
+                st.u2[p] = v;
+                st.p11[p] = st.p12[p] = st.p21[p] = st.p22[p] = 0.f;
+            }
+            warp_px(a.I0, a.I1, a.I1x, a.I1y, u, v, a.wx, a.wy, a.grad, a.rho, i, j, nx, ny);
+        }
+        return;
+    }
+    if (steps == 0) return;  // done
+    const FlowState& in = a.st[src];
+    const FlowState& out = a.st[src ^ 1];
+    const bool test = next.phase == kRun;
+    float u1[PX], u2[PX], p11[PX], p12[PX], p21[PX], p22[PX], gx[PX], gy[PX], g[PX], rc[PX];
+    unsigned flags[PX];  // edge bits, 16: in the image, 32: written
+#pragma unroll
+    for (int q = 0; q < PX; q++) {
+        const int li = t + q * NT, lx = li % RX, ly = li / RX, j = x0 + lx, i = y0 + ly;
+        flags[q] = 0;
+        u1[q] = u2[q] = p11[q] = p12[q] = p21[q] = p22[q] = gx[q] = gy[q] = g[q] = rc[q] = 0.f;
+        if (j >= 0 && i >= 0 && j < nx && i < ny) {
+            const size_t p = (size_t)i * nx + j;
+            u1[q] = in.u1[p];
+            u2[q] = in.u2[p];
+            p11[q] = in.p11[p];
+            p12[q] = in.p12[p];
+            p21[q] = in.p21[p];
+            p22[q] = in.p22[p];
+            gx[q] = a.wx[p];
+            gy[q] = a.wy[p];
+            g[q] = a.grad[p];
+            rc[q] = a.rho[p];
+            flags[q] = 16u | (j == 0 ? 1u : 0u) | (j == nx - 1 ? 2u : 0u) | (i == 0 ? 4u : 0u) | (i == ny - 1 ? 8u : 0u);
+            if (lx >= T && lx < RX - T && ly >= T && ly < RY - T) flags[q] |= 32u;
+        }
+        s_p11[li] = p11[q];
+        s_p12[li] = p12[q];
+        s_p21[li] = p21[q];
+        s_p22[li] = p22[q];
+    }
+    __syncthreads();
+    double es[T] = {};  // this thread's squared changes per iteration
+    auto iterate = [&](auto edge_t) {
+        constexpr bool EDGE = decltype(edge_t)::value;
+#pragma unroll 1
+        for (int k = 0; k < steps; k++) {
             double e = 0.0;
-            if (j < nx && i < ny) e = primal_px(u1, u2, wx, wy, grad, rho_c, p11, p12, p21, p22, i, j, nx, ny, l_t, theta);
-            for (int o = 32; o >= 1; o >>= 1) e += __shfl_xor(e, o, 64);
-            if (lane == 0) s_row[vr] = e;
+#pragma unroll
+            for (int q = 0; q < PX; q++) {
+                const int li = t + q * NT, ll = max(li - 1, 0), lu = li < RX ? li : li - RX;
+                float v1, v2;
+                threshold_px(u1[q], u2[q], gx[q], gy[q], g[q], rc[q], a.l_t, v1, v2);
+                const float n1 = v1 + a.theta * div_px<EDGE>(p11[q], s_p11[ll], p12[q], s_p12[lu], flags[q] & 15u);
+                const float n2 = v2 + a.theta * div_px<EDGE>(p21[q], s_p21[ll], p22[q], s_p22[lu], flags[q] & 15u);
+                if (flags[q] & 32u)
+                    e += (double)((n1 - u1[q]) * (n1 - u1[q]) + (n2 - u2[q]) * (n2 - u2[q]));
+                u1[q] = n1;
+                u2[q] = n2;
+                s_u1[li] = n1;
+                s_u2[li] = n2;
+            }
+#pragma unroll
+            for (int r = 0; r < T; r++) es[r] = k == r ? e : es[r];
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < PX; q++) {
+                const int li = t + q * NT, lr = min(li + 1, RX * RY - 1), ld = li >= RX * (RY - 1) ? li : li + RX;
+                const bool nr = EDGE && (flags[q] & 2u), nd = EDGE && (flags[q] & 8u);
+                dual_px(p11[q], p12[q], nr ? 0.f : s_u1[lr] - u1[q], nd ? 0.f : s_u1[ld] - u1[q], a.taut);
+                dual_px(p21[q], p22[q], nr ? 0.f : s_u2[lr] - u2[q], nd ? 0.f : s_u2[ld] - u2[q], a.taut);
+                s_p11[li] = p11[q];
+                s_p12[li] = p12[q];
+                s_p21[li] = p21[q];
+                s_p22[li] = p22[q];
+            }
+            __syncthreads();
+        }
+    };
+    if (x0 > 0 && y0 > 0 && x0 + RX < nx && y0 + RY < ny) iterate(std::false_type{});
+    else iterate(std::true_type{});
+    if (test) {
+#pragma unroll
+        for (int k = 0; k < T; k++) {
+            const double e = wave_sum(es[k]);
+            if ((t & 63) == 63) s_err[k][t >> 6] = e;
         }
         __syncthreads();
-        for (int b = t; b < nblk; b += 1024) {
-            double acc = 0.0;
-            for (int q = 0; q < BY; q++) acc += s_row[b * BY + q];
-            s_blk[b] = acc;
-        }
-        // dual, every pixel
-        for (int q = t; q < nx * ny; q += 1024) {
-            const int i = q / nx, j = q - i * nx;
-            dual_px(u1, u2, p11, p12, p21, p22, i, j, nx, ny, taut);
-        }
-        __syncthreads();
-        if (t < 256) {
-            double acc = 0.0;
-            for (int q = t; q < nblk; q += 256) acc += s_blk[q];
-            for (int o = 32; o >= 1; o >>= 1) acc += __shfl_xor(acc, o, 64);
-            if (lane == 0) s_w[w] = acc;
-        }
-        __syncthreads();
-        if (t == 0) {
-            double tt = 0.0;
-            for (int q = 0; q < 4; q++) tt += s_w[q];
-            float err = (float)tt;
-            err /= size;
-            s_iter += 1;
-            s_active = (err > eps2 && s_iter < kMaxIter) ? 1 : 0;
-            ctl->error = err;
-        }
     }
-    if (t == 0) {
-        ctl->iter = s_iter;
-        ctl->active = 0;
-        *count = s_iter;
+    if (test && t < steps) {
+        double acc = 0.0;
+        for (int q = 0; q < NT / 64; q++) acc += s_err[t][q];
+        a.part[((size_t)par * T + t) * nblk + blk] = acc;
+    }
+#pragma unroll
+    for (int q = 0; q < PX; q++) {
+        if (!(flags[q] & 32u)) continue;
+        const int li = t + q * NT;
+        const size_t p = (size_t)(y0 + li / RX) * nx + x0 + li % RX;
+        out.u1[p] = u1[q];
+        out.u2[p] = u2[q];
+        out.p11[p] = p11[q];
+        out.p12[p] = p12[q];
+        out.p21[p] = p21[q];
+        out.p22[p] = p22[q];
     }
 }
 
@@ -503,6 +596,48 @@ Taps make_taps(double sigma) {
 }
 
 dim3 grid2(int nx, int ny) { return dim3((unsigned)((nx + BX - 1) / BX), (unsigned)((ny + BY - 1) / BY)); }
+
+// The region and iterations per launch of k_level_step, 512 threads.  A level
+// whose 32 x 16 regions fit a round of the chip (kTestBlocks workgroups) is
+// bound by the latency of an iteration: one pixel per thread, about 2.3 us an
+// iteration with the launch (32 x 32 regions, 4 iterations: 3.1).  A larger
+// one is bound by instruction issue and the halo's share: two pixels per
+// thread of a 32 x 32 region, 4 iterations, 93 us a launch at 1920x1080
+// (the small form 77 for 3; 64 x 32 regions 116, 64 x 48 97, 64 x 64 101).
+struct StepShape {
+    int rx, ry, t;
+};
+constexpr int kStepNT = 512;
+constexpr StepShape kSmallStep = {32, 16, 3}, kLargeStep = {32, 32, 4};
+dim3 step_grid(const StepShape& sh, int nx, int ny) {
+    const int ux = sh.rx - 2 * sh.t, uy = sh.ry - 2 * sh.t;
+    return dim3((unsigned)((nx + ux - 1) / ux), (unsigned)((ny + uy - 1) / uy));
+}
+bool small_step(int nx, int ny) {
+    const dim3 g = step_grid(kSmallStep, nx, ny);
+    return (size_t)g.x * g.y <= (size_t)kTestBlocks;
+}
+// doubles of the sums of a level (two parities)
+size_t step_sums(int nx, int ny) {
+    const StepShape& sh = small_step(nx, ny) ? kSmallStep : kLargeStep;
+    const dim3 g = step_grid(sh, nx, ny);
+    return 2 * (size_t)sh.t * g.x * g.y;
+}
+
+hipError_t launch_step(const LevelArgs& a, int par, hipStream_t s) {
+    if (small_step(a.nx, a.ny)) {
+        constexpr StepShape S = kSmallStep;
+        hipLaunchKernelGGL((k_level_step<S.rx, S.ry, kStepNT, S.t>), step_grid(S, a.nx, a.ny), dim3(kStepNT), 0, s, a,
+                           par);
+    } else {
+        constexpr StepShape S = kLargeStep;
+        const dim3 g = step_grid(S, a.nx, a.ny);
+        if (g.x * g.y > (unsigned)kTestBlocks)
+            hipLaunchKernelGGL((k_level_test<S.t>), dim3(1), dim3(1024), 0, s, a, par, (int)(g.x * g.y));
+        hipLaunchKernelGGL((k_level_step<S.rx, S.ry, kStepNT, S.t>), g, dim3(kStepNT), 0, s, a, par);
+    }
+    return hipGetLastError();
+}
 
 struct Level {
     int nx, ny;
@@ -557,12 +692,13 @@ int tvl1_device(vbm3d_ctx* ctx, const float* I0, const float* I1, float* u, floa
     const size_t n0 = (size_t)nx * ny;
     size_t words = 0;
     for (int k = 0; k < nscales; k++) words += (size_t)L[k].nx * L[k].ny * (k == 0 ? 2 : 4);
-    const int nparts = (int)(grid2(nx, ny).x * grid2(nx, ny).y);
-    const size_t work_planes = 11;  // I1x I1y wx wy grad rho_c p11 p12 p21 p22 tmp
-    // planes, then the iteration partials, the min/max partials and the
-    // control word, each 256-byte aligned
-    const size_t bytes = (words + work_planes * n0) * 4 + (size_t)nparts * 8 + 256 * 4 + 4096 +
-                         (size_t)nscales * warps * 4;
+    // the step launches' sums
+    size_t nparts = 0;
+    for (int k = fscale; k < nscales; k++) nparts = std::max(nparts, step_sums(L[k].nx, L[k].ny));
+    const size_t work_planes = 19;  // I1x I1y wx wy grad rho_c tmp, two states of six planes
+    // planes, then the iterations' sums, the min/max partials, the control
+    // words and the iteration counts, each 256-byte aligned
+    const size_t bytes = (words + work_planes * n0) * 4 + nparts * 8 + 256 * 4 + 4096 + (size_t)nscales * warps * 4;
     void* base = nullptr;
     if (ctx_flow_workspace(ctx, bytes, &base) != hipSuccess)
         return ctx_fail(VBM3D_ERR_NOMEM, "device allocation of the flow workspace failed");
@@ -584,12 +720,17 @@ int tvl1_device(vbm3d_ctx* ctx, const float* I0, const float* I1, float* u, floa
         }
     }
     float *I1x = f, *I1y = f + n0, *wx = f + 2 * n0, *wy = f + 3 * n0, *grad = f + 4 * n0, *rho = f + 5 * n0;
-    float *p11 = f + 6 * n0, *p12 = f + 7 * n0, *p21 = f + 8 * n0, *p22 = f + 9 * n0, *tmp = f + 10 * n0;
+    float* tmp = f + 6 * n0;
+    FlowState st[2];
+    for (int q = 0; q < 2; q++) {
+        float* b = f + (7 + 6 * q) * n0;
+        st[q] = FlowState{b, b + n0, b + 2 * n0, b + 3 * n0, b + 4 * n0, b + 5 * n0};
+    }
     f += work_planes * n0;
     double* part = (double*)(((uintptr_t)f + 255) & ~(uintptr_t)255);
     float* mm = (float*)(part + nparts);  // 64 workgroups x 4 min/max partials
     FlowCtl* ctl = (FlowCtl*)(((uintptr_t)(mm + 256) + 255) & ~(uintptr_t)255);
-    int* counts = (int*)(ctl + 1);  // iterations of the single-workgroup levels, [level][warp]
+    int* counts = (int*)(ctl + 2);  // iterations, [level][warp]
 
     // normalisation and 0.8-sigma pre-smoothing (tvl1flow_lib.c:416-421)
     hipLaunchKernelGGL(k_minmax, dim3(64), dim3(256), 0, s, I0, I1, (long)n0, mm);
@@ -608,7 +749,7 @@ int tvl1_device(vbm3d_ctx* ctx, const float* I0, const float* I1, float* u, floa
             FLOW_TRY(hipMemcpyAsync(wx, src, sz * 4, hipMemcpyDeviceToDevice, s));
             if ((rc = gauss(wx, tmp, L[k - 1].nx, L[k - 1].ny, zsig, s)) != VBM3D_OK) return rc;
             hipLaunchKernelGGL(k_resample, grid2(L[k].nx, L[k].ny), dim3(BX, BY), 0, s, wx, dst, L[k - 1].nx,
-                               L[k - 1].ny, L[k].nx, L[k].ny, zf, zf, 1.f, 0);
+                               L[k - 1].ny, L[k].nx, L[k].ny, zf, zf);
         }
     }
     const long ncoarse = (long)L[nscales - 1].nx * L[nscales - 1].ny;
@@ -617,78 +758,48 @@ int tvl1_device(vbm3d_ctx* ctx, const float* I0, const float* I1, float* u, floa
     FLOW_TRY(hipGetLastError());
 
     const float inv = (float)1.0 / zf, l_t = lambda * theta, taut = tau / theta, eps2 = eps * eps;
-    auto upsample = [&](int k) -> int {
+    auto upsample = [&](int k, bool solved) -> int {
         const float fx = (float)L[k - 1].nx / L[k].nx, fy = (float)L[k - 1].ny / L[k].ny;
-        hipLaunchKernelGGL(k_resample, grid2(L[k - 1].nx, L[k - 1].ny), dim3(BX, BY), 0, s, L[k].u1, L[k - 1].u1,
-                           L[k].nx, L[k].ny, L[k - 1].nx, L[k - 1].ny, fx, fy, inv, 1);
-        hipLaunchKernelGGL(k_resample, grid2(L[k - 1].nx, L[k - 1].ny), dim3(BX, BY), 0, s, L[k].u2, L[k - 1].u2,
-                           L[k].nx, L[k].ny, L[k - 1].nx, L[k - 1].ny, fx, fy, inv, 1);
+        const FlowState plain{L[k].u1, L[k].u2, nullptr, nullptr, nullptr, nullptr};
+        hipLaunchKernelGGL(k_upsample, grid2(L[k - 1].nx, L[k - 1].ny), dim3(BX, BY), 0, s, solved ? ctl : nullptr,
+                           solved ? st[0] : plain, st[1], L[k - 1].u1, L[k - 1].u2, L[k].nx, L[k].ny, L[k - 1].nx,
+                           L[k - 1].ny, fx, fy, inv);
         FLOW_TRY(hipGetLastError());
         return VBM3D_OK;
     };
     int level = 0;
-    FlowCtl host_ctl{};
-    std::vector<char> small_level(nscales, 0);
     for (int k = nscales - 1; k >= fscale; k--, level++) {
         const int lx = L[k].nx, ly = L[k].ny;
         const long sz = (long)lx * ly;
-        const dim3 g = grid2(lx, ly), b(BX, BY);
-        const int np = (int)(g.x * g.y);
-        const bool small = sz <= kSmallPx && np <= kSmallBlocks;
-        small_level[level] = small;
         // one level (tvl1flow_lib.c:96-305)
-        hipLaunchKernelGGL(k_cgrad, g, b, 0, s, L[k].I1, I1x, I1y, lx, ly);
-        for (float* q : {p11, p12, p21, p22}) hipLaunchKernelGGL(k_fill, dim3(256), dim3(256), 0, s, q, sz, 0.f);
+        hipLaunchKernelGGL(k_cgrad, grid2(lx, ly), dim3(BX, BY), 0, s, L[k].I1, I1x, I1y, lx, ly, ctl);
         FLOW_TRY(hipGetLastError());
-        for (int w = 0; w < warps; w++) {
-            hipLaunchKernelGGL(k_warp, g, b, 0, s, L[k].I0, L[k].I1, I1x, I1y, L[k].u1, L[k].u2, wx, wy, grad, rho,
-                               lx, ly);
-            hipLaunchKernelGGL(k_ctl_start, dim3(1), dim3(1), 0, s, ctl);
-            if (small) {
-                hipLaunchKernelGGL(k_iter_small, dim3(1), dim3(1024), 0, s, ctl, L[k].u1, L[k].u2, wx, wy, grad, rho,
-                                   p11, p12, p21, p22, lx, ly, l_t, theta, taut, (float)sz, eps2,
-                                   counts + level * warps + w);
-                FLOW_TRY(hipGetLastError());
-                continue;
-            }
-            int launched = 0;
-            while (launched < kMaxIter) {
-                const int batch = std::min(kMaxIter - launched, launched == 0 ? 24 : 48);
-                for (int it = 0; it < batch; it++) {
-                    hipLaunchKernelGGL(k_iter_primal, g, b, 0, s, ctl, L[k].u1, L[k].u2, wx, wy, grad, rho, p11, p12,
-                                       p21, p22, part, lx, ly, l_t, theta);
-                    if (np <= kFuseBlocks) {
-                        hipLaunchKernelGGL(k_iter_dual_ctl, g, b, 0, s, ctl, L[k].u1, L[k].u2, p11, p12, p21, p22,
-                                           lx, ly, taut, part, np, (float)sz, eps2);
-                        continue;
-                    }
-                    hipLaunchKernelGGL(k_iter_dual, g, b, 0, s, ctl, L[k].u1, L[k].u2, p11, p12, p21, p22, lx, ly,
-                                       taut);
-                    hipLaunchKernelGGL(k_iter_ctl, dim3(1), dim3(256), 0, s, ctl, part, np, (float)sz, eps2);
-                }
-                launched += batch;
-                FLOW_TRY(hipGetLastError());
-                FLOW_TRY(hipMemcpyAsync(&host_ctl, ctl, sizeof(FlowCtl), hipMemcpyDeviceToHost, s));
-                FLOW_TRY(hipStreamSynchronize(s));
-                if (!host_ctl.active) break;
-            }
-            if (iters) iters[level * warps + w] = host_ctl.iter;
+        const LevelArgs la{ctl, part, {st[0], st[1]}, L[k].I0, L[k].I1, I1x, I1y, L[k].u1, L[k].u2, wx, wy, grad, rho,
+                           lx, ly, warps, l_t, theta, taut, (float)sz, eps2, counts + (size_t)level * warps};
+        // The launches follow one another without the host; it looks at the
+        // control word now and then and stops once the level is solved
+        // (launches past that end at once).  The first batch covers a set-up
+        // and about five step launches per warp.
+        FlowCtl host_ctl{};
+        int par = 0;
+        for (int batch = 7 * warps;; batch = 16) {
+            batch = (batch + 1) & ~1;  // the word read below is ctl[0]
+            for (int it = 0; it < batch; it++, par ^= 1) FLOW_TRY(launch_step(la, par, s));
+            FLOW_TRY(hipMemcpyAsync(&host_ctl, ctl, sizeof(FlowCtl), hipMemcpyDeviceToHost, s));
+            FLOW_TRY(hipStreamSynchronize(s));
+            if (host_ctl.phase == kDone) break;
         }
-        if (k == 0) break;
-        if ((rc = upsample(k)) != VBM3D_OK) return rc;
+        if (k == 0) {
+            hipLaunchKernelGGL(k_flow_out, dim3(1024), dim3(256), 0, s, ctl, st[0], st[1], u, v, (long)n0);
+            FLOW_TRY(hipGetLastError());
+            break;
+        }
+        if ((rc = upsample(k, true)) != VBM3D_OK) return rc;
     }
     for (int k = fscale - 1; k >= 1; k--)
-        if ((rc = upsample(k)) != VBM3D_OK) return rc;
-    if (iters) {
-        const int nlev = nscales - fscale;  // levels solved
-        std::vector<int> dev_counts((size_t)nlev * warps);
-        if (!dev_counts.empty())
-            FLOW_TRY(hipMemcpyAsync(dev_counts.data(), counts, dev_counts.size() * 4, hipMemcpyDeviceToHost, s));
-        FLOW_TRY(hipStreamSynchronize(s));
-        for (int lv = 0; lv < nlev; lv++)
-            if (small_level[lv])
-                for (int w = 0; w < warps; w++) iters[lv * warps + w] = dev_counts[(size_t)lv * warps + w];
-    }
+        if ((rc = upsample(k, false)) != VBM3D_OK) return rc;
+    if (iters)
+        FLOW_TRY(hipMemcpyAsync(iters, counts, (size_t)(nscales - fscale) * warps * 4, hipMemcpyDeviceToHost, s));
     FLOW_TRY(hipStreamSynchronize(s));
     return VBM3D_OK;
 }
