@@ -151,8 +151,9 @@ int vbm3d_step(vbm3d_ctx* ctx, int step, float sigma, const float* noisy,
  * frozen and step 2 is linear in the noisy video.  Computes
  * d_grad_noisy = J^T d_grad_out, J the Jacobian of the step-2 output
  * (num/den with the den == 0 fallback of vbm3d_run) with respect to the
- * colour-transformed noisy video.  The groups are recomputed from
- * d_basic (block matching runs twice) rather than stored.  d_final, if
+ * colour-transformed noisy video.  The groups are the forward pass's where
+ * the rings hold the whole clip, and recomputed from d_basic chunk by chunk
+ * where they do not.  d_final, if
  * not NULL, receives the forward output.  Device buffers, [F][C][H][W];
  * enqueued on `stream` (NULL = the context's stream) and synchronised. */
 int vbm3d_step2_adjoint(vbm3d_ctx* ctx, float sigma, const float* d_noisy,

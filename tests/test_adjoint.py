@@ -253,3 +253,26 @@ def test_gpu_sure_sweep(gpu_ctx, torch_dev, cfg5):
     r = res["full"]
     assert np.all(np.abs(r[:, 1] - r[:, 2]) <= 0.1 * r[:, 2] + 1.0)
     assert int(np.argmin(r[:, 1])) == int(np.argmin(r[:, 2]))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("C,k,N,T_2D,T_3D", [(1, 7, 8, 0, 3), (3, 7, 16, 0, 2), (3, 8, 8, 1, 3), (1, 5, 4, 0, 3)])
+def test_adjoint_chunked_equals_whole(monkeypatch, C, k, N, T_2D, T_3D):
+    """The adjoint that takes the forward pass's groups and weights (rings
+    holding the clip) against the one that recomputes them chunk by chunk
+    (a 1 MB ring budget): the same operations, so the same bits."""
+    import torch
+    import vbm3d_amd as V
+    from vbm3d_amd import synth
+    _, noisy = synth.noisy_clip(57, 43, 11, C, 20.0, 61)
+    p2 = V.initialize_parameters_2(20.0, k=k, N=N, T_2D=T_2D, T_3D=T_3D)
+    z = torch.from_numpy(noisy).to("cuda:0")
+    basic = torch.nn.functional.avg_pool2d(z, 3, 1, 1).contiguous()
+    g = torch.from_numpy(np.random.default_rng(5).standard_normal(noisy.shape).astype(np.float32)).to("cuda:0")
+    with V.Context(0) as whole:
+        a = V.step2_adjoint(20.0, z, basic, g, p2, ctx=whole)
+    monkeypatch.setenv("VBM3D_EST_BUDGET_MB", "1")
+    with V.Context(0) as chunked:
+        b = V.step2_adjoint(20.0, z, basic, g, p2, ctx=chunked)
+    assert torch.equal(a, b)
+    assert float(a.abs().max()) > 0

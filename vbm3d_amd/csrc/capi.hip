@@ -453,6 +453,9 @@ struct StepIO {
     bool adjoint;          // step-2 adjoint: num_raw receives J^T gy
     const float* gy;
     const float* den;      // the forward pass's denominator
+    // set by a run whose rings held every frame: groups and weights of the
+    // whole clip are there, and the adjoint run after it takes them
+    bool groups_kept = false;
     // Optional: called before each chunk's launches with the number of
     // leading frames the chunk reads (the host-buffer entry uploads the
     // video while step 1 runs); max_chunk caps the chunk (0 = no cap).
@@ -484,7 +487,7 @@ size_t ring_budget(const vbm3d_ctx* ctx, size_t held) {
     return (size_t)((double)(fr + held) * 0.6);
 }
 
-int run_step(vbm3d_ctx* ctx, const StepIO& io, hipStream_t s) {
+int run_step(vbm3d_ctx* ctx, StepIO& io, hipStream_t s) {
     const vbm3d_params& p = *io.p;
     int rc = check(p, io.W, io.H, io.F, io.C, io.step);
     if (rc) return rc;
@@ -656,6 +659,9 @@ int run_step(vbm3d_ctx* ctx, const StepIO& io, hipStream_t s) {
         ga.mpos = mpos_words ? (uint32_t*)ctx->mpos.p : nullptr;
     }
 
+    const bool kept = io.adjoint && io.groups_kept && S == Fr;
+    io.groups_kept = S == Fr;
+    fa.wgt_kept = kept ? 1 : 0;
     unsigned t_done = 0;
     for (unsigned a = 0; a < Fr; a += S) {
         const unsigned e = std::min(Fr, a + S);
@@ -668,8 +674,9 @@ int run_step(vbm3d_ctx* ctx, const StepIO& io, hipStream_t s) {
         }
         ga.r_begin = bm.r_begin;
         ga.r_end = bm.r_end;
-        HIP_TRY(timed(ctx, 0, io.step, s, [&] { return gen ? launch_bm_gen(ga, s) : launch_bm((int)K, bm, s); }));
-        if (ctx->count)
+        if (!kept)
+            HIP_TRY(timed(ctx, 0, io.step, s, [&] { return gen ? launch_bm_gen(ga, s) : launch_bm((int)K, bm, s); }));
+        if (ctx->count && !kept)
             HIP_TRY(launch_sum_counts(bm.count_out, bm.r_end - bm.r_begin,
                                       (unsigned long long*)ctx->stats.p + 4 * (io.step - 1), s));
         if (io.adjoint)
@@ -1092,7 +1099,7 @@ int plan_batch(vbm3d_ctx* ctx, const vbm3d_clip* clips, int n, int nb, const vbm
                         fa.est = d_est + m.est_base;
                         fa.ms = (int)m.ms;
                         fa.wgt = d_wgt + m.wgt_base;
-                        fa.gy = nullptr; fa.den = nullptr;
+                        fa.gy = nullptr; fa.den = nullptr; fa.wgt_kept = 0;
                         fa.dW = bm.dW; fa.dWHC = bm.dWHC;
                         Cls* cl = nullptr;
                         for (Cls& x : cls)
@@ -1647,7 +1654,8 @@ int vbm3d_step2_adjoint(vbm3d_ctx* ctx, float sigma, const float* d_noisy, const
     io.den_raw = (float*)ctx->den_raw.p;
     rc = run_step(ctx, io, s);
     if (rc) return rc;
-    // transposed pass: the same groups (recomputed), gathered gradient
+    // transposed pass: the same groups (the forward pass's when its rings held
+    // the clip, else recomputed), gathered gradient
     io.adjoint = true;
     io.gy = d_grad_out;
     io.den = (const float*)ctx->den_raw.p;

@@ -154,6 +154,7 @@ struct FArgs {
     Div32 dW, dWHC;      // division by W and by W*H*C
     const float* gy;   // step-2 adjoint: gradient with respect to the output
     const float* den;  // step-2 adjoint: the forward pass's denominator
+    int wgt_kept;      // step-2 adjoint: wgt holds the forward pass's weights
 };
 
 struct AArgs {

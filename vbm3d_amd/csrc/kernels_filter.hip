@@ -457,110 +457,20 @@ __global__ __launch_bounds__(256) void k_filter_queue(const FArgs* __restrict__ 
 // T3^-1 V T3 again for the orthonormal Haar and for the symmetric
 // Hadamard, and of the forward 2D transform F, scaled by w_g.  The
 // per-member results go to `est`; the aggregation kernel in raw mode then
-// sums them over every member patch covering a pixel.  Lane = coefficient
-// (or pixel) index; these are plain FP32 evaluations of the transposed
-// operators, not bit-replays of a reference computation.
+// sums them over every member patch covering a pixel.  These are plain
+// FP32 evaluations of the transposed operators, not bit-replays of a
+// reference computation.
+//
+// The 2D transforms run row-parallel like filter_one's: lane = (member,
+// row), a pass along the row, a transpose through LDS, a pass down the
+// column.  (One lane per coefficient, every member after the other, took
+// 6.08 ms on 32 grey frames 640x360, the forward filter 1.67; this form
+// takes 2.5.)  The aggregation weights are the forward pass's: read from
+// its ring where that still holds the clip (a.wgt_kept), else summed again.
 // ---------------------------------------------------------------------
-// Forward 2D transform of the K x K patch `in` (LDS, row-major) as the
-// forward pass computes it; returns coefficient `lane`.
-template <int K>
-__device__ float adj_fwd2d(const float* in, float* tmp, int lane, bool bior, const Tabs& T) {
-    constexpr int K2 = K * K;
-    const bool act = lane < K2;
-    const int a = lane / K, b = lane - (lane / K) * K;
-    float o = 0.f;
-    if (bior) {
-        if (act) {
-            float m = 0.f;
-            for (int s = 0; s < 8; s++) m = m + in[a * 8 + s] * T.biorF[b * 8 + s];
-            tmp[lane] = m;
-        }
-        wave_sync();
-        if (act)
-            for (int s = 0; s < 8; s++) o = o + tmp[s * 8 + a] * T.biorF[b * 8 + s];
-    } else {
-        // the forward filter's folded passes, so that the Wiener gains
-        // taken from these coefficients are the forward pass's bits
-        if (act) tmp[lane] = dct_fwd_one<K>(in + a * K, 1, b, T.dctF);
-        wave_sync();
-        if (act) o = dct_fwd_one<K>(tmp + b, K, a, T.dctF) * T.nrm[lane];
-    }
-    wave_sync();
-    return o;
-}
-
-// Transpose of the inverse 2D transform applied to the pixel tile `in`;
-// returns coefficient `lane`.  DCT: G(c) = dct_out M (c o inv) M^T with
-// M[x][y] = dctI[x*K+y], so G^T(r) = inv o dct_out (M^T r M).  BIOR:
-// G(c)[u][m] = sum S[u][p] c[q][p] S[m][q] with S = biorI, so
-// G^T(r)[q][p] = sum r[u][m] S[u][p] S[m][q].
-template <int K>
-__device__ float adj_inv2d_T(const float* in, float* tmp, int lane, bool bior, const Tabs& T) {
-    constexpr int K2 = K * K;
-    const bool act = lane < K2;
-    const int a = lane / K, b = lane - (lane / K) * K;
-    float o = 0.f;
-    if (bior) {
-        if (act) {  // t[u][q] = sum_m r[u][m] S[m][q]
-            float m = 0.f;
-            for (int mm = 0; mm < 8; mm++) m = m + in[a * 8 + mm] * T.biorI[mm * 8 + b];
-            tmp[lane] = m;
-        }
-        wave_sync();
-        if (act)  // c'[q = a][p = b] = sum_u S[u][p] t[u][q]
-            for (int u = 0; u < 8; u++) o = o + T.biorI[u * 8 + b] * tmp[u * 8 + a];
-    } else {
-        if (act) {  // t[u][b] = sum_m r[u][m] M[m][b]
-            float m = 0.f;
-            for (int mm = 0; mm < K; mm++) m = m + in[a * K + mm] * T.dctI[mm * K + b];
-            tmp[lane] = m;
-        }
-        wave_sync();
-        if (act) {  // c'[a][b] = inv dct_out sum_u M[u][a] t[u][b]
-            for (int u = 0; u < K; u++) o = o + T.dctI[u * K + a] * tmp[u * K + b];
-            o = T.inv[lane] * T.dct_out * o;
-        }
-    }
-    wave_sync();
-    return o;
-}
-
-// Transpose of the forward 2D transform applied to the coefficient tile
-// `in`; returns pixel `lane`.  DCT: F(x) = nrm o (A x A^T), A = dctF, so
-// F^T(c) = A^T (nrm o c) A.  BIOR: F(x) = B x^T B^T, B = biorF, so
-// F^T(c)[s][q] = sum c[i][j] B[j][s] B[i][q].
-template <int K>
-__device__ float adj_fwd2d_T(const float* in, float* tmp, int lane, bool bior, const Tabs& T) {
-    constexpr int K2 = K * K;
-    const bool act = lane < K2;
-    const int a = lane / K, b = lane - (lane / K) * K;
-    float o = 0.f;
-    if (bior) {
-        if (act) {  // t[i][s] = sum_j c[i][j] B[j][s]
-            float m = 0.f;
-            for (int j = 0; j < 8; j++) m = m + in[a * 8 + j] * T.biorF[j * 8 + b];
-            tmp[lane] = m;
-        }
-        wave_sync();
-        if (act)  // y[s = a][q = b] = sum_i t[i][s] B[i][q]
-            for (int i = 0; i < 8; i++) o = o + tmp[i * 8 + a] * T.biorF[i * 8 + b];
-    } else {
-        if (act) {  // t[u][q] = sum_v nrm[u][v] c[u][v] A[v][q]
-            float m = 0.f;
-            for (int v = 0; v < K; v++) m = m + T.nrm[a * K + v] * in[a * K + v] * T.dctF[v * K + b];
-            tmp[lane] = m;
-        }
-        wave_sync();
-        if (act)  // y[p = a][q = b] = sum_u A[u][p] t[u][q]
-            for (int u = 0; u < K; u++) o = o + T.dctF[u * K + a] * tmp[u * K + b];
-    }
-    wave_sync();
-    return o;
-}
-
 // Group operator of one channel, transposed: Wiener gains from the basic
-// coefficients eg, then T3^-1 V T3 applied to zg in place; v^2 to v2 at
-// the flat index n + kk*nSx.
+// coefficients eg, then T3^-1 V T3 applied to zg in place; v^2 to v2 (unless
+// null) as shrink stores it.
 template <int K, int NS>
 __device__ void adj_group(float* zg, const float* eg, float* v2, int lane, bool had, float sig) {
     constexpr int K2 = K * K;
@@ -581,7 +491,7 @@ __device__ void adj_group(float* zg, const float* eg, float* v2, int lane, bool 
         if (had) value = value * coef;
         value /= (value + s2);
         z[n] = had ? z[n] * value * coef : z[n] * value;
-        if (act) v2[lane * NS + n] = value * value;
+        if (v2 && act) v2[lane * NS + v2_col<NS>(lane, n)] = value * value;
     }
     t3_inv<NS>(z, had);
 #pragma unroll
@@ -589,71 +499,182 @@ __device__ void adj_group(float* zg, const float* eg, float* v2, int lane, bool 
         if (act) zg[n * K2 + lane] = z[n];
 }
 
-__host__ __device__ inline int adjoint_lds_words(int K, int N) { return 2 * K * K + 3 * N * K * K; }
+__host__ __device__ inline int adjoint_lds_words(int K, int N) {
+    return round4((64 / K) * xstride(K)) + 3 * round4(N * K * K);
+}
 
 template <int K, int C>
 __global__ __launch_bounds__(256) void k_filter_adjoint(FArgs a) {
-    constexpr int K2 = K * K;
+    constexpr int K2 = K * K, PB = 64 / K, XS = xstride(K), XP = K + 1;
     extern __shared__ float smem[];
     const int lane = threadIdx.x & 63;
     const int w = threadIdx.x >> 6;
     const int nw = blockDim.x >> 6;
-    const long r = a.r_begin + (long)blockIdx.x * nw + w;
+    const long r = a.r_begin + (long)xcd_order(blockIdx.x, gridDim.x) * nw + w;
     if (r >= a.r_end) return;
-    float* P = smem + (size_t)w * adjoint_lds_words(K, a.N);  // [K2] tile
-    float* Tm = P + K2;                                         // [K2] scratch
-    float* zg = Tm + K2;                                        // [N][K2]
-    float* eg = zg + a.N * K2;                                  // [N][K2]
-    float* v2 = eg + a.N * K2;                                  // [K2*N]
+    float* X = smem + (size_t)w * adjoint_lds_words(K, a.N);  // [PB][XS] transposes
+    const int gw = round4(a.N * K2);
+    float* zg = X + round4(PB * XS);  // [N][K2]
+    float* eg = zg + gw;              // [N][K2]
+    float* v2 = eg + gw;              // [K2*N]
     const unsigned t = (unsigned)(r / a.nrf), i = (unsigned)(r - (long)t * a.nrf);
     const unsigned slot = __builtin_amdgcn_readfirstlane((t % a.ring) * a.nrf + i);
     const unsigned W = a.W, wh = a.wh, whc = a.whc;
     const int nsx = (int)__builtin_amdgcn_readfirstlane(a.nsx[slot]);
     const bool bior = a.T2D == 1, had = a.T3D == 2;
-    const Tabs& T = *a.tabs;
     const uint32_t* mem = a.idx + (size_t)slot * a.N;
-    const bool act = lane < K2;
-    const int pr = lane / K, pc = lane - (lane / K) * K;
-
+    const Div32 dW = {a.dW.m, a.dW.s1, a.dW.s2}, dWHC = {a.dWHC.m, a.dWHC.s1, a.dWHC.s2};
+    typedef const __attribute__((address_space(4))) float cfloat;
+    const cfloat* TF = (const cfloat*)(bior ? a.tabs->biorF : a.tabs->dctF);
+    const cfloat* TI = (const cfloat*)(bior ? a.tabs->biorI : a.tabs->dctI);
+    const cfloat* NRM = (const cfloat*)a.tabs->nrm;
+    const cfloat* INV = (const cfloat*)a.tabs->inv;
+    const cfloat* KAI = (const cfloat*)a.tabs->kaiser;
+    const float dct_out = a.tabs->dct_out;
+    const int nl = lane / K, rr = lane - nl * K;
+    const bool lact = lane < PB * K;
+    // t[v] = sum_q x[q] T[q][v] of a row, stored transposed; then its
+    // column rr of the lane's member
+    auto pass_T = [&](const float (&x)[K], const cfloat* T, float (&col)[K], bool act) {
+        if (act)
+#pragma unroll
+            for (int v = 0; v < K; v++) {
+                float m = 0.f;
+#pragma unroll
+                for (int q = 0; q < K; q++) m = m + x[q] * T[q * K + v];
+                X[nl * XS + v * XP + rr] = m;
+            }
+        wave_sync();
+        if (act)
+#pragma unroll
+            for (int p = 0; p < K; p++) col[p] = X[nl * XS + rr * XP + p];
+        wave_sync();
+    };
     for (int c = 0; c < C; c++) {
-        for (int n = 0; n < nsx; n++) {
-            const unsigned mi = mem[n];
-            const unsigned px = mi % W, py = (mi % wh) / W, pt = mi / whc;
-            const size_t o = (size_t)pt * whc + (size_t)c * wh + (size_t)(py + pr) * W + px + pc;
-            if (act) P[lane] = a.basic[o];
-            wave_sync();
-            const float ev = adj_fwd2d<K>(P, Tm, lane, bior, T);
+        for (int nb0 = 0; nb0 < nsx; nb0 += PB) {
+            const int n = nb0 + nl;
+            const bool act = lact && n < nsx;
+            float x[K], u[K], col[K];
             if (act) {
-                eg[n * K2 + lane] = ev;
-                const float dn = a.den[o];
-                P[lane] = T.kaiser[lane] * (dn != 0.f ? a.gy[o] / dn : 0.f);
+                const unsigned mi = mem[n], pt = div32(mi, dWHC);
+                const unsigned py = div32(mi - pt * whc, dW), px = mi - pt * whc - py * W;
+                const size_t o = (size_t)pt * whc + (size_t)c * wh + (size_t)(py + rr) * W + px;
+#pragma unroll
+                for (int q = 0; q < K; q++) x[q] = a.basic[o + q];
+#pragma unroll
+                for (int q = 0; q < K; q++) {
+                    const float dn = a.den[o + q];
+                    u[q] = KAI[rr * K + q] * (dn != 0.f ? a.gy[o + q] / dn : 0.f);
+                }
+                // the basic patch's coefficients as the forward pass forms
+                // them (filter_one), so that the gains are its bits
+                if (bior) {
+#pragma unroll
+                    for (int v = 0; v < K; v++) {
+                        float m = 0.f;
+#pragma unroll
+                        for (int q = 0; q < K; q++) m = m + x[q] * TF[v * K + q];
+                        X[nl * XS + v * XP + rr] = m;
+                    }
+                } else {
+                    float y[K];
+                    dct_fwd_pass<K>(x, y, TF);
+#pragma unroll
+                    for (int v = 0; v < K; v++) X[nl * XS + v * XP + rr] = y[v];
+                }
             }
             wave_sync();
-            const float zv = adj_inv2d_T<K>(P, Tm, lane, bior, T);
-            if (act) zg[n * K2 + lane] = zv;
-        }
-        wave_sync();
-        switch (nsx) {
-            case 1: adj_group<K, 1>(zg, eg, v2, lane, had, a.sig[c]); break;
-            case 2: adj_group<K, 2>(zg, eg, v2, lane, had, a.sig[c]); break;
-            case 4: adj_group<K, 4>(zg, eg, v2, lane, had, a.sig[c]); break;
-            case 8: adj_group<K, 8>(zg, eg, v2, lane, had, a.sig[c]); break;
-            default: adj_group<K, 16>(zg, eg, v2, lane, had, a.sig[c]); break;
-        }
-        wave_sync();
-        // the group's aggregation weight, summed in the forward pass's order
-        float acc = 0.f;
-        if (lane == 0)
-            for (int f = 0; f < K2 * nsx; f++) acc = acc + v2[f];
-        acc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(acc), 0));
-        const float s2 = a.sig[c] * a.sig[c];
-        const float wg = had ? (acc > 0.0f ? 1.0f / (s2 * acc) : 1.0f) : 1.f / (s2 * acc);
-        float* dst = a.est + (size_t)slot * (unsigned)(a.N * a.ms) + c * K2;
-        for (int n = 0; n < nsx; n++) {
-            if (act) P[lane] = zg[n * K2 + lane];
+            if (act) {
+#pragma unroll
+                for (int p = 0; p < K; p++) col[p] = X[nl * XS + rr * XP + p];
+                if (bior) {
+#pragma unroll
+                    for (int v = 0; v < K; v++) {
+                        float m = 0.f;
+#pragma unroll
+                        for (int p = 0; p < K; p++) m = m + col[p] * TF[v * K + p];
+                        eg[n * K2 + rr * 8 + v] = m;
+                    }
+                } else {
+                    float y[K];
+                    dct_fwd_pass<K>(col, y, TF);
+#pragma unroll
+                    for (int v = 0; v < K; v++) eg[n * K2 + v * K + rr] = y[v] * NRM[v * K + rr];
+                }
+            }
             wave_sync();
-            const float y = adj_fwd2d_T<K>(P, Tm, lane, bior, T);
-            if (act) dst[n * a.ms + lane] = wg * y;
+            // Transpose of the inverse 2D transform.  DCT: G(c) = dct_out M
+            // (c o inv) M^T with M[x][y] = dctI[x*K+y], so G^T(r) = inv o
+            // dct_out (M^T r M).  BIOR: G(c)[u][m] = sum S[u][p] c[q][p]
+            // S[m][q] with S = biorI, so G^T(r)[q][p] = sum r[u][m] S[u][p]
+            // S[m][q].
+            pass_T(u, TI, col, act);
+            if (act)
+#pragma unroll
+                for (int v = 0; v < K; v++) {
+                    float o = 0.f;
+#pragma unroll
+                    for (int p = 0; p < K; p++) o = o + TI[p * K + v] * col[p];
+                    if (bior) zg[n * K2 + rr * 8 + v] = o;
+                    else zg[n * K2 + v * K + rr] = INV[v * K + rr] * dct_out * o;
+                }
+            wave_sync();
+        }
+        const float sg = sig_of(a, c);
+        float* v2c = a.wgt_kept ? nullptr : v2;
+        switch (nsx) {
+            case 1: adj_group<K, 1>(zg, eg, v2c, lane, had, sg); break;
+            case 2: adj_group<K, 2>(zg, eg, v2c, lane, had, sg); break;
+            case 4: adj_group<K, 4>(zg, eg, v2c, lane, had, sg); break;
+            case 8: adj_group<K, 8>(zg, eg, v2c, lane, had, sg); break;
+            default: adj_group<K, 16>(zg, eg, v2c, lane, had, sg); break;
+        }
+        wave_sync();
+        float wg;
+        if (a.wgt_kept) {
+            wg = a.wgt[(size_t)slot * C + c];
+        } else {
+            // the group's weight, summed in the forward pass's order
+            float acc = 0.f;
+            if (lane == 0) switch (nsx) {
+                    case 1: acc = wiener_sum<K, 1>(v2); break;
+                    case 2: acc = wiener_sum<K, 2>(v2); break;
+                    case 4: acc = wiener_sum<K, 4>(v2); break;
+                    case 8: acc = wiener_sum<K, 8>(v2); break;
+                    default: acc = wiener_sum<K, 16>(v2); break;
+                }
+            acc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(acc), 0));
+            const float s2 = sg * sg;
+            wg = had ? (acc > 0.0f ? 1.0f / (s2 * acc) : 1.0f) : 1.f / (s2 * acc);
+        }
+        // Transpose of the forward 2D transform.  DCT: F(x) = nrm o (A x
+        // A^T), A = dctF, so F^T(c) = A^T (nrm o c) A.  BIOR: F(x) = B x^T
+        // B^T, B = biorF, so F^T(c)[s][q] = sum c[i][j] B[j][s] B[i][q].
+        float* dst = a.est + (size_t)slot * (unsigned)(a.N * a.ms) + c * K2;
+        for (int nb0 = 0; nb0 < nsx; nb0 += PB) {
+            const int n = nb0 + nl;
+            const bool act = lact && n < nsx;
+            float x[K], col[K];
+            if (act)
+#pragma unroll
+                for (int q = 0; q < K; q++)
+                    x[q] = bior ? zg[n * K2 + rr * K + q] : NRM[rr * K + q] * zg[n * K2 + rr * K + q];
+            pass_T(x, TF, col, act);
+            if (act)
+#pragma unroll
+                for (int p = 0; p < K; p++) {
+                    float o = 0.f;
+#pragma unroll
+                    for (int q = 0; q < K; q++) o = o + TF[q * K + p] * col[q];
+                    // DCT: col is column rr of t, o = y[p][rr]; BIOR: col is
+                    // t[.][rr], o = y[rr][p]
+                    zg[n * K2 + (bior ? rr * K + p : p * K + rr)] = wg * o;
+                }
+            wave_sync();
+        }
+        for (int q = lane; q < nsx * K2; q += 64) {
+            const int n = q / K2;
+            dst[n * a.ms + (q - n * K2)] = zg[q];
         }
         wave_sync();
     }
