@@ -124,6 +124,38 @@ def test_run_general(oracle, gpu_ctx, case):
     assert synth.psnr(clean, gf) > synth.psnr(clean, noisy) + 3
 
 
+# the fast kernels' temporal forms: smallest and largest patches and slice
+# counts, one and several lane batches of member slices, group sizes that
+# are not powers of two, tiled grids, a clip of kt frames
+KT_CASES = {
+    "k4-kt8": (dict(k=4, kt=8), dict(k=4, kt=8), 1, 1, 9),
+    "k5-kt4-n12-nb2": (dict(k=5, kt=4, N=12), dict(k=5, kt=4, N=12), 1, 2, 7),
+    "k6-kt2-n16": (dict(k=6, kt=2, N=16), dict(k=6, kt=2, N=16, T_3D=2), 3, 1, 6),
+    "k8-kt2-nb4": (dict(k=8, kt=2), dict(k=8, kt=2, T_2D=1), 3, 4, 6),
+    "k7-kt3-f3": (dict(k=7, kt=3), dict(k=7, kt=3, N=1), 1, 1, 3),
+    "npr3-nb1": (dict(kt=2, Npr=3, Nb=1), dict(kt=2, Npr=7, Nb=1), 1, 1, 6),
+}
+
+
+@pytest.mark.parametrize("case", list(KT_CASES), ids=list(KT_CASES))
+def test_run_temporal_forms(oracle, gpu_ctx, case):
+    import vbm3d_amd as V
+    o1, o2, C, nb, F = KT_CASES[case]
+    _, noisy = synth.noisy_clip(97, 65, F, C, 20.0, 36)
+    _run_both(V, oracle, gpu_ctx, noisy, 20.0, V.initialize_parameters_1(20.0, **o1),
+              V.initialize_parameters_2(20.0, **o2), nb=nb)
+
+
+def test_run_temporal_with_flows(oracle, gpu_ctx):
+    """kt = 2 without trajectories, guided by flows."""
+    import vbm3d_amd as V
+    W, H, F = 80, 41, 7
+    _, noisy = synth.noisy_clip(W, H, F, 3, 20.0, 37)
+    ff, bf = motion_flow(F, H, W, 6)
+    _run_both(V, oracle, gpu_ctx, noisy, 20.0, V.initialize_parameters_1(20.0, kt=2),
+              V.initialize_parameters_2(20.0, kt=2), ff=ff, bf=bf)
+
+
 def test_run_mc_with_flows_and_tiled_grid(oracle, gpu_ctx):
     """kt = 3 with motion-compensated trajectories and flows, on the
     single-thread grid and on the 2-crop grid."""

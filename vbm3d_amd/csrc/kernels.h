@@ -136,6 +136,7 @@ struct BMArgs {
     int band;             // grid mode: workgroups in band order (band_order)
 };
 
+struct TabsG;
 struct FArgs {
     const float* noisy;
     const float* basic;  // step 2 only
@@ -155,6 +156,8 @@ struct FArgs {
     const float* gy;   // step-2 adjoint: gradient with respect to the output
     const float* den;  // step-2 adjoint: the forward pass's denominator
     int wgt_kept;      // step-2 adjoint: wgt holds the forward pass's weights
+    int kt;                 // temporal patches (k_filter_kt): slices per patch
+    const TabsG* tabsg;  // and the temporal DCT's tables
 };
 
 struct AArgs {
@@ -307,6 +310,8 @@ inline int bm_shape(const BMArgs& a) { return a.Ns == 7 && a.Npr == 5 && a.Nb ==
 
 hipError_t launch_bm(int K, const BMArgs& a, hipStream_t s);
 hipError_t launch_filter(int K, int step, const FArgs& a, hipStream_t s);
+hipError_t launch_filter_kt(int K, int step, const FArgs& a, hipStream_t s);
+int filter_kt_lds_words(int K, int C, int kt, int N, int step);  // per wave, 4-byte words
 hipError_t launch_aggregate(int C, const AArgs& a, unsigned frames, hipStream_t s);
 
 // Transform micro-benchmark (xform_bench.hip): the k x k DCT on the vector

@@ -449,6 +449,300 @@ __global__ __launch_bounds__(256) void k_filter_queue(const FArgs* __restrict__ 
 }
 
 // ---------------------------------------------------------------------
+// Group filtering of temporal patches (kt > 1 slices at one position in
+// consecutive frames; src/vbm3d.cpp:573-575, 589, 816-831, 1866-1956): the
+// row-parallel form of filter_one over the (member, slice) pairs, with the
+// temporal DCT of each coefficient's slices between the 2D transforms and
+// the transform along the group, in the operation order of k_filter_gen.
+// Bound by instruction issue and by the LDS of the Wiener weights' terms
+// (17.7 KB per wavefront at k 7, kt 2, N 8, three channels).  8 RGB frames
+// 320x240 at kt 2, against k_filter_gen, one lane per coefficient and a
+// member slice at a time: step 2 6.38 -> 1.95 ms, step 1 0.34 -> 0.14.
+// ---------------------------------------------------------------------
+// Words of a v^2 row of ns members: one more, so that the lanes' rows start
+// in different banks.
+__host__ __device__ constexpr int kt_row(int ns) { return ns + 1; }
+__host__ __device__ inline int filter_kt_words(int K, int C, int kt, int N, int step) {
+    const int g = round4(N * K * K * kt);
+    return round4((64 / K) * xstride(K)) + (step == 2 ? 2 : 1) * g +
+           (step == 2 ? C * round4(K * K * kt * kt_row(N)) : 0) + round4(N * kt);
+}
+
+// shrink over K2t coefficients, several per lane; zg, eg are [n][K2t].
+// Returns the number of kept coefficients (step 1).
+template <int NS, int STEP>
+__device__ int shrink_kt(float* zg, float* eg, float* v2, int K2t, int lane, bool had, float lambda, float sig) {
+    const float coef = 1.0f / (float)NS;
+    int cnt = 0;
+    for (int kk = lane; kk < K2t; kk += 64) {
+        float z[NS], e[NS];
+#pragma unroll
+        for (int n = 0; n < NS; n++) {
+            z[n] = zg[n * K2t + kk];
+            if (STEP == 2) e[n] = eg[n * K2t + kk];
+        }
+        t3_fwd<NS>(z, had);
+        if (STEP == 1) {
+            const float thr = had ? lambda * sig * sqrtf((float)NS) : lambda * sig;
+#pragma unroll
+            for (int n = 0; n < NS; n++) {
+                if ((n == 0 && kk == 0) || fabsf(z[n]) > thr) cnt++;
+                else z[n] = 0.f;
+            }
+            t3_inv<NS>(z, had);
+#pragma unroll
+            for (int n = 0; n < NS; n++) zg[n * K2t + kk] = had ? z[n] * coef : z[n];
+        } else {
+            t3_fwd<NS>(e, had);
+            const float s2 = sig * sig;
+#pragma unroll
+            for (int n = 0; n < NS; n++) {
+                float value = e[n] * e[n];
+                if (had) value = value * coef;
+                value /= (value + s2);
+                e[n] = had ? z[n] * value * coef : z[n] * value;
+                v2[kk * kt_row(NS) + n] = value * value;
+            }
+            t3_inv<NS>(e, had);
+#pragma unroll
+            for (int n = 0; n < NS; n++) eg[n * K2t + kk] = e[n];
+        }
+    }
+    return STEP == 1 ? wave_sum_i32(cnt) : 0;
+}
+
+// Sequential sum of a channel's v^2 in the flat order n + kk * NS.
+template <int NS>
+__device__ float wiener_sum_kt(const float* v, int K2t) {
+    float acc = 0.f;
+#pragma unroll 4
+    for (int kk = 0; kk < K2t; kk++)
+#pragma unroll
+        for (int n = 0; n < NS; n++) acc = acc + v[kk * kt_row(NS) + n];
+    return acc;
+}
+
+template <int K, int C, int STEP>
+__global__ __launch_bounds__(256) void k_filter_kt(FArgs a) {
+    constexpr int K2 = K * K, PB = 64 / K, XS = xstride(K), XP = K + 1;
+    extern __shared__ float smem[];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const long r = a.r_begin + (long)xcd_order(blockIdx.x, gridDim.x) * (blockDim.x >> 6) + w;
+    if (r >= a.r_end) return;
+    const int kt = a.kt, K2t = K2 * kt;
+    float* X = smem + (size_t)w * filter_kt_words(K, C, kt, a.N, STEP);
+    const int gw = round4(a.N * K2t), vw = round4(K2t * kt_row(a.N));
+    float* zg = X + round4(PB * XS);     // [n][kt][K2]
+    float* eg = zg + gw;                 // the same (step 2)
+    float* v2 = eg + gw;                 // [C][vw] (step 2)
+    unsigned* s_pos = (unsigned*)(STEP == 2 ? v2 + C * vw : zg + gw);  // [N * kt]
+    const unsigned t = (unsigned)(r / a.nrf), i = (unsigned)(r - (long)t * a.nrf);
+    const unsigned slot = __builtin_amdgcn_readfirstlane((t % a.ring) * a.nrf + i);
+    const unsigned W = a.W, wh = a.wh, whc = a.whc;
+    const int nsx = (int)__builtin_amdgcn_readfirstlane(a.nsx[slot]);
+    const int npair = nsx * kt;  // pair = n * kt + slice
+    const bool bior = a.T2D == 1, had = a.T3D == 2, temporal = !bior;
+    const uint32_t* mem = a.idx + (size_t)slot * a.N;
+    typedef const __attribute__((address_space(4))) float cfloat;
+    const cfloat* TF = (const cfloat*)(bior ? a.tabs->biorF : a.tabs->dctF);
+    const cfloat* TI = (const cfloat*)(bior ? a.tabs->biorI : a.tabs->dctI);
+    const cfloat* NRM = (const cfloat*)a.tabs->nrm;
+    const cfloat* INV = (const cfloat*)a.tabs->inv;
+    const cfloat* tF = (const cfloat*)a.tabsg->tF;
+    const cfloat* tI = (const cfloat*)a.tabsg->tI;
+    const float tnorm = a.tabsg->tnorm, dct_out = a.tabs->dct_out;
+    const Div32 dWHC = {a.dWHC.m, a.dWHC.s1, a.dWHC.s2};
+    const int nl = lane / K, rr = lane - nl * K;
+    const bool lact = lane < PB * K;
+    float wsel = 0.f;
+    // the pairs' corners, so that a batch's rows wait for no index load
+    for (int pi = lane; pi < npair; pi += 64) {
+        const int n = small_div(pi, kt);
+        const unsigned mi = mem[n], pt = div32(mi, dWHC);
+        s_pos[pi] = (pt + (unsigned)(pi - n * kt)) * whc + (mi - pt * whc);
+    }
+    wave_sync();
+    for (int c = 0; c < C; c++) {
+        for (int pb0 = 0; pb0 < npair; pb0 += PB) {
+            const int pi = pb0 + nl;
+            const bool act = lact && pi < npair;
+            // both sources' rows are loaded before the first is used
+            float x[STEP][K];
+            if (act) {
+                const size_t o = (size_t)s_pos[pi] + (size_t)c * wh + (size_t)rr * W;
+#pragma unroll
+                for (int g = 0; g < STEP; g++)
+#pragma unroll
+                    for (int q = 0; q < K; q++) x[g][q] = (g == 0 ? a.noisy : a.basic)[o + q];
+            }
+#pragma unroll
+            for (int g = 0; g < STEP; g++) {
+                float* dst = g == 0 ? zg : eg;
+                if (act) {
+                    if (bior) {
+#pragma unroll
+                        for (int v = 0; v < K; v++) {
+                            float m = 0.f;
+#pragma unroll
+                            for (int q = 0; q < K; q++) m = m + x[g][q] * TF[v * K + q];
+                            X[nl * XS + v * XP + rr] = m;
+                        }
+                    } else {
+                        float y[K];
+                        dct_fwd_pass<K>(x[g], y, TF);
+#pragma unroll
+                        for (int v = 0; v < K; v++) X[nl * XS + v * XP + rr] = y[v];
+                    }
+                }
+                wave_sync();
+                if (act) {
+                    float col[K];
+#pragma unroll
+                    for (int p = 0; p < K; p++) col[p] = X[nl * XS + rr * XP + p];
+                    if (bior) {
+#pragma unroll
+                        for (int u = 0; u < K; u++) {
+                            float m = 0.f;
+#pragma unroll
+                            for (int p = 0; p < K; p++) m = m + col[p] * TF[u * K + p];
+                            dst[pi * K2 + rr * 8 + u] = m;
+                        }
+                    } else {
+                        float y[K];
+                        dct_fwd_pass<K>(col, y, TF);
+#pragma unroll
+                        for (int u = 0; u < K; u++) dst[pi * K2 + u * K + rr] = y[u] * NRM[u * K + rr];
+                    }
+                }
+                wave_sync();
+            }
+        }
+        for (int g = 0; g < STEP; g++) {
+            float* dst = g == 0 ? zg : eg;
+            if (temporal) {  // along each coefficient's slices
+                for (int e = lane; e < K2 * nsx; e += 64) {
+                    const int n = e / K2;
+                    float* x = dst + n * K2t + (e - n * K2);
+                    float v[kGenMaxKt];
+#pragma unroll
+                    for (int q = 0; q < kGenMaxKt; q++) v[q] = q < kt ? x[q * K2] : 0.f;
+#pragma unroll
+                    for (int u = 0; u < kGenMaxKt; u++)
+                        if (u < kt) {
+                            float m = 0.f;
+#pragma unroll
+                            for (int q = 0; q < kGenMaxKt; q++)
+                                if (q < kt) m = m + v[q] * tF[u * kt + q];
+                            x[u * K2] = u == 0 ? (float)((double)(m * tnorm) * 0.7071067811865475) : m * tnorm;
+                        }
+                }
+                wave_sync();
+            }
+        }
+        float* v2c = v2 + c * vw;
+        const float sg = sig_of(a, c);
+        int cnt;
+        switch (nsx) {
+            case 1: cnt = shrink_kt<1, STEP>(zg, eg, v2c, K2t, lane, had, a.lambda, sg); break;
+            case 2: cnt = shrink_kt<2, STEP>(zg, eg, v2c, K2t, lane, had, a.lambda, sg); break;
+            case 4: cnt = shrink_kt<4, STEP>(zg, eg, v2c, K2t, lane, had, a.lambda, sg); break;
+            case 8: cnt = shrink_kt<8, STEP>(zg, eg, v2c, K2t, lane, had, a.lambda, sg); break;
+            default: cnt = shrink_kt<16, STEP>(zg, eg, v2c, K2t, lane, had, a.lambda, sg); break;
+        }
+        if (STEP == 1 && lane == c) wsel = 1.f / (sg * sg * (float)cnt);
+        wave_sync();
+        float* est = STEP == 2 ? eg : zg;
+        if (temporal) {
+            for (int e = lane; e < K2 * nsx; e += 64) {
+                const int n = e / K2;
+                float* x = est + n * K2t + (e - n * K2);
+                float z[kGenMaxKt];
+#pragma unroll
+                for (int u = 0; u < kGenMaxKt; u++) z[u] = u < kt ? x[u * K2] : 0.f;
+                z[0] = (float)((double)z[0] * 1.414213562373095);
+#pragma unroll
+                for (int q = 0; q < kGenMaxKt; q++)
+                    if (q < kt) {
+                        float m = 0.f;
+#pragma unroll
+                        for (int u = 0; u < kGenMaxKt; u++)
+                            if (u < kt) m = m + z[u] * tI[q * kt + u];
+                        x[q * K2] = m * tnorm;
+                    }
+            }
+            wave_sync();
+        }
+        for (int pb0 = 0; pb0 < npair; pb0 += PB) {
+            const int pi = pb0 + nl;
+            const bool act = lact && pi < npair;
+            if (act) {
+                float x[K];
+#pragma unroll
+                for (int q = 0; q < K; q++)
+                    x[q] = bior ? est[pi * K2 + q * 8 + rr] : est[pi * K2 + rr * K + q] * INV[rr * K + q];
+                if (bior) {
+#pragma unroll
+                    for (int v = 0; v < K; v++) {
+                        float m = 0.f;
+#pragma unroll
+                        for (int q = 0; q < K; q++) m = m + x[q] * TI[v * K + q];
+                        X[nl * XS + v * XP + rr] = m;
+                    }
+                } else {
+                    float y[K];
+                    dct_inv_pass<K>(x, y, TI);
+#pragma unroll
+                    for (int v = 0; v < K; v++) X[nl * XS + v * XP + rr] = y[v];
+                }
+            }
+            wave_sync();
+            if (act) {
+                float col[K];
+#pragma unroll
+                for (int p = 0; p < K; p++) col[p] = X[nl * XS + rr * XP + p];
+                if (bior) {
+#pragma unroll
+                    for (int u = 0; u < K; u++) {
+                        float m = 0.f;
+#pragma unroll
+                        for (int p = 0; p < K; p++) m = m + col[p] * TI[u * K + p];
+                        est[pi * K2 + u * K + rr] = m;
+                    }
+                } else {
+                    float y[K];
+                    dct_inv_pass<K>(col, y, TI);
+#pragma unroll
+                    for (int u = 0; u < K; u++) est[pi * K2 + u * K + rr] = dct_out * y[u];
+                }
+            }
+            wave_sync();
+        }
+        // est[slot][n][c][slice][pixel]
+        float* dstg = a.est + (size_t)slot * (unsigned)(a.N * a.ms) + c * K2t;
+        for (int n = 0; n < nsx; n++)
+            for (int q = lane; q < K2t; q += 64) dstg[n * a.ms + q] = est[n * K2t + q];
+        wave_sync();
+    }
+    if (STEP == 2) {
+        if (lane < C) {
+            const float* vc = v2 + lane * vw;
+            float acc;
+            switch (nsx) {
+                case 1: acc = wiener_sum_kt<1>(vc, K2t); break;
+                case 2: acc = wiener_sum_kt<2>(vc, K2t); break;
+                case 4: acc = wiener_sum_kt<4>(vc, K2t); break;
+                case 8: acc = wiener_sum_kt<8>(vc, K2t); break;
+                default: acc = wiener_sum_kt<16>(vc, K2t); break;
+            }
+            const float sg = sig_of(a, lane), s2 = sg * sg;
+            a.wgt[(size_t)slot * C + lane] = had ? (acc > 0.0f ? 1.0f / (s2 * acc) : 1.0f) : 1.f / (s2 * acc);
+        }
+    } else if (lane < C) {
+        a.wgt[(size_t)slot * C + lane] = wsel;
+    }
+}
+
+// ---------------------------------------------------------------------
 // Adjoint of step 2 with the groups, Wiener gains and weights frozen by
 // the basic estimate.  Step 2 is then linear in the noisy video:
 //   final = D^-1 sum_g Agg_g (kaiser w_g) G T3^-1 V_g T3 F Gather_g z,
@@ -719,6 +1013,42 @@ hipError_t launch_filter(int K, int step, const FArgs& a, hipStream_t s) {
         default: return hipErrorInvalidValue;
     }
 }
+
+template <int K, int C, int STEP>
+static hipError_t filter_kt_k(const FArgs& a, hipStream_t s) {
+    const long n = a.r_end - a.r_begin;
+    if (n <= 0) return hipSuccess;
+    const size_t per_wave = (size_t)filter_kt_words(K, C, a.kt, a.N, STEP) * 4;
+    if (per_wave > 64 * 1024) return hipErrorInvalidValue;
+    // the workgroup that leaves most wavefronts on a CU's 160 KB of LDS
+    int waves = 1, best = 0;
+    for (int v = 1; v <= 4 && per_wave * v <= 64 * 1024; v++) {
+        const int on = (int)(160 * 1024 / (per_wave * v)) * v;
+        if (on >= best) best = on, waves = v;
+    }
+    hipLaunchKernelGGL((k_filter_kt<K, C, STEP>), dim3((unsigned)((n + waves - 1) / waves)), dim3(64 * waves),
+                       per_wave * waves, s, a);
+    return hipGetLastError();
+}
+
+template <int K>
+static hipError_t filter_kt_kc(int step, const FArgs& a, hipStream_t s) {
+    if (a.C == 1) return step == 1 ? filter_kt_k<K, 1, 1>(a, s) : filter_kt_k<K, 1, 2>(a, s);
+    return step == 1 ? filter_kt_k<K, 3, 1>(a, s) : filter_kt_k<K, 3, 2>(a, s);
+}
+
+hipError_t launch_filter_kt(int K, int step, const FArgs& a, hipStream_t s) {
+    switch (K) {
+        case 4: return filter_kt_kc<4>(step, a, s);
+        case 5: return filter_kt_kc<5>(step, a, s);
+        case 6: return filter_kt_kc<6>(step, a, s);
+        case 7: return filter_kt_kc<7>(step, a, s);
+        case 8: return filter_kt_kc<8>(step, a, s);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+int filter_kt_lds_words(int K, int C, int kt, int N, int step) { return filter_kt_words(K, C, kt, N, step); }
 
 template <int K>
 static hipError_t filter_adj_k(const FArgs& a, hipStream_t s) {
