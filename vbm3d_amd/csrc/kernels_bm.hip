@@ -74,11 +74,20 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
     const unsigned rt = div32(ridx, dWHC), ry = div32(ridx - rt * whc, dW), rx = ridx - rt * whc - ry * W;
     const float norm = (float)(unsigned)(K * K * a.kt * C);
     constexpr int K2 = K * K;
+    // Positions are kept as x | y << 16 (a pick's frame follows from where it
+    // stands in the list of picks), so that windows, candidates and the
+    // already-seen test are packed 16-bit operations, with no division or
+    // 32-bit multiplication before the picks' indices at the end.
+    typedef unsigned short ushort2v __attribute__((ext_vector_type(2)));
+    auto pk = [](unsigned v) { return __builtin_bit_cast(ushort2v, v); };
+    auto un = [](ushort2v v) { return __builtin_bit_cast(unsigned, v); };
+    const unsigned ref2 = rx | (ry << 16);
 
     // The reference patch is wave-uniform: read it through the constant
     // address space so it arrives in scalar registers (SMEM loads) and
     // costs neither LDS bandwidth nor vector issue slots.
     typedef const __attribute__((address_space(4))) float cfloat;
+    typedef __attribute__((address_space(3))) float lds_float;
     float* refp = base + L.ref;  // the reference patch, [c][y][x] (general form only)
     for (int i = lane; i < (L.piped ? 0 : K2 * C); i += 64) {
         const int c = i / K2, e = i - c * K2;
@@ -90,16 +99,22 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
     // (KT: added to `acc`, of the slice `so` words on.)
     auto ssd = [&](const float* t, int tp, int cs, float acc = 0.f, unsigned so = 0u) -> float {
 #pragma unroll
-        for (int c = 0; c < C; ++c)
+        for (int c = 0; c < C; ++c) {
+            // one LDS address per channel, kept opaque: every sample of the
+            // channel is then an immediate offset from it
+            unsigned tc = (unsigned)(size_t)(const lds_float*)t + (unsigned)(c * cs * 4);
+            if (C > 1) asm volatile("" : "+v"(tc));
+            const lds_float* tl = (const lds_float*)(size_t)tc;
 #pragma unroll
             for (int y = 0; y < K; ++y) {
                 cfloat* row = (cfloat*)(vid + ridx + (KT ? so : 0u) + c * wh + y * W);
 #pragma unroll
                 for (int x = 0; x < K; ++x) {
-                    const float dif = row[x] - t[c * cs + y * tp + x];
+                    const float dif = row[x] - tl[y * tp + x];
                     acc = acc + dif * dif;
                 }
             }
+        }
         return acc;
     };
     // two candidates at once: independent accumulators, shared reference
@@ -144,7 +159,7 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
         const int wx = x1 - x0 + 1, wy = y1 - y0 + 1, m = wx * wy;
         const int cs = L.tp0 * L.th0;
         float ss = 0.f;
-        const int lx = lane % wx, ly = lane / wx;
+        const int ly = small_div(lane, wx), lx = lane - ly * wx;
         for (unsigned ht = 0; ht < (KT ? (unsigned)a.kt : 1u); ht++) {
             // the (wx+K-1) x (wy+K-1) area, memory to LDS: word e = k*64 +
             // lane of a channel's area is its row e / tp0, column e % tp0
@@ -182,7 +197,7 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
             const float s = ss / norm;
             const unsigned qx = x0 + lx, qy = y0 + ly;
             c_d[lane] = s - ((qx == rx && qy == ry) ? a.d : 0.f);
-            c_i[lane] = rt * whc + qy * W + qx;
+            c_i[lane] = qx | (qy << 16);
         }
         wave_sync();
         n_eval += m;
@@ -220,45 +235,50 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
         const int nfr[2] = {nfw, nbw};
         uint32_t* lst = (uint32_t*)c_d;  // c_d and c_i, adjacent: 128 entries
         // windows of frame f of both chains: flow projection of the chain's
-        // current matches (x first, then y at the updated x), clamped
-        // Npr x Npr box in the next frame.  Lane wn < 2 Nb keeps window wn
-        // in registers (x0, y0, width, height, frame), which the copies and
-        // the slot list read with readlane: no LDS round trip.
-        int wx0 = 0, wy0 = 0, wwx = 0, wwy = 0, wfr = 0;
+        // current matches (x first, then y at the updated x; without a flow
+        // the matches' own positions), clamped Npr x Npr box in the next
+        // frame.  Lane wn < 2 Nb keeps window wn in registers (its corner and
+        // its extent less one, packed), which the copies and the slot list
+        // read with readlane: no LDS round trip.
+        const unsigned hs2 = (unsigned)hs * 0x10001u, lim2 = (W - K) | ((H - K) << 16);
+        const unsigned full = (unsigned)(Npr - 1) * 0x10001u;  // extent of an unclipped window
+        unsigned wP = 0, wS = 0;
         auto windows = [&](int f) {
             if (lane < 2 * Nb) {
                 const int ch = lane >= Nb ? 1 : 0, m = lane - ch * Nb;
                 if (f < nfr[ch]) {
-                    const int dir = ch == 0 ? 1 : -1;
                     const float* fl = ch == 0 ? a.ff : a.bf;
-                    const unsigned mi = pp[(ch == 0 ? 8 : 0) + m];
-                    const unsigned pt = div32(mi, dWHC);
-                    unsigned py = div32(mi - pt * whc, dW), px = mi - pt * whc - py * W;
-                    const unsigned ft = ch == 0 ? pt : pt - 1;
-                    const unsigned hk = K / 2;
-                    const float fx = fl ? fl[(size_t)ft * 2 * wh + (py + hk) * W + px + hk] : 0.f;
-                    px = (unsigned)min(max((int)((float)px + roundf(fx)), 0), (int)(W - K));
-                    const float fy = fl ? fl[(size_t)ft * 2 * wh + wh + (py + hk) * W + px + hk] : 0.f;
-                    py = (unsigned)min(max((int)((float)py + roundf(fy)), 0), (int)(H - K));
-                    const int x0 = max(0, (int)px - hs), y0 = max(0, (int)py - hs);
-                    wx0 = x0;
-                    wy0 = y0;
-                    wwx = min((int)W - K, (int)px + hs) - x0 + 1;
-                    wwy = min((int)H - K, (int)py + hs) - y0 + 1;
-                    wfr = (int)(pt + dir);
+                    unsigned p = pp[(ch == 0 ? 8 : 0) + m];
+                    if (fl) {
+                        unsigned px = p & 0xFFFFu, py = p >> 16;
+                        const unsigned ft = ch == 0 ? rt + f : rt - f - 1;
+                        const unsigned hk = K / 2;
+                        const float fx = fl[(size_t)ft * 2 * wh + (py + hk) * W + px + hk];
+                        px = (unsigned)min(max((int)((float)px + roundf(fx)), 0), (int)(W - K));
+                        const float fy = fl[(size_t)ft * 2 * wh + wh + (py + hk) * W + px + hk];
+                        py = (unsigned)min(max((int)((float)py + roundf(fy)), 0), (int)(H - K));
+                        p = px | (py << 16);
+                    }
+                    const ushort2v lo = __builtin_elementwise_sub_sat(pk(p), pk(hs2));
+                    const ushort2v hi =
+                        __builtin_elementwise_min(__builtin_elementwise_add_sat(pk(p), pk(hs2)), pk(lim2));
+                    wP = un(lo);
+                    wS = un(hi - lo);
                 }
             }
             wave_sync();
         };
         // a (window, channel) area is th1 rows of pitch tp1 (at most 192
         // words); word e = k*64 + lane sits at row e / tp1, column e % tp1
+        // (an unclipped window needs no test for the area's words: the lanes
+        // in the pitch's spare columns read the last column again)
         int er[3], ec[3];
         unsigned goff[3];  // byte offset in the frame
 #pragma unroll
         for (int k = 0; k < 3; k++) {
             er[k] = small_div(k * 64 + lane, L.tp1);
             ec[k] = k * 64 + lane - er[k] * L.tp1;
-            goff[k] = ((unsigned)er[k] * W + (unsigned)ec[k]) * 4u;
+            goff[k] = ((unsigned)er[k] * W + (unsigned)min(ec[k], L.th1 - 1)) * 4u;
         }
         const unsigned tile_lds = lds_addr(tile);
         // slot lane of a chain: window m = lane / P2p, position l = ly*Npr + lx
@@ -266,6 +286,10 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
         // keep its raster order)
         const int sm = lane >> lg2, sl = lane & (P2p - 1);
         const int sly = small_div(sl, Npr), slx = sl - sly * Npr;
+        // packed position in the window (beyond any window where the lane has
+        // no slot), and the chain 0 list entry
+        const unsigned slp = sm < Nb && sl < P2 ? (unsigned)slx | ((unsigned)sly << 16) : 0xFFFFFFFFu;
+        const unsigned ent0 = ((unsigned)lane << 16) | (unsigned)(sm * L.ws + sly * L.tp1 + slx);
         if (nst > 0) windows(0);
         for (int f = 0; f < nst; f++) {
             const bool act[2] = {f < nfw, f < nbw};
@@ -283,11 +307,9 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
                     for (int m = 0; m < 2; m++) {
                         if (!act[ch] || m >= Nb) continue;
                         const int wn = ch * Nb + m;
-                        const int aw = __builtin_amdgcn_readlane(wwx, wn) + K - 1;
-                        const int ah = __builtin_amdgcn_readlane(wwy, wn) + K - 1;
-                        unsigned fb = ((unsigned)__builtin_amdgcn_readlane(wfr, wn) + (KT ? ht : 0u)) * whc +
-                                      (unsigned)__builtin_amdgcn_readlane(wy0, wn) * W +
-                                      (unsigned)__builtin_amdgcn_readlane(wx0, wn);
+                        const unsigned P = __builtin_amdgcn_readlane(wP, wn), S = __builtin_amdgcn_readlane(wS, wn);
+                        unsigned fb = ((ch == 0 ? rt + 1 + f : rt - 1 - f) + (KT ? ht : 0u)) * whc + (P >> 16) * W +
+                                      (P & 0xFFFFu);
                         if (KT) fb = __builtin_amdgcn_readfirstlane(fb);
                         // one scalar base per channel, kept opaque so that
                         // the copies take the scalar-base form (no 64-bit
@@ -300,17 +322,27 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
                             asm volatile("" : "+s"(lo), "+s"(hi));
                             cb[c] = (const char*)(((unsigned long long)hi << 32) | lo);
                         }
+                        auto put = [&](int k) __attribute__((always_inline)) {
+                            // a 32-bit lane offset at the copy (not a hoisted
+                            // 64-bit one) keeps the scalar-base form
+                            unsigned go = goff[k];
+                            asm volatile("" : "+v"(go));
 #pragma unroll
-                        for (int k = 0; k < 3; k++) {
-                            if (k * 64 >= ne) break;
-                            if (er[k] < ah && ec[k] < aw) {
-                                // a 32-bit lane offset at the copy (not a
-                                // hoisted 64-bit one) keeps the scalar-base form
-                                unsigned go = goff[k];
-                                asm volatile("" : "+v"(go));
+                            for (int c = 0; c < C; c++)
+                                lds_dma(cb[c] + go, tl + (unsigned)((wn * L.ws + c * cs1 + k * 64) * 4));
+                        };
+                        if (S == full) {  // wave-uniform
 #pragma unroll
-                                for (int c = 0; c < C; c++)
-                                    lds_dma(cb[c] + go, tl + (unsigned)((wn * L.ws + c * cs1 + k * 64) * 4));
+                            for (int k = 0; k < 3; k++) {
+                                if (k * 64 >= ne) break;
+                                if (k * 64 + 64 <= ne || lane < ne - k * 64) put(k);
+                            }
+                        } else {
+                            const int aw = (int)(S & 0xFFFFu) + K, ah = (int)(S >> 16) + K;
+#pragma unroll
+                            for (int k = 0; k < 3; k++) {
+                                if (k * 64 >= ne) break;
+                                if (er[k] < ah && ec[k] < aw) put(k);
                             }
                         }
                     }
@@ -329,25 +361,17 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
                 // wave-uniform; lanes of window 1 select its values, and a
                 // candidate inside window 0 was seen
                 const int ia = h * Nb, ib = h * Nb + (Nb > 1 ? 1 : 0);
-                const int ax0 = __builtin_amdgcn_readlane(wx0, ia), ay0 = __builtin_amdgcn_readlane(wy0, ia);
-                const int awx = __builtin_amdgcn_readlane(wwx, ia), awy = __builtin_amdgcn_readlane(wwy, ia);
-                const int bx0 = __builtin_amdgcn_readlane(wx0, ib), by0 = __builtin_amdgcn_readlane(wy0, ib);
-                const int bwx = __builtin_amdgcn_readlane(wwx, ib), bwy = __builtin_amdgcn_readlane(wwy, ib);
+                const unsigned aP = __builtin_amdgcn_readlane(wP, ia), aS = __builtin_amdgcn_readlane(wS, ia);
+                const unsigned bP = __builtin_amdgcn_readlane(wP, ib), bS = __builtin_amdgcn_readlane(wS, ib);
                 const bool m1 = sm == 1;
-                const int x0 = m1 ? bx0 : ax0, y0 = m1 ? by0 : ay0;
-                const int wx = m1 ? bwx : awx, wy = m1 ? bwy : awy;
-                const int qx = x0 + slx, qy = y0 + sly;
-                const bool seen = m1 & (qx >= ax0) & (qx < ax0 + awx) & (qy >= ay0) & (qy < ay0 + awy);
-                const bool valid = act[h] & (sm < Nb) & (sl < P2) & (slx < wx) & (sly < wy) & !seen;
-                unsigned ent = 0;
-                if (valid) {
-                    const int wn = h * Nb + sm;
-                    const unsigned toff = (unsigned)(wn * L.ws + sly * L.tp1 + slx);
-                    const bool self = (unsigned)qx == rx && (unsigned)qy == ry;
-                    ent = ((unsigned)(h * 64 + lane) << 16) | (self ? 0x8000u : 0u) | toff;
-                    const int fr = m1 ? __builtin_amdgcn_readlane(wfr, ib) : __builtin_amdgcn_readlane(wfr, ia);
-                    s_i[h * 64 + lane] = (unsigned)fr * whc + qy * W + qx;
-                }
+                const unsigned q = un(pk(m1 ? bP : aP) + pk(slp));
+                const bool in = un(__builtin_elementwise_min(pk(slp), pk(m1 ? bS : aS))) == slp;
+                const unsigned dq = un(pk(q) - pk(aP));
+                const bool seen = m1 & (un(__builtin_elementwise_min(pk(dq), pk(aS))) == dq);
+                const bool valid = act[h] & in & !seen;
+                const unsigned ent = (ent0 + ((unsigned)(h * 64) << 16) + (unsigned)(h * Nb * L.ws)) |
+                                     (q == ref2 ? 0x8000u : 0u);
+                if (valid) s_i[h * 64 + lane] = q;
                 bal[h] = __ballot(valid);
                 if (valid) lst[(h ? __popcll(bal[0]) : 0) + lanes_below(bal[h], lane)] = ent;
             }
@@ -456,9 +480,9 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
             if (act[ch]) {
                 const int dir = ch == 0 ? 1 : -1;
                 const float* fl = ch == 0 ? a.ff : a.bf;
-                const unsigned mi = pp[(ch == 0 ? 8 : 0) + m];
-                const unsigned pt = div32(mi, dWHC);
-                unsigned py = div32(mi - pt * whc, dW), px = mi - pt * whc - py * W;
+                const unsigned p = pp[(ch == 0 ? 8 : 0) + m];
+                const unsigned pt = ch == 0 ? rt + f : rt - f;
+                unsigned py = p >> 16, px = p & 0xFFFFu;
                 const unsigned ft = ch == 0 ? pt : pt - 1;
                 const unsigned hk = K / 2;
                 const float fx = fl ? fl[(size_t)ft * 2 * wh + (py + hk) * W + px + hk] : 0.f;
@@ -485,7 +509,6 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
         for (int b0 = 0; b0 < nslots; b0 += 128) {
             bool valid[2] = {false, false};
             int toff[2] = {0, 0}, qxs[2] = {0, 0}, qys[2] = {0, 0};
-            unsigned tfs[2] = {0, 0};
 #pragma unroll
             for (int h = 0; h < 2; h++) {
                 const int s = b0 + 64 * h + lane;
@@ -506,7 +529,6 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
                             toff[h] = wn * L.ws + ly * L.tp1 + lx;
                             qxs[h] = qx;
                             qys[h] = qy;
-                            tfs[h] = (unsigned)win[wn * 5 + 4];
                         }
                     }
                 }
@@ -520,7 +542,7 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
                     const int s = b0 + 64 * h + lane;
                     if (valid[h]) {
                         s_d[s] = sv[h] / norm - (((unsigned)qxs[h] == rx && (unsigned)qys[h] == ry) ? a.d : 0.f);
-                        s_i[s] = tfs[h] * whc + qys[h] * W + qxs[h];
+                        s_i[s] = (unsigned)qxs[h] | ((unsigned)qys[h] << 16);
                     }
                 }
             }
@@ -565,6 +587,15 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
         }
     }
     nbest = Nb * (1 + nfw + nbw);
+    // the picks' indices: Nb of the reference frame, then of every forward
+    // frame, then of every backward frame
+    if (lane < nbest) {
+        const int g = small_div(lane, Nb);
+        const unsigned tf = g <= nfw ? rt + (unsigned)g : rt - (unsigned)(g - nfw);
+        const unsigned p = b_i[lane];
+        b_i[lane] = tf * whc + (p >> 16) * W + (p & 0xFFFFu);
+    }
+    wave_sync();
 
     // -- N best overall, tau cut, power-of-two group size
     //    (src/vbm3d.cpp:1169-1184)
