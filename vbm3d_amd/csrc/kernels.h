@@ -38,7 +38,7 @@ __host__ __device__ inline uint32_t div32(uint32_t n, Div32 v) {
     return (t + ((n - t) >> v.s1)) >> v.s2;
 }
 
-__host__ __device__ inline int pow2ceil(int v) {
+__host__ __device__ constexpr int pow2ceil(int v) {
     int r = 1;
     while (r < v) r *= 2;
     return r;
@@ -65,8 +65,9 @@ struct BMLay {
     int ref, tile, sd, si, sv, cd, ci, bd, bi, fd, fi, od, oi, scr, pp, win, total;
 };
 
-__host__ __device__ inline BMLay bm_layout(int K, int C, int Ns, int Npr, int Nb, int Nf) {
-    BMLay L;
+constexpr int kBMLists = 232;  // words of the paired form beside its tile, at Nf 4 and Nb 2
+__host__ __device__ constexpr BMLay bm_layout(int K, int C, int Ns, int Npr, int Nb, int Nf) {
+    BMLay L{};
     int o = 0;
     L.th0 = Ns + K - 1;
     L.tp0 = L.th0 | 1;
@@ -84,30 +85,54 @@ __host__ __device__ inline BMLay bm_layout(int K, int C, int Ns, int Npr, int Nb
     // Pitch 13 and window areas 5 words apart modulo 32 spread those
     // addresses over the LDS banks: in a model of typical window overlaps,
     // about 36 % fewer bank cycles per read than pitch th1 | 1 with
-    // back-to-back areas.  (The smallest such padding keeps four 4-wave
-    // workgroups of the 8x8 RGB form within a CU's LDS.)
+    // back-to-back areas.  Where that distance costs a workgroup of a CU's
+    // 160 KB (four wavefronts, allocated in pieces of 1280 bytes), 25 modulo
+    // 32 is next, then none: five workgroups instead of four for 7x7 RGB
+    // (30 frames 960x540: 12.7 -> 11.4 ms; 11.5 without padding).
     if (L.piped) L.tp1 = 13;
     L.ws = L.th1 * L.tp1 * C;
-    if (L.piped) L.ws += ((5 - L.ws) % 32 + 32) % 32;
+    if (L.piped) {
+        int best = 0, ws = L.ws;
+        for (int q = 0; q < 3; q++) {
+            const int pad = q == 2 ? 0 : (((q == 0 ? 5 : 25) - L.ws) % 32 + 32) % 32;
+            const int bytes = (2 * Nb * (L.ws + pad) + kBMLists) * 4 * 4;
+            const int n = 160 * 1024 / ((bytes + 1279) / 1280 * 1280);
+            if (n > best) {
+                best = n;
+                ws = L.ws + pad;
+            }
+        }
+        L.ws = ws;
+    }
     const int S = L.piped ? 128 : ((2 * Nb * P2p + 127) / 128) * 128;
     const int t0 = L.th0 * L.tp0 * C, t1 = 2 * Nb * L.ws;
     int t = t0 > t1 ? t0 : t1;
-    t = t > 128 ? t : 128;  // the slow-path scratch (64 entries) reuses the tile
+    // the selections' scratch (64 entries) reuses the tile, and so do the
+    // paired form's candidate and exact-selection lists (64 words each)
+    const int tmin = L.piped ? 320 : 128;
+    t = t > tmin ? t : tmin;
     const int nbest = (Nb * (2 * Nf + 1) + 3) & ~3;  // picks of all frames
     L.ref = o; o += L.piped ? 0 : K * K * C;
     L.tile = o; o += t;
     L.scr = L.tile;
-    L.sd = o; o += S;
-    L.si = o; o += S;
-    L.sv = o; o += L.piped ? 0 : S;
-    L.cd = o; o += 64;
-    L.ci = o; o += 64;  // directly after cd: the paired form's slot list spans both
+    L.sd = o; o += S;  // the paired form's slot list goes here first
+    if (L.piped) {
+        L.cd = L.tile + 128;
+        L.ci = L.tile + 192;
+        L.si = L.tile + 256;
+        L.sv = L.win = 0;
+    } else {
+        L.si = o; o += S;
+        L.sv = o; o += S;
+        L.cd = o; o += 64;
+        L.ci = o; o += 64;
+    }
     L.fd = o; o += L.piped ? 8 : 64;
     L.fi = o; o += L.piped ? 8 : 64;
     L.od = o; o += 16;
     L.oi = o; o += 16;
     L.pp = o; o += 16;
-    L.win = o; o += L.piped ? 20 : 80;
+    if (!L.piped) { L.win = o; o += 80; }
     L.bd = o; o += nbest;  // last: the only arrays whose place depends on Nf
     L.bi = o; o += nbest;
     L.total = o;

@@ -233,7 +233,7 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
     const bool piped = KT || L.piped;
     if (piped) {
         const int nfr[2] = {nfw, nbw};
-        uint32_t* lst = (uint32_t*)c_d;  // c_d and c_i, adjacent: 128 entries
+        uint32_t* lst = (uint32_t*)s_d;  // read by its lanes before they store their distances
         // windows of frame f of both chains: flow projection of the chain's
         // current matches (x first, then y at the updated x; without a flow
         // the matches' own positions), clamped Npr x Npr box in the next
@@ -355,6 +355,7 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
             // tile offset (bits 0..14; at most 4 windows of 12 x 13 x 3
             // words)
             unsigned long long bal[2];
+            unsigned qs[2];  // slot lane's position
 #pragma unroll
             for (int h = 0; h < 2; h++) {
                 // the chain's windows 0 and 1 (window 0 again when Nb = 1),
@@ -371,16 +372,19 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
                 const bool valid = act[h] & in & !seen;
                 const unsigned ent = (ent0 + ((unsigned)(h * 64) << 16) + (unsigned)(h * Nb * L.ws)) |
                                      (q == ref2 ? 0x8000u : 0u);
-                if (valid) s_i[h * 64 + lane] = q;
+                qs[h] = q;
                 bal[h] = __ballot(valid);
                 if (valid) lst[(h ? __popcll(bal[0]) : 0) + lanes_below(bal[h], lane)] = ent;
             }
             __builtin_amdgcn_s_waitcnt(0);  // the window copies
             wave_sync();
             const int nv = __popcll(bal[0]) + __popcll(bal[1]);
+            // at most 128 slots: the lane's entries, out before a distance
+            // goes into their place
+            const unsigned ea = lane < nv ? lst[lane] : 0u, eb = 64 + lane < nv ? lst[64 + lane] : 0u;
+            wave_sync();
             if constexpr (KT) {
-                // at most 128 slots: each lane's two sums run over the slices
-                const unsigned ea = lane < nv ? lst[lane] : 0u, eb = 64 + lane < nv ? lst[64 + lane] : 0u;
+                // each lane's two sums run over the slices
                 float sa = 0.f, sb = 0.f;
                 for (unsigned ht = 0; ht < (unsigned)a.kt; ht++) {
                     if (ht) {
@@ -397,7 +401,7 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
             } else {
                 for (int e0 = 0; e0 < nv; e0 += 64) {
                     if (e0 + lane < nv) {
-                        const unsigned e = lst[e0 + lane];
+                        const unsigned e = e0 == 0 ? ea : eb;
                         const float sv = ssd(tile + (e & 0x7FFFu), L.tp1, cs1);
                         s_d[e >> 16] = sv / norm - ((e & 0x8000u) ? a.d : 0.f);
                     }
@@ -432,7 +436,8 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
                         const int at = Nb * (1 + (ch == 0 ? f : nfw + f));
                         if (lane < Nb) {
                             const int sl = ch * 64 + (lane == 0 ? p1 : p2);
-                            const uint32_t iv = s_i[sl];
+                            const uint32_t i1 = __builtin_amdgcn_readlane(qs[ch], p1);
+                            const uint32_t iv = lane == 0 ? i1 : __builtin_amdgcn_readlane(qs[ch], p2);
                             pp[(ch == 0 ? 8 : 0) + lane] = iv;
                             b_d[at + lane] = s_d[sl];
                             b_i[at + lane] = iv;
@@ -443,6 +448,8 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
                 }
                 // top Nb of each window's list, appended in window order
                 int nfb = 0;
+                s_i[lane] = qs[ch];
+                wave_sync();
                 for (int m = 0; m < Nb; m++) {
                     const int sb = ch * 64 + m * P2p;
                     const unsigned long long wmask = P2p >= 64 ? ~0ull : ((1ull << P2p) - 1ull);
@@ -451,7 +458,7 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
                     const int mm = __popcll(bm);
                     n_eval += mm;
                     const int nb = min(Nb, mm);
-                    wave_select_sparse(s_d + sb, s_i + sb, v, bm, nb, o_d, o_i, c_d, c_i, scr, lane);
+                    wave_select_sparse(s_d + sb, s_i + m * P2p, v, bm, nb, o_d, o_i, c_d, c_i, scr, lane);
                     if (lane < nb) {
                         f_d[nfb + lane] = o_d[lane];
                         f_i[nfb + lane] = o_i[lane];
