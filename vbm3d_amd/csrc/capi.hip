@@ -732,8 +732,7 @@ int flow_absmax(vbm3d_ctx* ctx, const float* ff, const float* bf, unsigned W, un
     HIP_TRY(ensure(ctx->scal, 4));
     HIP_TRY(hipMemsetAsync(ctx->scal.p, 0, 4, s));
     const size_t n = (size_t)(F > 1 ? F - 1 : 0) * W * H * 2;
-    if (ff) HIP_TRY(launch_flow_absmax(ff, n, (unsigned*)ctx->scal.p, s));
-    if (bf) HIP_TRY(launch_flow_absmax(bf, n, (unsigned*)ctx->scal.p, s));
+    HIP_TRY(launch_flow_absmax(ff, bf, n, (unsigned*)ctx->scal.p, s));
     HIP_TRY(hipMemcpyAsync(out, ctx->scal.p, 4, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
     return VBM3D_OK;

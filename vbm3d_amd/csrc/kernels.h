@@ -368,7 +368,7 @@ int bm_lds_words(int K, int C, int Ns, int Npr, int Nb, int Nf);  // per wave, 4
 int filter_words(int K, int C, int N, int step);
 hipError_t launch_adjoint_fallback(float* gz, const float* gy, const float* den, size_t n, hipStream_t s);
 hipError_t launch_sum_counts(const uint32_t* counts, long n, unsigned long long* stats, hipStream_t s);
-hipError_t launch_flow_absmax(const float* fl, size_t n, unsigned* out, hipStream_t s);
+hipError_t launch_flow_absmax(const float* ff, const float* bf, size_t n, unsigned* out, hipStream_t s);
 hipError_t launch_bm_gen(const GenArgs& a, hipStream_t s);
 hipError_t launch_filter_gen(int step, const GenArgs& a, hipStream_t s);
 hipError_t launch_aggregate_gen(int C, const AArgs& a, const uint32_t* mpos, const TabsG* tabs, unsigned frames,

@@ -542,16 +542,35 @@ __global__ void k_sum_counts(const uint32_t* cnt, long n, unsigned long long* st
     }
 }
 
-__global__ void k_flow_absmax(const float* fl, size_t n, unsigned* out) {
+// Largest rounded magnitude of the flows given, in one launch with one
+// atomic per workgroup and eight loads in flight: a launch per flow with an
+// atomic per wavefront took 112 us for both flows of 12 frames 637x357, this
+// takes 30.
+__global__ __launch_bounds__(256) void k_flow_absmax(const float* __restrict__ ff, const float* __restrict__ bf, size_t n,
+                                                     unsigned* out) {
     unsigned m = 0;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * blockDim.x)
-        m = max(m, (unsigned)fminf(fabsf(roundf(fl[i])), 65535.f));  // NaN and huge values -> 65535
+    const float* fl[2] = {ff, bf};
+#pragma unroll
+    for (int d = 0; d < 2; d++) {
+        if (!fl[d]) continue;
+        for (size_t i0 = (size_t)blockIdx.x * 2048 + threadIdx.x; i0 < n; i0 += (size_t)gridDim.x * 2048) {
+            float v[8];  // in flight together
+#pragma unroll
+            for (int q = 0; q < 8; q++) v[q] = i0 + q * 256 < n ? fl[d][i0 + q * 256] : 0.f;
+#pragma unroll
+            for (int q = 0; q < 8; q++) m = max(m, (unsigned)fminf(fabsf(roundf(v[q])), 65535.f));  // NaN, huge: 65535
+        }
+    }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, o, 64));
-    if ((threadIdx.x & 63) == 0) atomicMax(out, m);
+    __shared__ unsigned s[4];
+    if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        m = max(max(s[0], s[1]), max(s[2], s[3]));
+        if (m) atomicMax(out, m);
+    }
 }
-
 
 }  // namespace
 
@@ -643,9 +662,10 @@ hipError_t launch_sum_counts(const uint32_t* counts, long n, unsigned long long*
     return hipGetLastError();
 }
 
-hipError_t launch_flow_absmax(const float* fl, size_t n, unsigned* out, hipStream_t s) {
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_flow_absmax, dim3(1024), dim3(256), 0, s, fl, n, out);
+hipError_t launch_flow_absmax(const float* ff, const float* bf, size_t n, unsigned* out, hipStream_t s) {
+    if (n == 0 || (!ff && !bf)) return hipSuccess;
+    const size_t blocks = (n + 2047) / 2048;
+    hipLaunchKernelGGL(k_flow_absmax, dim3((unsigned)(blocks < 1024 ? blocks : 1024)), dim3(256), 0, s, ff, bf, n, out);
     return hipGetLastError();
 }
 
