@@ -26,7 +26,16 @@ namespace {
 // frame, then every forward and backward frame) first copies the pixel
 // area its windows cover into a per-wave LDS tile; every lane then forms
 // one candidate's sum of squared differences from LDS against the
-// reference patch (also in LDS), in the reference's (c, y, x) order.
+// reference patch, whose rows arrive in scalar registers, in the reference's
+// (c, y, x) order.
+//
+// What bounds it: vector instruction issue, 84 % busy at 3,690 instructions
+// per 7x7 RGB patch of which 2,360 are the distances' separately rounded
+// subtractions, multiplications and additions; then the chain of dependent
+// steps per frame pair (copies, slot list, passes, two selections), which
+// the wavefronts of a SIMD hide from each other.  30 RGB frames 960x540,
+// step 2: 13.2 ms at 4,318 instructions and four wavefronts per SIMD, 12.6
+// at 3,690, 11.4 with a fifth wavefront.
 // ---------------------------------------------------------------------
 // KT: temporal patches (a.kt > 1 slices, at one position in consecutive
 // frames; the paired form only): each slice of the windows goes through the
@@ -632,13 +641,13 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
 
 // Occupancy floor per instantiation (waves per SIMD the register
 // allocator must leave room for), measured: with three channels the kernel
-// runs fastest held to 5 waves (96 registers, a few spills; 4 and 6 are
-// slower), with one channel unconstrained.
+// runs fastest held to 5 waves (4 and 6 are slower), with one channel
+// unconstrained.
 template <int K, int C>
 constexpr int bm_waves_floor() { return C == 3 ? 5 : 1; }
 
 template <int K, int C, int SH, bool KT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bm_waves_floor<K, C>()))) void k_bm(BMArgs a) {
+__device__ __forceinline__ void bm_block(const BMArgs& a) {
     extern __shared__ float smem[];
     const BMLay L = SH == 1 ? bm_layout(K, C, 7, 5, 2, a.Nf) : bm_layout(K, C, a.Ns, a.Npr, a.Nb, a.Nf);
     const int lane = threadIdx.x & 63;
@@ -649,6 +658,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bm_waves_fl
     const long r = a.r_begin + (long)lb * nw + w;
     if (r >= a.r_end) return;  // wave-uniform
     bm_one<K, C, SH, KT>(a, r, smem + (size_t)w * L.total, lane);
+}
+
+template <int K, int C, int SH>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bm_waves_floor<K, C>()))) void k_bm(BMArgs a) {
+    bm_block<K, C, SH, false>(a);
+}
+
+// Temporal patches.
+template <int K, int C, int SH>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bm_waves_floor<K, C>()))) void k_bm_kt(BMArgs a) {
+    bm_block<K, C, SH, true>(a);
 }
 
 template <int K, int C, int SH>
@@ -704,12 +724,12 @@ static hipError_t bm_k(const BMArgs& a, hipStream_t s) {
     const dim3 grid((unsigned)((n + waves - 1) / waves)), block(64 * waves);
     if (a.kt > 1) {
         if (!L.piped) return hipErrorInvalidValue;
-        if (bm_shape(a) == 1) hipLaunchKernelGGL((k_bm<K, C, 1, true>), grid, block, per_wave * waves, s, a);
-        else hipLaunchKernelGGL((k_bm<K, C, 0, true>), grid, block, per_wave * waves, s, a);
+        if (bm_shape(a) == 1) hipLaunchKernelGGL((k_bm_kt<K, C, 1>), grid, block, per_wave * waves, s, a);
+        else hipLaunchKernelGGL((k_bm_kt<K, C, 0>), grid, block, per_wave * waves, s, a);
     } else if (bm_shape(a) == 1) {
-        hipLaunchKernelGGL((k_bm<K, C, 1, false>), grid, block, per_wave * waves, s, a);
+        hipLaunchKernelGGL((k_bm<K, C, 1>), grid, block, per_wave * waves, s, a);
     } else {
-        hipLaunchKernelGGL((k_bm<K, C, 0, false>), grid, block, per_wave * waves, s, a);
+        hipLaunchKernelGGL((k_bm<K, C, 0>), grid, block, per_wave * waves, s, a);
     }
     return hipGetLastError();
 }
