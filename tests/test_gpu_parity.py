@@ -345,3 +345,22 @@ def test_step_error_against_fp64(cfg1, oracle, gpu_ctx):
     err2 = np.abs(final - np.where(e2 == 0, basic, m2 / np.where(e2 == 0, 1, e2))).max()
     print(f"max |GPU - FP64|: step 1 {err1:.3g}, step 2 {err2:.3g}")
     assert err1 < 1e-3 and err2 < 1e-3
+
+
+@pytest.mark.parametrize("W,H,F,C,skip2", [(700, 411, 15, 1, False), (512, 301, 10, 3, False), (512, 301, 10, 3, True)])
+def test_host_entry_in_pieces(gpu_ctx, W, H, F, C, skip2):
+    """Clips of 16 MB and more, whose result leaves the host-buffer entry in
+    pieces: all three videos equal the device-buffer entry's."""
+    import torch
+    import vbm3d_amd as V
+    _, noisy = synth.noisy_clip(W, H, F, C, 20.0, 71)
+    p1, p2 = V.initialize_parameters_1(20.0), V.initialize_parameters_2(20.0)
+    if skip2:
+        p2.k = 0
+    nz, basic, final = noisy.copy(), np.zeros_like(noisy), np.zeros_like(noisy)
+    V.run_vbm3d(20.0, nz, None, None, basic, final, p1, p2, True, 1, ctx=gpu_ctx)
+    z = torch.from_numpy(noisy).to("cuda:0")
+    b, f = torch.empty_like(z), torch.empty_like(z)
+    V.run_device(20.0, z, b, f, p1, p2, True, 1, ctx=gpu_ctx)
+    for host, dev in ((nz, z), (basic, b), (final, f)):
+        np.testing.assert_array_equal(host.view(np.uint32), dev.cpu().numpy().view(np.uint32))
