@@ -2,9 +2,9 @@
 // companion (tvl1flow/tvl1flow_lib.c; Zach, Pock and Bischof 2007 with
 // Chambolle's dual projection), and its C-ABI entry points.
 //
-// The pyramid, warps and the primal-dual iterations run as element-wise
-// and stencil kernels over [ny][nx] float planes in HBM, one thread per
-// pixel.  Every kernel evaluates the reference's expressions in its order
+// The pyramid runs as element-wise and stencil kernels over [ny][nx] float
+// planes in HBM, one thread per pixel; the primal-dual iterations run
+// several per launch on regions held in registers and LDS.  Every kernel evaluates the reference's expressions in its order
 // and precision -- float where it stores float, double where its
 // expressions promote (Gaussian taps and sums, bicubic cells, the
 // normalisation, 1.0 + taut * |grad|) -- with no FMA contraction and
