@@ -374,7 +374,7 @@ void member_reach_steps(const vbm3d_params& p, unsigned maxflow, unsigned W, uns
 // per crop, for each tile row and frame distance k the first grid row at
 // or below y0 - R_k - (K - 1) and the first beyond y0 + TY - 1 + R_k, then
 // the same for the tile columns with the division by their count;
-// R_k = min(R, R0 + k Rs).
+// R_k = min(R, R0 + k Rs).  Appended to `box`.
 void box_table(const GridDef& g, unsigned W, unsigned H, int K, unsigned Nf, int R, int R0, int Rs,
                std::vector<int4>& box) {
     const int nty = (int)((H + kAggTileY - 1) / kAggTileY), ntx = (int)((W + kAggTileX - 1) / kAggTileX);
@@ -387,8 +387,7 @@ void box_table(const GridDef& g, unsigned W, unsigned H, int K, unsigned Nf, int
         }
         return (int)lo;
     };
-    box.clear();
-    box.reserve(g.rows.size() * (size_t)(nty + ntx) * (Nf + 1));
+    box.reserve(box.size() + g.rows.size() * (size_t)(nty + ntx) * (Nf + 1));
     for (size_t c = 0; c < g.rows.size(); c++) {
         for (int ty = 0; ty < nty; ty++)
             for (unsigned k = 0; k <= Nf; k++) {
@@ -440,7 +439,7 @@ struct vbm3d_ctx {
     double pix_per_cand[3] = {0, 0, 0};   // k*k*C of each step's matching
     // batched form: rings shared by the clips of a batch, the plan (job
     // arrays and queue prefixes), queue counters, and the captured graph
-    DevBuf b_idx, b_nsx, b_est, b_wgt, b_refxy, b_meta, b_gpos, b_tabs, b_plan, b_cnt, b_save;
+    DevBuf b_idx, b_nsx, b_est, b_wgt, b_refxy, b_meta, b_gpos, b_tabs, b_box, b_plan, b_cnt, b_save;
     hipGraph_t b_graph = nullptr;
     hipGraphExec_t b_exec = nullptr;
     std::string b_key;
@@ -640,12 +639,13 @@ int run_step(vbm3d_ctx* ctx, StepIO& io, hipStream_t s) {
     ag.idx = bm.idx_out; ag.nsx = bm.nsx_out;
     ag.est = fa.est; ag.ms = (int)ms; ag.wgt = fa.wgt; ag.tabs = fa.tabs;
     ag.R = member_reach(p, io.maxflow, io.W, io.H);
-    member_reach_steps(p, io.maxflow, io.W, io.H, &ag.R0, &ag.Rs);
     if (!gen) {
         // each tile's grid box per frame distance, as the kernel would
         // search it (one load per bound instead of a chain of dependent ones)
         std::vector<int4> box;
-        box_table(g, io.W, io.H, (int)K, p.Nf, ag.R, ag.R0, ag.Rs, box);
+        int R0, Rs;
+        member_reach_steps(p, io.maxflow, io.W, io.H, &R0, &Rs);
+        box_table(g, io.W, io.H, (int)K, p.Nf, ag.R, R0, Rs, box);
         HIP_TRY(ensure(ctx->boxtab, box.size() * sizeof(int4)));
         HIP_TRY(hipMemcpyAsync(ctx->boxtab.p, box.data(), box.size() * sizeof(int4), hipMemcpyHostToDevice, s));
         ag.boxtab = (const int4*)ctx->boxtab.p;
@@ -921,7 +921,7 @@ struct Member {
     const vbm3d_params* p;
     unsigned K, C, N, nrf, Fr, ms = 0, ring = 0, maxflow = 0;
     size_t per_frame = 0;  // ring bytes per frame of reference patches
-    size_t refxy = 0, meta = 0, gpos = 0, tab = 0;
+    size_t refxy = 0, meta = 0, gpos = 0, tab = 0, box = 0;
     int ncrop = 0;
     size_t slot_base = 0, idx_base = 0, est_base = 0, wgt_base = 0;
     unsigned t_done = 0;
@@ -970,6 +970,7 @@ int plan_batch(vbm3d_ctx* ctx, const vbm3d_clip* clips, int n, int nb, const vbm
     std::vector<int> h_meta;
     std::vector<uint16_t> h_gpos;
     std::vector<Tabs> h_tabs;
+    std::vector<int4> h_box;
     std::vector<std::vector<Member>> steps(3);
     for (int st = 1; st <= 2; st++)
         for (int i = 0; i < n; i++) {
@@ -988,7 +989,11 @@ int plan_batch(vbm3d_ctx* ctx, const vbm3d_clip* clips, int n, int nb, const vbm
             m.refxy = h_refxy.size();
             m.meta = h_meta.size();
             m.gpos = h_gpos.size();
+            m.box = h_box.size();
             m.ncrop = (int)g.rows.size();
+            int R0, Rs;
+            member_reach_steps(p, m.maxflow, c.W, c.H, &R0, &Rs);
+            box_table(g, c.W, c.H, (int)m.K, p.Nf, member_reach(p, m.maxflow, c.W, c.H), R0, Rs, h_box);
             for (size_t q = 0; q < g.rows.size(); q++) {
                 h_meta.push_back((int)(h_refxy.size() - m.refxy));
                 h_meta.push_back((int)g.rows[q].size());
@@ -1075,10 +1080,12 @@ int plan_batch(vbm3d_ctx* ctx, const vbm3d_clip* clips, int n, int nb, const vbm
     HIP_TRY(ensure(ctx->b_meta, std::max<size_t>(h_meta.size(), 1) * 4));
     HIP_TRY(ensure(ctx->b_gpos, std::max<size_t>(h_gpos.size(), 1) * 2));
     HIP_TRY(ensure(ctx->b_tabs, std::max<size_t>(h_tabs.size(), 1) * sizeof(Tabs)));
+    HIP_TRY(ensure(ctx->b_box, std::max<size_t>(h_box.size(), 1) * sizeof(int4)));
     if (!h_refxy.empty()) HIP_TRY(hipMemcpyAsync(ctx->b_refxy.p, h_refxy.data(), h_refxy.size() * 4, hipMemcpyHostToDevice, s));
     if (!h_meta.empty()) HIP_TRY(hipMemcpyAsync(ctx->b_meta.p, h_meta.data(), h_meta.size() * 4, hipMemcpyHostToDevice, s));
     if (!h_gpos.empty()) HIP_TRY(hipMemcpyAsync(ctx->b_gpos.p, h_gpos.data(), h_gpos.size() * 2, hipMemcpyHostToDevice, s));
     if (!h_tabs.empty()) HIP_TRY(hipMemcpyAsync(ctx->b_tabs.p, h_tabs.data(), h_tabs.size() * sizeof(Tabs), hipMemcpyHostToDevice, s));
+    if (!h_box.empty()) HIP_TRY(hipMemcpyAsync(ctx->b_box.p, h_box.data(), h_box.size() * sizeof(int4), hipMemcpyHostToDevice, s));
     HIP_TRY(hipStreamSynchronize(s));  // the host vectors go out of scope
 
     uint32_t* d_idx = (uint32_t*)ctx->b_idx.p;
@@ -1089,6 +1096,7 @@ int plan_batch(vbm3d_ctx* ctx, const vbm3d_clip* clips, int n, int nb, const vbm
     const int* d_meta = (const int*)ctx->b_meta.p;
     const uint16_t* d_gpos = (const uint16_t*)ctx->b_gpos.p;
     const Tabs* d_tabs = (const Tabs*)ctx->b_tabs.p;
+    const int4* d_box = (const int4*)ctx->b_box.p;
 
     auto colour = [&](float* v, const vbm3d_clip& c, bool fwd) {
         BatchOp op;
@@ -1182,7 +1190,9 @@ int plan_batch(vbm3d_ctx* ctx, const vbm3d_clip* clips, int n, int nb, const vbm
                         ag.wgt = d_wgt + m.wgt_base;
                         ag.tabs = d_tabs + m.tab;
                         ag.R = member_reach(p, m.maxflow, c.W, c.H);
-                        member_reach_steps(p, m.maxflow, c.W, c.H, &ag.R0, &ag.Rs);
+                        ag.boxtab = d_box + m.box;
+                        ag.nty = (int)((c.H + kAggTileY - 1) / kAggTileY);
+                        ag.ntx = (int)((c.W + kAggTileX - 1) / kAggTileX);
                         ag.divW = make_div32(c.W);
                         ag.t_begin = m.t_done;
                         ag.fallback = st == 1 ? c.noisy : (nb == 1 ? c.basic : c.noisy);
@@ -1456,7 +1466,7 @@ void vbm3d_destroy(vbm3d_ctx* c) {
                       &c->idx, &c->nsx, &c->nsim, &c->dist, &c->est, &c->wgt, &c->tabs,
                       &c->refxy, &c->meta, &c->gpos, &c->rlist, &c->scal, &c->stats, &c->counts,
                       &c->b_idx, &c->b_nsx, &c->b_est, &c->b_wgt, &c->b_refxy, &c->b_meta, &c->b_gpos,
-                      &c->b_tabs, &c->b_plan, &c->b_cnt, &c->b_save, &c->tabsg, &c->mpos, &c->tv, &c->pyr, &c->msbuf,
+                      &c->b_tabs, &c->b_box, &c->b_plan, &c->b_cnt, &c->b_save, &c->tabsg, &c->mpos, &c->tv, &c->pyr, &c->msbuf,
                       &c->boxtab})
         if (b->p) (void)hipFree(b->p);
     if (c->b_exec) (void)hipGraphExecDestroy(c->b_exec);

@@ -23,16 +23,6 @@ namespace {
 // Aggregation (src/vbm3d.cpp:612-650, 860-924) with the division and the
 // den == 0 fallback (:168-170, :198-202, :267-280, :333-346).
 // ---------------------------------------------------------------------
-__device__ __forceinline__ int lower_bound_u16(const uint16_t* a, int n, int v) {
-    int lo = 0, hi = n;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if ((int)a[mid] < v) lo = mid + 1;
-        else hi = mid;
-    }
-    return lo;
-}
-
 // One 32x16 output tile of one frame per workgroup (eight wavefronts).
 // The reference patches whose groups can reach the tile are scanned in
 // processing order (crop, frame, row, column), one per thread at a time;
@@ -144,22 +134,10 @@ __device__ __forceinline__ void agg_tile(const A& a, const int bx, const int by,
     uint32_t crops = 1u;
     if (!ONE) {
         __shared__ int s_any[2 * kMaxCrops];
-        const int Rk = (int)min((long)a.R, (long)a.R0 + (long)a.Nf * a.Rs);
         for (int q = tid; q < 2 * a.ncrop; q += NT) {
             const int ci = q >> 1, col = q & 1;
-            int lo, hi;
-            if (a.boxtab) {
-                const int4 v = a.boxtab[((size_t)ci * (a.nty + a.ntx) + (col ? a.nty + bx : by)) * (a.Nf + 1) + a.Nf];
-                lo = v.x;
-                hi = v.y;
-            } else {
-                const int* meta = a.crop_meta + ci * 5;
-                const uint16_t* g = a.grid_pos + meta[3 + col];
-                const int b0 = (col ? x0 : y0) - Rk - (K - 1), b1 = (col ? x0 + TX : y0 + TY) + Rk;
-                lo = lower_bound_u16(g, meta[1 + col], b0);
-                hi = lower_bound_u16(g, meta[1 + col], b1);
-            }
-            s_any[q] = hi > lo;
+            const int4 v = a.boxtab[((size_t)ci * (a.nty + a.ntx) + (col ? a.nty + bx : by)) * (a.Nf + 1) + a.Nf];
+            s_any[q] = v.y > v.x;
         }
         __syncthreads();
         crops = (uint32_t)__ballot(lane < a.ncrop && s_any[2 * (lane & (kMaxCrops - 1))] && s_any[2 * (lane & (kMaxCrops - 1)) + 1]);
@@ -168,40 +146,28 @@ __device__ __forceinline__ void agg_tile(const A& a, const int bx, const int by,
     for (; crops; crops &= crops - 1) {
         const int ci = ONE ? 0 : __builtin_ctz(crops);
         const int* meta = a.crop_meta + ci * 5;
-        const int off = meta[0], nrows = meta[1], ncols = meta[2];
-        const uint16_t* rows = a.grid_pos + meta[3];
-        const uint16_t* cols = a.grid_pos + meta[4];
+        const int off = meta[0], ncols = meta[2];
         // A member k frames away from its reference patch lies within
         // min(R, R0 + k Rs) of it, so the box narrows towards the output
         // frame.  The frames' boxes are concatenated in frame order: the
         // scan below still visits the patches in processing order (crop,
         // frame, row, column).
         __syncthreads();  // the previous crop's table is no longer read
-        if (a.boxtab) {
-            // the host's table of the same bounds: one load per bound, the
-            // columns' division with them
-            if (tid < 2 * nfr) {
-                const int q = tid >> 1, col = tid & 1;
-                const int k = far(trlo + q);
-                const size_t tl = (size_t)ci * (a.nty + a.ntx) + (col ? a.nty + bx : by);
-                const int4 v = a.boxtab[tl * (a.Nf + 1) + k];
-                s_bnd[6 * q + 2 * col] = v.x;
-                s_bnd[6 * q + 2 * col + 1] = v.y;
-                if (col) {
-                    s_bnd[6 * q + 4] = v.z;
-                    s_bnd[6 * q + 5] = v.w;
-                }
-            }
-        } else if (tid < 4 * nfr) {
-            // the four searches of a frame run in four threads (each is a
-            // chain of dependent loads)
-            const int q = tid >> 2, which = tid & 3;
+        // the host's table of the bounds: one load per bound, the columns'
+        // division with them.  (Searched here, they are a chain of dependent
+        // loads ahead of everything else a tile does: a batch of 64 mixed
+        // clips 576 -> 567 ms without it.)
+        if (tid < 2 * nfr) {
+            const int q = tid >> 1, col = tid & 1;
             const int k = far(trlo + q);
-            const int Rk = (int)min((long)a.R, (long)a.R0 + (long)k * a.Rs);
-            const bool row = which < 2;
-            const int lo = row ? y0 - Rk - (K - 1) : x0 - Rk - (K - 1);
-            const int hi = row ? y0 + TY + Rk : x0 + TX + Rk;
-            s_bnd[6 * q + which] = lower_bound_u16(row ? rows : cols, row ? nrows : ncols, (which & 1) ? hi : lo);
+            const size_t tl = (size_t)ci * (a.nty + a.ntx) + (col ? a.nty + bx : by);
+            const int4 v = a.boxtab[tl * (a.Nf + 1) + k];
+            s_bnd[6 * q + 2 * col] = v.x;
+            s_bnd[6 * q + 2 * col + 1] = v.y;
+            if (col) {
+                s_bnd[6 * q + 4] = v.z;
+                s_bnd[6 * q + 5] = v.w;
+            }
         }
         __syncthreads();
         // wavefront 0: lane q < nfr assembles frame q's box; the boxes'
@@ -214,12 +180,8 @@ __device__ __forceinline__ void agg_tile(const A& a, const int bx, const int by,
                 const int nr = max(s_bnd[6 * lane + 1] - ia, 0);
                 nc = max(s_bnd[6 * lane + 3] - ja, 0);
                 cnt = nr * nc;
-                if (a.boxtab) {
-                    const unsigned sh = (unsigned)s_bnd[6 * lane + 5];
-                    s_div[lane] = Div32{(uint32_t)s_bnd[6 * lane + 4], sh & 0xFFu, sh >> 8};
-                } else {
-                    s_div[lane] = make_div32(nc > 0 ? nc : 1);
-                }
+                const unsigned sh = (unsigned)s_bnd[6 * lane + 5];
+                s_div[lane] = Div32{(uint32_t)s_bnd[6 * lane + 4], sh & 0xFFu, sh >> 8};
             }
             int incl = cnt;
 #pragma unroll
