@@ -202,6 +202,9 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
             wave_sync();
             if (lane < m) ss = ssd(tile + ly * L.tp0 + lx, L.tp0, cs, ss, ht * whc);
         }
+        // the paired form's candidate list lies over the tile: no entry (the
+        // positions depend on no distance) before every read of the tile
+        wave_sync();
         if (lane < m) {
             const float s = ss / norm;
             const unsigned qx = x0 + lx, qy = y0 + ly;
