@@ -1,0 +1,40 @@
+"""Search shapes known at run time, bit for bit against the oracle where
+their kernels differ: grey and RGB, paired and unpaired, clips of tied
+distances (the exact selection)."""
+import numpy as np
+import pytest
+
+from vbm3d_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def _bits(a):
+    return np.ascontiguousarray(a, np.float32).view(np.uint32)
+
+
+def _run(V, noisy, sigma, p1, p2, ctx):
+    nz, b, f = noisy.copy(), np.zeros_like(noisy), np.zeros_like(noisy)
+    V.run_vbm3d(sigma, nz, None, None, b, f, p1, p2, True, 1, ctx=ctx)
+    return b, f
+
+
+# (channels, shape); the last two are the paired form at every k
+CASES = [(3, dict(Npr=7)), (1, dict(Npr=7)), (3, dict(Ns=8, Npr=8, Nb=4, Nf=2)), (1, dict(Ns=8, Npr=8, Nb=4, Nf=2)),
+         (1, dict(Npr=3)), (1, dict(Npr=7, Nb=1, k=5))]
+
+
+@pytest.mark.parametrize("ties", [False, True], ids=["noise", "ties"])
+@pytest.mark.parametrize("C,shape", CASES, ids=lambda v: str(v) if isinstance(v, int) else "-".join(f"{k}{x}" for k, x in v.items()))
+def test_shapes(oracle, gpu_ctx, C, shape, ties):
+    import vbm3d_amd as V
+    W, H, F = 41, 35, 4
+    if ties:
+        noisy = np.random.default_rng(6).integers(0, 3, (F, C, H, W)).astype(np.float32)
+    else:
+        _, noisy = synth.noisy_clip(W, H, F, C, 20.0, 71)
+    p1, p2 = V.initialize_parameters_1(20.0, **shape), V.initialize_parameters_2(20.0, **shape)
+    b, f = _run(V, noisy, 20.0, p1, p2, gpu_ctx)
+    ob, of, _ = oracle.run_vbm3d(20.0, noisy, p1, p2, True, 1)
+    np.testing.assert_array_equal(_bits(b), _bits(ob))
+    np.testing.assert_array_equal(_bits(f), _bits(of))

@@ -300,7 +300,7 @@ bool fast_kt_ok(const vbm3d_params& p, unsigned W, unsigned H, unsigned C) {
     vbm3d_params q = p;
     q.kt = 1;
     q.N = (unsigned)pow2ceil((int)p.N);  // any group size up to 16
-    if (!fast_ok(q, W, H) || !bm_layout((int)p.k, (int)C, p.Ns, p.Npr, p.Nb, p.Nf).piped) return false;
+    if (!fast_ok(q, W, H) || !bm_paired((int)p.k, (int)p.Npr, (int)p.Nb)) return false;
     return (size_t)filter_kt_lds_words((int)p.k, (int)C, (int)p.kt, (int)p.N, 2) * 4 <= 64 * 1024;
 }
 
@@ -595,6 +595,7 @@ int run_step(vbm3d_ctx* ctx, StepIO& io, hipStream_t s) {
     bm.ref_list = nullptr;
     bm.ring = ring;
     bm.Ns = p.Ns; bm.Npr = p.Npr; bm.Nb = p.Nb; bm.Nf = p.Nf; bm.N = p.N; bm.kt = p.kt;
+    bm.ws = bm_window_words((int)K, (int)C, p.Npr, p.Nb);
     bm.d = p.d; bm.tau = p.tau;
     bm.dW = make_div32(io.W);
     bm.dWHC = make_div32(bm.whc);
@@ -1137,6 +1138,7 @@ int plan_batch(vbm3d_ctx* ctx, const vbm3d_clip* clips, int n, int nb, const vbm
                         bm.r_end = (long)e * m.nrf;
                         bm.ring = m.ring;
                         bm.Ns = p.Ns; bm.Npr = p.Npr; bm.Nb = p.Nb; bm.Nf = p.Nf; bm.N = p.N; bm.kt = p.kt;
+                        bm.ws = bm_window_words((int)m.K, (int)m.C, p.Npr, p.Nb);
                         bm.d = p.d; bm.tau = p.tau;
                         bm.dW = make_div32(c.W);
                         bm.dWHC = make_div32(whc);
@@ -1785,6 +1787,7 @@ int vbm3d_block_match(vbm3d_ctx* ctx, const float* vid, unsigned W, unsigned H, 
     bm.r_begin = 0; bm.r_end = nrefs;
     bm.nrf = 1; bm.ring = 1;
     bm.Ns = prm->Ns; bm.Npr = prm->Npr; bm.Nb = prm->Nb; bm.Nf = prm->Nf; bm.N = prm->N; bm.kt = prm->kt;
+    bm.ws = bm_window_words((int)prm->k, (int)C, prm->Npr, prm->Nb);
     bm.d = prm->d; bm.tau = prm->tau;
     bm.dW = make_div32(W);
     bm.dWHC = make_div32(W * H * C);

@@ -66,44 +66,58 @@ struct BMLay {
 };
 
 constexpr int kBMLists = 232;  // words of the paired form beside its tile, at Nf 4 and Nb 2
-__host__ __device__ constexpr BMLay bm_layout(int K, int C, int Ns, int Npr, int Nb, int Nf) {
+
+// The paired form of k_bm: at most 2 matches per frame, one chain's slots
+// within 64 (P2p = Npr^2 rounded up to a power of two each), at most 12 tile
+// rows.
+__host__ __device__ constexpr bool bm_paired(int K, int Npr, int Nb) {
+    return Nb <= 2 && Nb * pow2ceil(Npr * Npr) <= 64 && Npr + K - 1 <= 12;
+}
+
+// Words from one predictive window's area to the next.
+// The paired form's lanes hold the valid slots of up to four windows in
+// list order, each reading its window's area at (row * tp1 + column).
+// Pitch 13 and window areas 5 words apart modulo 32 spread those
+// addresses over the LDS banks: in a model of typical window overlaps,
+// about 36 % fewer bank cycles per read than pitch th1 | 1 with
+// back-to-back areas.  Where that distance costs a workgroup of a CU's
+// 160 KB (four wavefronts, allocated in pieces of 1280 bytes), 25 modulo
+// 32 is next, then none: five workgroups instead of four for 7x7 RGB
+// (30 frames 960x540: 12.7 -> 11.4 ms; 11.5 without padding).
+// The kernels take it from the host for shapes known at run time
+// (BMArgs::ws): with these divisions in every wavefront step 2 of 8 grey
+// frames 640x360 at Npr 3 matched in 0.774 ms instead of 0.756.
+__host__ __device__ constexpr int bm_window_words(int K, int C, int Npr, int Nb) {
+    const int th1 = Npr + K - 1;
+    if (!bm_paired(K, Npr, Nb)) return th1 * (th1 | 1) * C;
+    const int w = th1 * 13 * C;
+    int best = 0, ws = w;
+    for (int q = 0; q < 3; q++) {
+        const int pad = q == 2 ? 0 : (((q == 0 ? 5 : 25) - w) % 32 + 32) % 32;
+        const int bytes = (2 * Nb * (w + pad) + kBMLists) * 4 * 4;
+        const int n = 160 * 1024 / ((bytes + 1279) / 1280 * 1280);
+        if (n > best) {
+            best = n;
+            ws = w + pad;
+        }
+    }
+    return ws;
+}
+
+// ws: bm_window_words.
+__host__ __device__ constexpr BMLay bm_layout(int K, int C, int Ns, int Npr, int Nb, int Nf, int ws) {
     BMLay L{};
     int o = 0;
     L.th0 = Ns + K - 1;
     L.tp0 = L.th0 | 1;
     L.th1 = Npr + K - 1;
-    L.tp1 = L.th1 | 1;
-    // predictive-stage slots: window w owns [w * P2p, (w + 1) * P2p),
-    // P2p = Npr^2 rounded up to a power of two.  The paired form (at most
-    // 2 matches per frame, one chain's slots within 64, at most 12 tile
-    // rows) gives chain h the slots [64 h, 64 h + 64), reads the reference
-    // patch through scalar loads and needs no validity array.
+    // predictive-stage slots: window w owns [w * P2p, (w + 1) * P2p); the
+    // paired form gives chain h the slots [64 h, 64 h + 64), reads the
+    // reference patch through scalar loads and needs no validity array
     const int P2p = pow2ceil(Npr * Npr);
-    L.piped = Nb <= 2 && Nb * P2p <= 64 && L.th1 <= 12;
-    // The paired form's lanes hold the valid slots of up to four windows in
-    // list order, each reading its window's area at (row * tp1 + column).
-    // Pitch 13 and window areas 5 words apart modulo 32 spread those
-    // addresses over the LDS banks: in a model of typical window overlaps,
-    // about 36 % fewer bank cycles per read than pitch th1 | 1 with
-    // back-to-back areas.  Where that distance costs a workgroup of a CU's
-    // 160 KB (four wavefronts, allocated in pieces of 1280 bytes), 25 modulo
-    // 32 is next, then none: five workgroups instead of four for 7x7 RGB
-    // (30 frames 960x540: 12.7 -> 11.4 ms; 11.5 without padding).
-    if (L.piped) L.tp1 = 13;
-    L.ws = L.th1 * L.tp1 * C;
-    if (L.piped) {
-        int best = 0, ws = L.ws;
-        for (int q = 0; q < 3; q++) {
-            const int pad = q == 2 ? 0 : (((q == 0 ? 5 : 25) - L.ws) % 32 + 32) % 32;
-            const int bytes = (2 * Nb * (L.ws + pad) + kBMLists) * 4 * 4;
-            const int n = 160 * 1024 / ((bytes + 1279) / 1280 * 1280);
-            if (n > best) {
-                best = n;
-                ws = L.ws + pad;
-            }
-        }
-        L.ws = ws;
-    }
+    L.piped = bm_paired(K, Npr, Nb);
+    L.tp1 = L.piped ? 13 : L.th1 | 1;
+    L.ws = ws;
     const int S = L.piped ? 128 : ((2 * Nb * P2p + 127) / 128) * 128;
     const int t0 = L.th0 * L.tp0 * C, t1 = 2 * Nb * L.ws;
     int t = t0 > t1 ? t0 : t1;
@@ -150,6 +164,7 @@ struct BMArgs {
     long r_begin, r_end;      // global ref ids t*nrf + i (or list positions)
     unsigned ring;            // slot = (t % ring) * nrf + i (grid mode)
     int Ns, Npr, Nb, Nf, N, kt;
+    int ws;                   // bm_window_words
     float d, tau;
     uint32_t* idx_out;   // [slot][N]
     float* dist_out;     // [slot][N] or null

@@ -48,7 +48,7 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
     // time, so that tile and window offsets become instruction immediates
     constexpr bool FIX = SH == 1;
     const int Ns = FIX ? 7 : a.Ns, Npr = FIX ? 5 : a.Npr, Nb = FIX ? 2 : a.Nb;
-    const BMLay L = bm_layout(K, C, Ns, Npr, Nb, a.Nf);
+    const BMLay L = bm_layout(K, C, Ns, Npr, Nb, a.Nf, FIX ? bm_window_words(K, C, 5, 2) : a.ws);
     float* tile = base + L.tile;
     float* s_d = base + L.sd;
     uint32_t* s_i = (uint32_t*)(base + L.si);
@@ -644,15 +644,19 @@ __device__ __forceinline__ void bm_one(const A& a, const long r, float* base, co
 
 // Occupancy floor per instantiation (waves per SIMD the register
 // allocator must leave room for), measured: with three channels the kernel
-// runs fastest held to 5 waves (4 and 6 are slower), with one channel
-// unconstrained.
+// runs fastest held to 5 waves (4 and 6 are slower).  With one channel the
+// default shape needs 58 to 64 registers by itself; shapes known at run time
+// take up to 81, one more than six waves have, and up to 98 for temporal
+// patches (8 grey frames 640x360, Npr 3, step 2: 0.756 -> 0.707 ms held to
+// six; 320x240 at kt 2, Npr 3: 0.395 -> 0.333, though 44 bytes spill).
 template <int K, int C>
-constexpr int bm_waves_floor() { return C == 3 ? 5 : 1; }
+constexpr int bm_waves_floor() { return C == 3 ? 5 : 6; }
 
 template <int K, int C, int SH, bool KT>
 __device__ __forceinline__ void bm_block(const BMArgs& a) {
     extern __shared__ float smem[];
-    const BMLay L = SH == 1 ? bm_layout(K, C, 7, 5, 2, a.Nf) : bm_layout(K, C, a.Ns, a.Npr, a.Nb, a.Nf);
+    const BMLay L = SH == 1 ? bm_layout(K, C, 7, 5, 2, a.Nf, bm_window_words(K, C, 5, 2))
+                            : bm_layout(K, C, a.Ns, a.Npr, a.Nb, a.Nf, a.ws);
     const int lane = threadIdx.x & 63;
     const int w = threadIdx.x >> 6;
     const int nw = blockDim.x >> 6;
@@ -719,7 +723,7 @@ template <int K, int C>
 static hipError_t bm_k(const BMArgs& a, hipStream_t s) {
     const long n = a.r_end - a.r_begin;
     if (n <= 0) return hipSuccess;
-    const BMLay L = bm_layout(K, C, a.Ns, a.Npr, a.Nb, a.Nf);
+    const BMLay L = bm_layout(K, C, a.Ns, a.Npr, a.Nb, a.Nf, a.ws);
     const size_t per_wave = (size_t)L.total * 4;
     int waves = 4;
     while (waves > 1 && per_wave * waves > 64 * 1024) waves--;
@@ -798,6 +802,8 @@ hipError_t launch_bm_queue(int K, int C, const BMArgs* jobs, const WorkQueue& q,
 #undef VB_BMQ
 }
 
-int bm_lds_words(int K, int C, int Ns, int Npr, int Nb, int Nf) { return bm_layout(K, C, Ns, Npr, Nb, Nf).total; }
+int bm_lds_words(int K, int C, int Ns, int Npr, int Nb, int Nf) {
+    return bm_layout(K, C, Ns, Npr, Nb, Nf, bm_window_words(K, C, Npr, Nb)).total;
+}
 
 }  // namespace vb
