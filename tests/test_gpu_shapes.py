@@ -1,6 +1,7 @@
 """Search shapes known at run time, bit for bit against the oracle where
-their kernels differ: grey and RGB, paired and unpaired, clips of tied
-distances (the exact selection)."""
+their launches differ: grey clips, one to four wavefronts per workgroup in
+the unpaired form, clips of tied distances (the exact selection), and a
+batch whose clips need the paired and the unpaired form in one launch."""
 import numpy as np
 import pytest
 
@@ -19,7 +20,8 @@ def _run(V, noisy, sigma, p1, p2, ctx):
     return b, f
 
 
-# (channels, shape); the last two are the paired form at every k
+# (channels, shape): unpaired RGB at k 7 takes one wavefront per workgroup,
+# unpaired grey one to four; the last two are the paired form
 CASES = [(3, dict(Npr=7)), (1, dict(Npr=7)), (3, dict(Ns=8, Npr=8, Nb=4, Nf=2)), (1, dict(Ns=8, Npr=8, Nb=4, Nf=2)),
          (1, dict(Npr=3)), (1, dict(Npr=7, Nb=1, k=5))]
 
@@ -38,3 +40,21 @@ def test_shapes(oracle, gpu_ctx, C, shape, ties):
     ob, of, _ = oracle.run_vbm3d(20.0, noisy, p1, p2, True, 1)
     np.testing.assert_array_equal(_bits(b), _bits(ob))
     np.testing.assert_array_equal(_bits(f), _bits(of))
+
+
+@pytest.mark.parametrize("persistent", [0, 1])
+def test_batch_of_paired_and_unpaired(oracle, persistent):
+    import torch
+    import vbm3d_amd as V
+    items, ref = [], []
+    for i, shape in enumerate((dict(), dict(Npr=7), dict(Nb=3))):
+        _, noisy = synth.noisy_clip(43 + i, 37, 4, 3, 20.0, 72 + i)
+        p1, p2 = V.initialize_parameters_1(20.0, **shape), V.initialize_parameters_2(20.0, **shape)
+        items.append(V.BatchItem(20.0, torch.from_numpy(noisy).to("cuda:0"), p1, p2))
+        ref.append(oracle.run_vbm3d(20.0, noisy, p1, p2, True, 1))
+    V.run_batch(items, 1, dict(chunk_frames=0, waves_per_group=0, grab=1, groups_per_cu=8, use_graph=0,
+                               persistent=persistent))
+    for it, (ob, of, _) in zip(items, ref):
+        # run_vbm3d's outputs after the colour round trip, as the batch's
+        np.testing.assert_array_equal(_bits(it.basic.cpu().numpy()), _bits(ob))
+        np.testing.assert_array_equal(_bits(it.denoised.cpu().numpy()), _bits(of))

@@ -900,6 +900,7 @@ struct BatchOp {
     int fwd = 0;
     size_t bytes = 0;
     int shape = 0;  // match: bm_shape shared by every job, else 0; aggregate: largest N
+    bool paired = true;  // match: every job in k_bm's paired form
 };
 
 struct BatchPlan {
@@ -1216,8 +1217,10 @@ int plan_batch(vbm3d_ctx* ctx, const vbm3d_clip* clips, int n, int nb, const vbm
                     op.prefix = blob_put(plan.blob, cl.pre.data(), cl.pre.size() * sizeof(long));
                     op.njobs = (int)cl.bm.size(); op.total = cl.pre.back(); op.words = cl.wb;
                     op.shape = 1;
-                    for (const BMArgs& b : cl.bm)
+                    for (const BMArgs& b : cl.bm) {
                         if (bm_shape(b) != 1) op.shape = 0;
+                        op.paired = op.paired && bm_paired(cl.K, b.Npr, b.Nb);
+                    }
                     op.counter = plan.counters++;
                     plan.ops.push_back(op);
                 }
@@ -1290,7 +1293,9 @@ int exec_batch(vbm3d_ctx* ctx, const BatchPlan& plan, const vbm3d_batch_config& 
                 }
                 continue;
             }
-            int waves = cfg.waves_per_group > 0 ? std::min(cfg.waves_per_group, 4) : 4;
+            int waves = cfg.waves_per_group > 0 ? std::min(cfg.waves_per_group, 4)
+                        : op.kind == 0          ? bm_group_waves((size_t)op.words * 4, op.paired)
+                                                : 4;
             while (waves > 1 && (size_t)op.words * 4 * waves > 64 * 1024) waves--;
             if ((size_t)op.words * 4 > 64 * 1024) return fail(VBM3D_ERR_UNSUPPORTED, "patch working set above 64 KB of LDS");
             const long need = (op.total + (long)q.grab * waves - 1) / ((long)q.grab * waves);

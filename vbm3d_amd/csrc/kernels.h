@@ -104,6 +104,22 @@ __host__ __device__ constexpr int bm_window_words(int K, int C, int Npr, int Nb)
     return ws;
 }
 
+// Wavefronts per workgroup of k_bm at `bytes` of LDS each: four; in the
+// unpaired form, which takes up to 22 KB, as many as leave most wavefronts on
+// a CU's 160 KB (8 RGB frames 320x240 at Npr 7, four leaving 8 and one 11:
+// step 2 2.10 -> 1.50 ms; grey, 20 and 23: 1.67 -> 1.57).
+inline int bm_group_waves(size_t bytes, bool paired) {
+    int waves = 4;
+    while (waves > 1 && bytes * waves > 64 * 1024) waves--;
+    if (paired) return waves;
+    int best = 0;
+    for (int v = 1, top = waves; v <= top; v++) {
+        const int on = (int)(160 * 1024 / ((bytes * v + 1279) / 1280 * 1280)) * v;
+        if (on >= best) best = on, waves = v;
+    }
+    return waves;
+}
+
 // ws: bm_window_words.
 __host__ __device__ constexpr BMLay bm_layout(int K, int C, int Ns, int Npr, int Nb, int Nf, int ws) {
     BMLay L{};

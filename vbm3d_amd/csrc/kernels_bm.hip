@@ -725,9 +725,8 @@ static hipError_t bm_k(const BMArgs& a, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     const BMLay L = bm_layout(K, C, a.Ns, a.Npr, a.Nb, a.Nf, a.ws);
     const size_t per_wave = (size_t)L.total * 4;
-    int waves = 4;
-    while (waves > 1 && per_wave * waves > 64 * 1024) waves--;
     if (per_wave > 64 * 1024) return hipErrorInvalidValue;
+    const int waves = bm_group_waves(per_wave, L.piped);
     const dim3 grid((unsigned)((n + waves - 1) / waves)), block(64 * waves);
     if (a.kt > 1) {
         if (!L.piped) return hipErrorInvalidValue;
