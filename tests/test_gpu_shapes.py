@@ -1,7 +1,7 @@
 """Search shapes known at run time, bit for bit against the oracle where
 their launches differ: grey clips, one to four wavefronts per workgroup in
-the unpaired form, clips of tied distances (the exact selection), and a
-batch whose clips need the paired and the unpaired form in one launch."""
+the unpaired form, clips of tied distances (the exact selection), and
+batches whose clips differ in form or group size in one launch."""
 import numpy as np
 import pytest
 
@@ -56,5 +56,22 @@ def test_batch_of_paired_and_unpaired(oracle, persistent):
                                persistent=persistent))
     for it, (ob, of, _) in zip(items, ref):
         # run_vbm3d's outputs after the colour round trip, as the batch's
+        np.testing.assert_array_equal(_bits(it.basic.cpu().numpy()), _bits(ob))
+        np.testing.assert_array_equal(_bits(it.denoised.cpu().numpy()), _bits(of))
+
+
+@pytest.mark.parametrize("nb", [1, 4])
+def test_batch_groups_of_16(oracle, nb):
+    """A batch whose largest group is 16, beside clips of groups of 4 and 8."""
+    import torch
+    import vbm3d_amd as V
+    items, ref = [], []
+    for i, (C, N) in enumerate(((3, 16), (3, 4), (1, 16), (1, 8))):
+        _, noisy = synth.noisy_clip(90 + i, 70, 3, C, 20.0, 75 + i)
+        p1, p2 = V.initialize_parameters_1(20.0, N=N), V.initialize_parameters_2(20.0, N=N)
+        items.append(V.BatchItem(20.0, torch.from_numpy(noisy).to("cuda:0"), p1, p2))
+        ref.append(oracle.run_vbm3d(20.0, noisy, p1, p2, True, nb))
+    V.run_batch(items, nb)
+    for it, (ob, of, _) in zip(items, ref):
         np.testing.assert_array_equal(_bits(it.basic.cpu().numpy()), _bits(ob))
         np.testing.assert_array_equal(_bits(it.denoised.cpu().numpy()), _bits(of))

@@ -400,11 +400,20 @@ __device__ __forceinline__ void agg_tile(const A& a, const int bx, const int by,
     }
 }
 
-// Occupancy floor of 8 waves per SIMD (64 registers): the kernel waits on
-// memory more than it computes (6 waves with twice the entries in flight:
-// 3.04 against 2.94 ms).
+// Occupancy floor by the members the scan holds.  Up to 8: 8 waves per SIMD
+// (64 registers), the kernel waits on memory more than it computes (6 waves
+// with twice the entries in flight: 3.04 against 2.94 ms).  Above 8 the list
+// takes up to 64 KB, which leaves two workgroups to a CU (4 waves per SIMD),
+// and 64 registers spilled up to 280 bytes a lane for waves that could not
+// run: 5.  (N 16, step 2 at floor 8 / 6 / 5 / 4: 8 grey frames 640x360 0.564 /
+// 0.476 / 0.500 / 0.501 ms, on 16 crops 0.999 / 0.908 / 0.874 / 0.895, 8 RGB
+// frames 320x240 0.287 / 0.246 / 0.244 / 0.255; a batch of 12 RGB clips
+// 200x150x6, whole call, 5.54 / 5.04 / 4.81 / 4.80.)
+constexpr int agg_waves_floor(int NM) { return NM > 8 ? 5 : 8; }
+
 template <int C, bool RAW, int NM, bool ONE, bool KT>
-__global__ __launch_bounds__(kAggThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_aggregate(AArgs a) {
+__global__ __launch_bounds__(kAggThreads) __attribute__((amdgpu_waves_per_eu(agg_waves_floor(NM)))) void k_aggregate(
+    AArgs a) {
     agg_tile<C, RAW, NM, ONE, KT>(a, blockIdx.x, blockIdx.y, blockIdx.z, a.N);
 }
 
@@ -412,7 +421,7 @@ __global__ __launch_bounds__(kAggThreads) __attribute__((amdgpu_waves_per_eu(8))
 // the hardware's dispatch order is the queue; item -> (job, frame, tile
 // row, tile column).  The same occupancy floor as k_aggregate.
 template <int C, int NM>
-__global__ __launch_bounds__(kAggThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_aggregate_multi(
+__global__ __launch_bounds__(kAggThreads) __attribute__((amdgpu_waves_per_eu(agg_waves_floor(NM)))) void k_aggregate_multi(
     const AArgs* __restrict__ jobs, WorkQueue q, int nl) {
     const long it = (long)blockIdx.x;
     if (it >= q.total) return;  // workgroup-uniform
