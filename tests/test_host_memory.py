@@ -1,0 +1,63 @@
+"""Host logic of libvbm3d_hip.so where device memory is short or a launch
+fails, on a stand-in for the HIP runtime (fake_hip.cpp): what a context keeps
+after a call, what fits, and that no copy on the caller's buffers is left in
+flight.  Each case runs in a process of its own, which binds the stand-in."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+from conftest import ROOT
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+PRELUDE = """
+import ctypes as C, sys
+fake = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+sys.modules["torch"] = None  # one runtime only: the stand-in
+sys.path.insert(0, sys.argv[2])
+import numpy as np
+import vbm3d_amd as V
+for f in ("used", "peak"):
+    getattr(fake, "fake_" + f).restype = C.c_size_t
+for f in ("launches", "in_flight", "h2d"):
+    getattr(fake, "fake_" + f).restype = C.c_long
+fake.fake_reset.argtypes = [C.c_size_t, C.c_long]
+MB = 1 << 20
+"""
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-o", so, os.path.join(HERE, "fake_hip.cpp")])
+
+    def run(body, **env):
+        r = subprocess.run([sys.executable, "-c", PRELUDE + body, so, ROOT], capture_output=True, text=True, timeout=120,
+                           env={**os.environ, **env})
+        assert r.returncode == 0, r.stdout + r.stderr
+        return r.stdout
+    return run
+
+
+def test_multiscale_gives_its_memory_back(fake):
+    """200 grey frames 512x384: the video, its levels twice and a basic
+    estimate are 4.6 clips; the pyramid's workspace is many frames'.  Of them
+    only a bounded part may outlive the call."""
+    fake("""
+v = np.zeros((200, 1, 384, 512), np.float32)
+ctx = V.Context(0)
+V.multiscale_denoise(v[:2], 20.0, 2, ctx=ctx)
+V.denoise(v, 20.0, ctx=ctx)  # the denoiser's own rings, which a context keeps
+for _ in range(2):
+    before = fake.fake_used()
+    V.multiscale_denoise(v, 20.0, 2, ctx=ctx)
+    kept = fake.fake_used() - before
+    assert kept <= 1024 * MB, kept
+small = V.Context(0)
+V.multiscale_denoise(v[:2, :, :96, :128], 20.0, 2, ctx=small)
+n = fake.fake_used()
+V.multiscale_denoise(v[:2, :, :96, :128], 20.0, 2, ctx=small)
+assert fake.fake_used() == n
+""", VBM3D_EST_BUDGET_MB="1")

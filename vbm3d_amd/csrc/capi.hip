@@ -1434,6 +1434,15 @@ hipError_t ctx_multiscale_buffer(vbm3d_ctx* c, size_t bytes, void** p) {
     *p = c->msbuf.p;
     return e;
 }
+// Frees the multiscale buffer and the pyramid workspace where together they
+// exceed `keep` bytes.  Nothing may be running on them.
+void ctx_multiscale_trim(vbm3d_ctx* c, size_t keep) {
+    if (c->msbuf.cap + c->pyr.cap <= keep) return;
+    for (DevBuf* b : {&c->msbuf, &c->pyr}) {
+        if (b->p) (void)hipFree(b->p);
+        *b = DevBuf{};
+    }
+}
 rocblas_handle ctx_blas(vbm3d_ctx* c) {
     if (!c->blas) {
         if (rocblas_create_handle(&c->blas) != rocblas_status_success) {

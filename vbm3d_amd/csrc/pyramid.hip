@@ -33,6 +33,7 @@ hipStream_t ctx_stream(vbm3d_ctx* c);
 int ctx_device(vbm3d_ctx* c);
 hipError_t ctx_pyr_workspace(vbm3d_ctx* c, size_t bytes, void** p);
 hipError_t ctx_multiscale_buffer(vbm3d_ctx* c, size_t bytes, void** p);
+void ctx_multiscale_trim(vbm3d_ctx* c, size_t keep);
 rocblas_handle ctx_blas(vbm3d_ctx* c);
 int ctx_fail(int code, const std::string& msg);
 }  // namespace vb
@@ -43,6 +44,12 @@ namespace {
 constexpr int BX = 64, BY = 4;
 constexpr int kMaxPyrTaps = 32;
 constexpr size_t kPyrBatchBytes = (size_t)1 << 30;  // workspace bound of a batch of frames
+// Bytes of multiscale denoising's buffers (about 4.7 clips and the batch's
+// workspace) that a context keeps for its next call; larger ones are freed at
+// the call's end, where allocating them again is small beside the call (20 RGB
+// frames 1280x720: 96.7 -> 97.4 ms; 30 grey frames 640x480, 0.57 GB, would take
+// 17.8 ms instead of 16.9).
+constexpr size_t kMultiscaleKeep = (size_t)1 << 30;
 
 struct PTaps {
     float k[kMaxPyrTaps];
@@ -490,6 +497,79 @@ struct Dev {
     }
 };
 
+// Multiscale denoising on the context's buffers (vbm3d_multiscale_denoise).
+int multiscale_denoise(vbm3d_ctx* ctx, float sigma, const float* noisy, unsigned W, unsigned H, unsigned F,
+                       unsigned C, const vbm3d_params* p1, const vbm3d_params* p2, int levels, int type,
+                       float factor, int color_space, int ref_grid_nb, float* denoised, float* noisy_levels,
+                       float* denoised_levels) {
+    int rc = check_image((int)H, (int)W, (int)C, levels, type);
+    if (rc) return rc;
+    if (!noisy || !denoised || F == 0) return ctx_fail(VBM3D_ERR_ARG, "null buffer or empty video");
+    if (!(sigma > 0.f)) return ctx_fail(VBM3D_ERR_ARG, "sigma must be positive");
+    // frames that go through the pyramid together: as many as a workspace of
+    // kPyrBatchBytes holds (planes are a grid dimension: at most 65535)
+    const size_t frame_bytes = pyr_bytes((int)H, (int)W, (int)C);
+    const int batch = (int)std::max<size_t>(
+        1, std::min<size_t>(std::min<size_t>(F, 65535 / C), kPyrBatchBytes / std::max<size_t>(frame_bytes, 1)));
+    Pyr P;
+    if ((rc = pyr_open(ctx, P, pyr_bytes((int)H, (int)W, (int)C * batch)))) return rc;
+    std::vector<int> lr, lc;
+    level_sizes((int)H, (int)W, levels, lr, lc);
+    const size_t fw = (size_t)C * H * W, flev = level_words((int)H, (int)W, (int)C, levels);
+    // the video, its levels (noisy and denoised: per level [F][C][h][w],
+    // level after level) and a basic estimate
+    void* base = nullptr;
+    if (ctx_multiscale_buffer(ctx, (2 * fw + 2 * flev) * F * 4, &base) != hipSuccess)
+        return ctx_fail(VBM3D_ERR_NOMEM, "device allocation failed");
+    float *dn = (float*)base, *dbas = dn + fw * F, *dlev = dbas + fw * F, *dden = dlev + flev * F;
+    std::vector<size_t> loff(levels);
+    size_t o = 0;
+    for (int i = 0; i < levels; i++) {
+        loff[i] = o;
+        o += (size_t)C * lr[i] * lc[i] * F;
+    }
+    PYR_TRY(hipMemcpyAsync(dn, noisy, fw * F * 4, hipMemcpyHostToDevice, P.s));
+    // 1. every frame into its levels
+    for (unsigned t = 0; t < F; t += (unsigned)batch) {
+        const int nf = (int)std::min<unsigned>((unsigned)batch, F - t);
+        if ((rc = decompose_dev(P, dn + fw * t, (int)H, (int)W, (int)C * nf, levels, type,
+                                level_ptrs(dlev, (int)H, (int)W, (int)(C * F), levels, (int)(C * t)))))
+            return rc;
+    }
+    if (noisy_levels) {
+        PYR_TRY(hipMemcpyAsync(noisy_levels, dlev, flev * F * 4, hipMemcpyDeviceToHost, P.s));
+    }
+    PYR_TRY(hipStreamSynchronize(P.s));
+    // 2. each level denoised as a video with sigma / 2^level, truncated to
+    //    two decimals as the multiscale shell script's `bc` computes it
+    //    (src/utils/VBM3Ddenoising_multiscale.sh:52-58)
+    for (int i = 0; i < levels; i++) {
+        const double sl_exact = (double)sigma / std::ldexp(1.0, i);
+        const float sl = (float)(std::floor(sl_exact * 100.0 + 1e-9) / 100.0);
+        vbm3d_params q1, q2;
+        if (p1) q1 = *p1;
+        else vbm3d_default_params_1(&q1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1.f, -1.f, (unsigned)-1, (unsigned)-1, sl);
+        if (p2) q2 = *p2;
+        else vbm3d_default_params_2(&q2, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1.f, (unsigned)-1, (unsigned)-1, sl);
+        if ((rc = vbm3d_run_device(ctx, sl, dlev + loff[i], nullptr, nullptr, (unsigned)lc[i], (unsigned)lr[i], F, C, &q1,
+                                   &q2, color_space, ref_grid_nb, dbas, dden + loff[i], nullptr)))
+            return rc;
+    }
+    if (denoised_levels) {
+        PYR_TRY(hipMemcpyAsync(denoised_levels, dden, flev * F * 4, hipMemcpyDeviceToHost, P.s));
+    }
+    // 3. every frame recomposed from its denoised levels
+    for (unsigned t = 0; t < F; t += (unsigned)batch) {
+        const int nf = (int)std::min<unsigned>((unsigned)batch, F - t);
+        if ((rc = recompose_dev(P, level_ptrs((const float*)dden, (int)H, (int)W, (int)(C * F), levels, (int)(C * t)),
+                                (int)H, (int)W, (int)C * nf, levels, type, factor, dn + fw * t)))
+            return rc;
+    }
+    PYR_TRY(hipMemcpyAsync(denoised, dn, fw * F * 4, hipMemcpyDeviceToHost, P.s));
+    PYR_TRY(hipStreamSynchronize(P.s));
+    return VBM3D_OK;
+}
+
 }  // namespace
 }  // namespace vb
 
@@ -581,72 +661,10 @@ int vbm3d_multiscale_denoise(vbm3d_ctx* ctx, float sigma, const float* noisy, un
                              unsigned C, const vbm3d_params* p1, const vbm3d_params* p2, int levels, int type,
                              float factor, int color_space, int ref_grid_nb, float* denoised, float* noisy_levels,
                              float* denoised_levels) {
-    int rc = check_image((int)H, (int)W, (int)C, levels, type);
-    if (rc) return rc;
-    if (!noisy || !denoised || F == 0) return ctx_fail(VBM3D_ERR_ARG, "null buffer or empty video");
-    if (!(sigma > 0.f)) return ctx_fail(VBM3D_ERR_ARG, "sigma must be positive");
-    // frames that go through the pyramid together: as many as a workspace of
-    // kPyrBatchBytes holds (planes are a grid dimension: at most 65535)
-    const size_t frame_bytes = pyr_bytes((int)H, (int)W, (int)C);
-    const int batch = (int)std::max<size_t>(
-        1, std::min<size_t>(std::min<size_t>(F, 65535 / C), kPyrBatchBytes / std::max<size_t>(frame_bytes, 1)));
-    Pyr P;
-    if ((rc = pyr_open(ctx, P, pyr_bytes((int)H, (int)W, (int)C * batch)))) return rc;
-    std::vector<int> lr, lc;
-    level_sizes((int)H, (int)W, levels, lr, lc);
-    const size_t fw = (size_t)C * H * W, flev = level_words((int)H, (int)W, (int)C, levels);
-    // the video, its levels (noisy and denoised: per level [F][C][h][w],
-    // level after level) and a basic estimate
-    void* base = nullptr;
-    if (ctx_multiscale_buffer(ctx, (2 * fw + 2 * flev) * F * 4, &base) != hipSuccess)
-        return ctx_fail(VBM3D_ERR_NOMEM, "device allocation failed");
-    float *dn = (float*)base, *dbas = dn + fw * F, *dlev = dbas + fw * F, *dden = dlev + flev * F;
-    std::vector<size_t> loff(levels);
-    size_t o = 0;
-    for (int i = 0; i < levels; i++) {
-        loff[i] = o;
-        o += (size_t)C * lr[i] * lc[i] * F;
-    }
-    PYR_TRY(hipMemcpyAsync(dn, noisy, fw * F * 4, hipMemcpyHostToDevice, P.s));
-    // 1. every frame into its levels
-    for (unsigned t = 0; t < F; t += (unsigned)batch) {
-        const int nf = (int)std::min<unsigned>((unsigned)batch, F - t);
-        if ((rc = decompose_dev(P, dn + fw * t, (int)H, (int)W, (int)C * nf, levels, type,
-                                level_ptrs(dlev, (int)H, (int)W, (int)(C * F), levels, (int)(C * t)))))
-            return rc;
-    }
-    if (noisy_levels) {
-        PYR_TRY(hipMemcpyAsync(noisy_levels, dlev, flev * F * 4, hipMemcpyDeviceToHost, P.s));
-    }
-    PYR_TRY(hipStreamSynchronize(P.s));
-    // 2. each level denoised as a video with sigma / 2^level, truncated to
-    //    two decimals as the multiscale shell script's `bc` computes it
-    //    (src/utils/VBM3Ddenoising_multiscale.sh:52-58)
-    for (int i = 0; i < levels; i++) {
-        const double sl_exact = (double)sigma / std::ldexp(1.0, i);
-        const float sl = (float)(std::floor(sl_exact * 100.0 + 1e-9) / 100.0);
-        vbm3d_params q1, q2;
-        if (p1) q1 = *p1;
-        else vbm3d_default_params_1(&q1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1.f, -1.f, (unsigned)-1, (unsigned)-1, sl);
-        if (p2) q2 = *p2;
-        else vbm3d_default_params_2(&q2, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1.f, (unsigned)-1, (unsigned)-1, sl);
-        if ((rc = vbm3d_run_device(ctx, sl, dlev + loff[i], nullptr, nullptr, (unsigned)lc[i], (unsigned)lr[i], F, C, &q1,
-                                   &q2, color_space, ref_grid_nb, dbas, dden + loff[i], nullptr)))
-            return rc;
-    }
-    if (denoised_levels) {
-        PYR_TRY(hipMemcpyAsync(denoised_levels, dden, flev * F * 4, hipMemcpyDeviceToHost, P.s));
-    }
-    // 3. every frame recomposed from its denoised levels
-    for (unsigned t = 0; t < F; t += (unsigned)batch) {
-        const int nf = (int)std::min<unsigned>((unsigned)batch, F - t);
-        if ((rc = recompose_dev(P, level_ptrs((const float*)dden, (int)H, (int)W, (int)(C * F), levels, (int)(C * t)),
-                                (int)H, (int)W, (int)C * nf, levels, type, factor, dn + fw * t)))
-            return rc;
-    }
-    PYR_TRY(hipMemcpyAsync(denoised, dn, fw * F * 4, hipMemcpyDeviceToHost, P.s));
-    PYR_TRY(hipStreamSynchronize(P.s));
-    return VBM3D_OK;
+    const int rc = multiscale_denoise(ctx, sigma, noisy, W, H, F, C, p1, p2, levels, type, factor, color_space, ref_grid_nb,
+                                      denoised, noisy_levels, denoised_levels);
+    if (ctx) ctx_multiscale_trim(ctx, kMultiscaleKeep);
+    return rc;
 }
 
 }  // extern "C"
