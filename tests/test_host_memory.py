@@ -61,3 +61,24 @@ n = fake.fake_used()
 V.multiscale_denoise(v[:2, :, :96, :128], 20.0, 2, ctx=small)
 assert fake.fake_used() == n
 """, VBM3D_EST_BUDGET_MB="1")
+
+
+def test_multiscale_leaves_no_copy_in_flight(fake):
+    """A call that fails at any of its launches returns with nothing of the
+    caller's video or levels still being read or written."""
+    fake("""
+v = np.zeros((3, 1, 64, 96), np.float32)
+ctx = V.Context(0)
+fake.fake_reset(1 << 40, -1)
+V.multiscale_denoise(v, 20.0, 2, return_levels=True, ctx=ctx)
+n = fake.fake_launches()
+assert n > 20 and fake.fake_in_flight() == 0
+for i in range(n):
+    fake.fake_reset(1 << 40, i)
+    try:
+        V.multiscale_denoise(v, 20.0, 2, return_levels=True, ctx=ctx)
+        failed = False
+    except V.VBM3DError:
+        failed = True
+    assert failed and fake.fake_in_flight() == 0, (i, n, failed, fake.fake_in_flight())
+""")

@@ -663,6 +663,8 @@ int vbm3d_multiscale_denoise(vbm3d_ctx* ctx, float sigma, const float* noisy, un
                              float* denoised_levels) {
     const int rc = multiscale_denoise(ctx, sigma, noisy, W, H, F, C, p1, p2, levels, type, factor, color_space, ref_grid_nb,
                                       denoised, noisy_levels, denoised_levels);
+    // a call that failed midway leaves no copy on the caller's buffers behind
+    if (rc && ctx) (void)hipStreamSynchronize(ctx_stream(ctx));
     if (ctx) ctx_multiscale_trim(ctx, kMultiscaleKeep);
     return rc;
 }
