@@ -82,3 +82,20 @@ for i in range(n):
         failed = True
     assert failed and fake.fake_in_flight() == 0, (i, n, failed, fake.fake_in_flight())
 """)
+
+
+def test_multiscale_takes_fewer_frames_where_memory_is_short(fake):
+    """40 grey frames 512x384 where the video, its levels, one frame's pyramid
+    workspace (11 MB) and the smallest rings fit, but not the workspace of all
+    frames (318 MB): the call runs, with fewer frames at a time."""
+    fake("""
+v = np.zeros((40, 1, 384, 512), np.float32)
+fake.fake_reset(600 * MB, -1)
+with V.Context(0) as ctx:
+    V.multiscale_denoise(v, 20.0, 2, ctx=ctx)
+    few = fake.fake_launches()
+fake.fake_reset(1 << 40, -1)
+with V.Context(0) as ctx:
+    V.multiscale_denoise(v, 20.0, 2, ctx=ctx)
+    assert few > fake.fake_launches()
+""", VBM3D_EST_BUDGET_MB="1")

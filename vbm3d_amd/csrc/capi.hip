@@ -1429,6 +1429,7 @@ hipError_t ctx_pyr_workspace(vbm3d_ctx* c, size_t bytes, void** p) {
     *p = c->pyr.p;
     return e;
 }
+size_t ctx_pyr_held(const vbm3d_ctx* c) { return c->pyr.cap; }
 hipError_t ctx_multiscale_buffer(vbm3d_ctx* c, size_t bytes, void** p) {
     const hipError_t e = ensure(c->msbuf, bytes);
     *p = c->msbuf.p;

@@ -34,6 +34,7 @@ int ctx_device(vbm3d_ctx* c);
 hipError_t ctx_pyr_workspace(vbm3d_ctx* c, size_t bytes, void** p);
 hipError_t ctx_multiscale_buffer(vbm3d_ctx* c, size_t bytes, void** p);
 void ctx_multiscale_trim(vbm3d_ctx* c, size_t keep);
+size_t ctx_pyr_held(const vbm3d_ctx* c);
 rocblas_handle ctx_blas(vbm3d_ctx* c);
 int ctx_fail(int code, const std::string& msg);
 }  // namespace vb
@@ -506,13 +507,8 @@ int multiscale_denoise(vbm3d_ctx* ctx, float sigma, const float* noisy, unsigned
     if (rc) return rc;
     if (!noisy || !denoised || F == 0) return ctx_fail(VBM3D_ERR_ARG, "null buffer or empty video");
     if (!(sigma > 0.f)) return ctx_fail(VBM3D_ERR_ARG, "sigma must be positive");
-    // frames that go through the pyramid together: as many as a workspace of
-    // kPyrBatchBytes holds (planes are a grid dimension: at most 65535)
-    const size_t frame_bytes = pyr_bytes((int)H, (int)W, (int)C);
-    const int batch = (int)std::max<size_t>(
-        1, std::min<size_t>(std::min<size_t>(F, 65535 / C), kPyrBatchBytes / std::max<size_t>(frame_bytes, 1)));
-    Pyr P;
-    if ((rc = pyr_open(ctx, P, pyr_bytes((int)H, (int)W, (int)C * batch)))) return rc;
+    if (!ctx) return ctx_fail(VBM3D_ERR_ARG, "null context");
+    if (hipSetDevice(ctx_device(ctx)) != hipSuccess) return ctx_fail(VBM3D_ERR_HIP, "hipSetDevice failed");
     std::vector<int> lr, lc;
     level_sizes((int)H, (int)W, levels, lr, lc);
     const size_t fw = (size_t)C * H * W, flev = level_words((int)H, (int)W, (int)C, levels);
@@ -522,6 +518,22 @@ int multiscale_denoise(vbm3d_ctx* ctx, float sigma, const float* noisy, unsigned
     if (ctx_multiscale_buffer(ctx, (2 * fw + 2 * flev) * F * 4, &base) != hipSuccess)
         return ctx_fail(VBM3D_ERR_NOMEM, "device allocation failed");
     float *dn = (float*)base, *dbas = dn + fw * F, *dlev = dbas + fw * F, *dden = dlev + flev * F;
+    // frames that go through the pyramid together: as many as a workspace of
+    // kPyrBatchBytes holds, or of 1/64 of the free memory (the denoiser's
+    // rings come out of the same), and fewer if it cannot be had, down to one
+    // (planes are a grid dimension: at most 65535)
+    size_t room = 0, total = 0;
+    if (hipMemGetInfo(&room, &total) != hipSuccess) room = 0;
+    room = std::min(kPyrBatchBytes, std::max(room / 64, ctx_pyr_held(ctx)));
+    const size_t frame_bytes = pyr_bytes((int)H, (int)W, (int)C);
+    int batch = (int)std::max<size_t>(
+        1, std::min<size_t>(std::min<size_t>(F, 65535 / C), room / std::max<size_t>(frame_bytes, 1)));
+    Pyr P;
+    while ((rc = pyr_open(ctx, P, pyr_bytes((int)H, (int)W, (int)C * batch))) == VBM3D_ERR_NOMEM && batch > 1) {
+        batch = (batch + 1) / 2;
+        (void)hipGetLastError();  // the failed allocation's
+    }
+    if (rc) return rc;
     std::vector<size_t> loff(levels);
     size_t o = 0;
     for (int i = 0; i < levels; i++) {
