@@ -64,3 +64,22 @@ def test_unpadded_members(oracle):
     ob, of, _ = oracle.run_vbm3d(sigma, noisy, p1, p2, True, 1)
     np.testing.assert_array_equal(_bits(b.cpu().numpy()), _bits(ob))
     np.testing.assert_array_equal(_bits(f.cpu().numpy()), _bits(of))
+
+
+def test_unpadded_rings_under_a_small_budget(oracle, monkeypatch):
+    """A ring budget below the smallest padded ring: members unpadded, in the
+    per-clip form and in a batch."""
+    import torch
+    import vbm3d_amd as V
+    sigma = 20.0
+    _, noisy = synth.noisy_clip(45, 37, 6, 3, sigma, 43)
+    p1, p2 = V.initialize_parameters_1(sigma), V.initialize_parameters_2(sigma)
+    ob, of, _ = oracle.run_vbm3d(sigma, noisy, p1, p2, True, 1)
+    monkeypatch.setenv("VBM3D_EST_BUDGET_MB", "1")
+    with V.Context(0) as ctx:
+        basic, final = V.denoise(noisy, sigma, True, 1, p1, p2, ctx)
+        it = V.BatchItem(sigma, torch.from_numpy(noisy).to("cuda:0"), p1, p2)
+        V.run_batch([it], ctx=ctx)
+    for b, f in ((basic, final), (it.basic.cpu().numpy(), it.denoised.cpu().numpy())):
+        np.testing.assert_array_equal(_bits(b), _bits(ob))
+        np.testing.assert_array_equal(_bits(f), _bits(of))

@@ -99,3 +99,33 @@ with V.Context(0) as ctx:
     V.multiscale_denoise(v, 20.0, 2, ctx=ctx)
     assert few > fake.fake_launches()
 """, VBM3D_EST_BUDGET_MB="1")
+
+
+RINGS = """
+v = np.zeros((30, 3, 256, 256), np.float32)
+p1, p2 = V.initialize_parameters_1(20.0), V.initialize_parameters_2(20.0)
+refs = len(V.grid(256, 256, p2.k, p2.p, 16, 1)[0])
+ring = 9 * refs * p2.N * 3 * p2.k ** 2 * 4  # step 2's smallest, members unpadded: 299 MB (padded: 325)
+"""
+
+
+def test_unpadded_rings_where_memory_is_short(fake):
+    """30 RGB frames 256x256 where step 2's smallest ring fits with unpadded
+    members only."""
+    fake(RINGS + """
+fake.fake_reset(5 * v.nbytes + ring + 10 * MB, -1)
+with V.Context(0) as ctx:
+    V.denoise(v, 20.0, ctx=ctx)
+""")
+
+
+def test_unpadded_rings_of_a_batch(fake):
+    fake(RINGS + """
+from vbm3d_amd.api import Clip
+clip = (Clip * 1)(Clip(4096, 4096, 4096, None, None, 256, 256, 30, 3, 20.0, p1, p2, 1))
+cfg = V.BatchConfig(0, 0, 1, 8, 0, 0)
+fake.fake_reset(ring + 10 * MB, -1)
+with V.Context(0) as ctx:
+    rc = V.lib().vbm3d_run_batch(ctx.h, clip, 1, 1, C.byref(cfg), None)
+    assert rc == 0, V.lib().vbm3d_last_error()
+""")

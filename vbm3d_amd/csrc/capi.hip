@@ -555,11 +555,15 @@ int run_step(vbm3d_ctx* ctx, StepIO& io, hipStream_t s) {
     // the general path's members span kt frames, so the ring keeps kt - 1
     // more frames of reference patches for the aggregation
     const size_t mpos_words = gen && kt > 1 ? (size_t)N * kt : 0;
-    // the scratch array holds members unpadded, so that it takes the same clips
-    const unsigned ms = gen || ktf ? C * K2t : est_words(K, C, !g_arena);
+    const size_t budget = ring_budget(ctx, ctx->est.cap + ctx->idx.cap + ctx->nsx.cap + ctx->wgt.cap);
+    // Members are padded where the smallest ring of padded ones is within the
+    // budget; the scratch array holds them unpadded.  So what memory there is
+    // takes the same clips with padding as without.
+    const size_t least = std::min<size_t>(Fr, 1 + 2 * (size_t)p.Nf + (kt - 1)) * nrf * N * 4;
+    const bool pad = !g_arena && least * est_words(K, C, true) <= budget;
+    const unsigned ms = gen || ktf ? C * K2t : est_words(K, C, pad);
     const size_t per_frame = g_arena ? (size_t)nrf * (N * ms + N + 1 + C + mpos_words) * sizeof(float)
                                      : (size_t)nrf * N * ms * sizeof(float);
-    const size_t budget = ring_budget(ctx, ctx->est.cap + ctx->idx.cap + ctx->nsx.cap + ctx->wgt.cap);
     size_t cap_frames = std::max<size_t>(1, budget / std::max<size_t>(per_frame, 1));
     unsigned S = (unsigned)std::max<long>(1, (long)cap_frames - 2 * (long)p.Nf - (long)(kt - 1));
     if (ctx->chunk_frames) S = std::min(S, ctx->chunk_frames);
@@ -967,6 +971,7 @@ int plan_batch(vbm3d_ctx* ctx, const vbm3d_clip* clips, int n, int nb, const vbm
         if (rc) return rc;
         if (c.C == 3 && c.color_space) plan.save_bytes += (size_t)c.W * c.H * c.F * 3 * 4 * (c.p1.k == 0 ? 2 : 1);
     }
+    const size_t budget = ring_budget(ctx, ctx->b_est.cap + ctx->b_idx.cap + ctx->b_nsx.cap + ctx->b_wgt.cap);
     // host copies of grids and tables for both steps
     std::vector<uint32_t> h_refxy;
     std::vector<int> h_meta;
@@ -1008,8 +1013,12 @@ int plan_batch(vbm3d_ctx* ctx, const vbm3d_clip* clips, int n, int nb, const vbm
                     for (unsigned x : g.cols[q]) h_refxy.push_back(x | (y << 16));
             }
             m.nrf = (unsigned)(h_refxy.size() - m.refxy);
-            m.ms = est_words(m.K, m.C, true);
-            m.per_frame = (size_t)m.nrf * (m.N * m.ms * 4 + m.N * 4 + 4 + m.C * 4);
+            // padded, unless the clip's smallest ring is within the budget only without
+            for (const bool pad : {true, false}) {
+                m.ms = est_words(m.K, m.C, pad);
+                m.per_frame = (size_t)m.nrf * (m.N * m.ms * 4 + m.N * 4 + 4 + m.C * 4);
+                if (std::min<size_t>(m.Fr, 1 + 2 * p.Nf) * m.per_frame <= budget) break;
+            }
             Tabs t;
             fill_tabs(t, m.K);
             m.tab = h_tabs.size();
@@ -1019,7 +1028,6 @@ int plan_batch(vbm3d_ctx* ctx, const vbm3d_clip* clips, int n, int nb, const vbm
     // shared rings: sub-batches of members whose smallest rings fit the budget,
     // then the largest chunk that fits
     struct Sub { size_t b, e; unsigned S; };
-    const size_t budget = ring_budget(ctx, ctx->b_est.cap + ctx->b_idx.cap + ctx->b_nsx.cap + ctx->b_wgt.cap);
     std::vector<std::vector<Sub>> subs(3);
     size_t need_slots = 0, need_idx = 0, need_est = 0, need_wgt = 0;
     for (int st = 1; st <= 2; st++) {
