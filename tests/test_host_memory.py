@@ -129,3 +129,19 @@ with V.Context(0) as ctx:
     rc = V.lib().vbm3d_run_batch(ctx.h, clip, 1, 1, C.byref(cfg), None)
     assert rc == 0, V.lib().vbm3d_last_error()
 """)
+
+
+def test_uploads_of_a_step(fake):
+    """Each step of the fast kernels uploads what they read and no more:
+    tables, reference patches, crops, boxes (the general kernels: their own
+    tables and the grid positions as well, no boxes)."""
+    fake("""
+def uploads(p1, p2):
+    fake.fake_reset(1 << 40, -1)
+    ctx = V.Context(0)
+    assert V.lib().vbm3d_run_device(ctx.h, 20.0, 4096, None, None, 64, 48, 5, 1, C.byref(p1), C.byref(p2), 0, 1,
+                                    4096, 4096, None) == 0
+    return fake.fake_h2d()
+assert uploads(V.initialize_parameters_1(20.0), V.initialize_parameters_2(20.0)) == 8
+assert uploads(V.initialize_parameters_1(20.0, N=32), V.initialize_parameters_2(20.0, N=32)) == 10
+""")

@@ -439,7 +439,7 @@ struct vbm3d_ctx {
     double pix_per_cand[3] = {0, 0, 0};   // k*k*C of each step's matching
     // batched form: rings shared by the clips of a batch, the plan (job
     // arrays and queue prefixes), queue counters, and the captured graph
-    DevBuf b_idx, b_nsx, b_est, b_wgt, b_refxy, b_meta, b_gpos, b_tabs, b_box, b_plan, b_cnt, b_save;
+    DevBuf b_idx, b_nsx, b_est, b_wgt, b_refxy, b_meta, b_tabs, b_box, b_plan, b_cnt, b_save;
     hipGraph_t b_graph = nullptr;
     hipGraphExec_t b_exec = nullptr;
     std::string b_key;
@@ -511,7 +511,12 @@ int run_step(vbm3d_ctx* ctx, StepIO& io, hipStream_t s) {
     GridDef g;
     if (!build_grid(g, io.W, io.H, p.k, p.p, p.n, io.nb))
         return fail(VBM3D_ERR_ARG, "invalid reference grid for these sizes (ref_grid_nb, p, n)");
-    // frame-local ref list in (crop, row, col) order, crop metadata
+    const unsigned K = p.k, K2 = K * K, C = io.C, N = p.N;
+    const unsigned Fr = io.F - p.kt + 1;
+    const bool ktf = fast_kt_ok(p, io.W, io.H, C);     // the fast kernels' temporal forms
+    const bool gen = !fast_ok(p, io.W, io.H) && !ktf;  // the general kernels
+    // frame-local ref list in (crop, row, col) order, crop metadata, and the
+    // grid positions that the general aggregation searches
     std::vector<uint32_t> refxy;
     std::vector<int> meta;
     std::vector<uint16_t> gpos;
@@ -519,18 +524,14 @@ int run_step(vbm3d_ctx* ctx, StepIO& io, hipStream_t s) {
         meta.push_back((int)refxy.size());
         meta.push_back((int)g.rows[c].size());
         meta.push_back((int)g.cols[c].size());
-        meta.push_back((int)gpos.size());
-        for (unsigned v : g.rows[c]) gpos.push_back((uint16_t)v);
-        meta.push_back((int)gpos.size());
-        for (unsigned v : g.cols[c]) gpos.push_back((uint16_t)v);
+        for (const std::vector<unsigned>* axis : {&g.rows[c], &g.cols[c]}) {
+            meta.push_back((int)gpos.size());
+            if (gen) gpos.insert(gpos.end(), axis->begin(), axis->end());
+        }
         for (unsigned y : g.rows[c])
             for (unsigned x : g.cols[c]) refxy.push_back(x | (y << 16));
     }
     const unsigned nrf = (unsigned)refxy.size();
-    const unsigned K = p.k, K2 = K * K, C = io.C, N = p.N;
-    const unsigned Fr = io.F - p.kt + 1;
-    const bool ktf = fast_kt_ok(p, io.W, io.H, C);     // the fast kernels' temporal forms
-    const bool gen = !fast_ok(p, io.W, io.H) && !ktf;  // the general kernels
     if ((gen || ktf) && io.adjoint)
         return fail(VBM3D_ERR_UNSUPPORTED, "the step-2 adjoint runs the fast kernels' parameter sets only");
     const unsigned kt = p.kt, K2t = K2 * kt;
@@ -550,7 +551,7 @@ int run_step(vbm3d_ctx* ctx, StepIO& io, hipStream_t s) {
     if (gen || ktf) HIP_TRY(ensure(ctx->tabsg, sizeof(TabsG)));
     HIP_TRY(ensure(ctx->refxy, refxy.size() * 4));
     HIP_TRY(ensure(ctx->meta, meta.size() * 4));
-    HIP_TRY(ensure(ctx->gpos, gpos.size() * 2));
+    if (gen) HIP_TRY(ensure(ctx->gpos, gpos.size() * 2));
     // chunk size from the estimate budget; ring holds S + 2 Nf frames
     // the general path's members span kt frames, so the ring keeps kt - 1
     // more frames of reference patches for the aggregation
@@ -583,7 +584,7 @@ int run_step(vbm3d_ctx* ctx, StepIO& io, hipStream_t s) {
     if (gen || ktf) HIP_TRY(hipMemcpyAsync(ctx->tabsg.p, &tabsg, sizeof tabsg, hipMemcpyHostToDevice, s));
     HIP_TRY(hipMemcpyAsync(ctx->refxy.p, refxy.data(), refxy.size() * 4, hipMemcpyHostToDevice, s));
     HIP_TRY(hipMemcpyAsync(ctx->meta.p, meta.data(), meta.size() * 4, hipMemcpyHostToDevice, s));
-    HIP_TRY(hipMemcpyAsync(ctx->gpos.p, gpos.data(), gpos.size() * 2, hipMemcpyHostToDevice, s));
+    if (gen) HIP_TRY(hipMemcpyAsync(ctx->gpos.p, gpos.data(), gpos.size() * 2, hipMemcpyHostToDevice, s));
 
     float sig[3] = {0, 0, 0};
     sigma_rows(io.sigma, C, io.cs, sig);
@@ -645,8 +646,7 @@ int run_step(vbm3d_ctx* ctx, StepIO& io, hipStream_t s) {
     ag.est = fa.est; ag.ms = (int)ms; ag.wgt = fa.wgt; ag.tabs = fa.tabs;
     ag.R = member_reach(p, io.maxflow, io.W, io.H);
     if (!gen) {
-        // each tile's grid box per frame distance, as the kernel would
-        // search it (one load per bound instead of a chain of dependent ones)
+        // each tile's grid box per frame distance
         std::vector<int4> box;
         int R0, Rs;
         member_reach_steps(p, io.maxflow, io.W, io.H, &R0, &Rs);
@@ -927,7 +927,7 @@ struct Member {
     const vbm3d_params* p;
     unsigned K, C, N, nrf, Fr, ms = 0, ring = 0, maxflow = 0;
     size_t per_frame = 0;  // ring bytes per frame of reference patches
-    size_t refxy = 0, meta = 0, gpos = 0, tab = 0, box = 0;
+    size_t refxy = 0, meta = 0, tab = 0, box = 0;
     int ncrop = 0;
     size_t slot_base = 0, idx_base = 0, est_base = 0, wgt_base = 0;
     unsigned t_done = 0;
@@ -975,7 +975,6 @@ int plan_batch(vbm3d_ctx* ctx, const vbm3d_clip* clips, int n, int nb, const vbm
     // host copies of grids and tables for both steps
     std::vector<uint32_t> h_refxy;
     std::vector<int> h_meta;
-    std::vector<uint16_t> h_gpos;
     std::vector<Tabs> h_tabs;
     std::vector<int4> h_box;
     std::vector<std::vector<Member>> steps(3);
@@ -995,7 +994,6 @@ int plan_batch(vbm3d_ctx* ctx, const vbm3d_clip* clips, int n, int nb, const vbm
             m.maxflow = maxflow[i];
             m.refxy = h_refxy.size();
             m.meta = h_meta.size();
-            m.gpos = h_gpos.size();
             m.box = h_box.size();
             m.ncrop = (int)g.rows.size();
             int R0, Rs;
@@ -1005,10 +1003,7 @@ int plan_batch(vbm3d_ctx* ctx, const vbm3d_clip* clips, int n, int nb, const vbm
                 h_meta.push_back((int)(h_refxy.size() - m.refxy));
                 h_meta.push_back((int)g.rows[q].size());
                 h_meta.push_back((int)g.cols[q].size());
-                h_meta.push_back((int)(h_gpos.size() - m.gpos));
-                for (unsigned v : g.rows[q]) h_gpos.push_back((uint16_t)v);
-                h_meta.push_back((int)(h_gpos.size() - m.gpos));
-                for (unsigned v : g.cols[q]) h_gpos.push_back((uint16_t)v);
+                h_meta.insert(h_meta.end(), 2, 0);
                 for (unsigned y : g.rows[q])
                     for (unsigned x : g.cols[q]) h_refxy.push_back(x | (y << 16));
             }
@@ -1088,12 +1083,10 @@ int plan_batch(vbm3d_ctx* ctx, const vbm3d_clip* clips, int n, int nb, const vbm
     HIP_TRY(ensure(ctx->b_wgt, std::max<size_t>(need_wgt, 1) * 4));
     HIP_TRY(ensure(ctx->b_refxy, std::max<size_t>(h_refxy.size(), 1) * 4));
     HIP_TRY(ensure(ctx->b_meta, std::max<size_t>(h_meta.size(), 1) * 4));
-    HIP_TRY(ensure(ctx->b_gpos, std::max<size_t>(h_gpos.size(), 1) * 2));
     HIP_TRY(ensure(ctx->b_tabs, std::max<size_t>(h_tabs.size(), 1) * sizeof(Tabs)));
     HIP_TRY(ensure(ctx->b_box, std::max<size_t>(h_box.size(), 1) * sizeof(int4)));
     if (!h_refxy.empty()) HIP_TRY(hipMemcpyAsync(ctx->b_refxy.p, h_refxy.data(), h_refxy.size() * 4, hipMemcpyHostToDevice, s));
     if (!h_meta.empty()) HIP_TRY(hipMemcpyAsync(ctx->b_meta.p, h_meta.data(), h_meta.size() * 4, hipMemcpyHostToDevice, s));
-    if (!h_gpos.empty()) HIP_TRY(hipMemcpyAsync(ctx->b_gpos.p, h_gpos.data(), h_gpos.size() * 2, hipMemcpyHostToDevice, s));
     if (!h_tabs.empty()) HIP_TRY(hipMemcpyAsync(ctx->b_tabs.p, h_tabs.data(), h_tabs.size() * sizeof(Tabs), hipMemcpyHostToDevice, s));
     if (!h_box.empty()) HIP_TRY(hipMemcpyAsync(ctx->b_box.p, h_box.data(), h_box.size() * sizeof(int4), hipMemcpyHostToDevice, s));
     HIP_TRY(hipStreamSynchronize(s));  // the host vectors go out of scope
@@ -1104,7 +1097,6 @@ int plan_batch(vbm3d_ctx* ctx, const vbm3d_clip* clips, int n, int nb, const vbm
     float* d_wgt = (float*)ctx->b_wgt.p;
     const uint32_t* d_refxy = (const uint32_t*)ctx->b_refxy.p;
     const int* d_meta = (const int*)ctx->b_meta.p;
-    const uint16_t* d_gpos = (const uint16_t*)ctx->b_gpos.p;
     const Tabs* d_tabs = (const Tabs*)ctx->b_tabs.p;
     const int4* d_box = (const int4*)ctx->b_box.p;
 
@@ -1193,7 +1185,6 @@ int plan_batch(vbm3d_ctx* ctx, const vbm3d_clip* clips, int n, int nb, const vbm
                         ag.nrf = m.nrf; ag.ring = m.ring; ag.Fr = m.Fr;
                         ag.ncrop = m.ncrop;
                         ag.crop_meta = d_meta + m.meta;
-                        ag.grid_pos = d_gpos + m.gpos;
                         ag.idx = d_idx + m.idx_base;
                         ag.nsx = d_nsx + m.slot_base;
                         ag.est = d_est + m.est_base;
@@ -1410,7 +1401,7 @@ size_t step_scratch_bytes(const vbm3d_params& p, unsigned W, unsigned H, unsigne
     const size_t nbox = gen ? 0
                             : g.rows.size() * (size_t)((H + kAggTileY - 1) / kAggTileY + (W + kAggTileX - 1) / kAggTileX) *
                                   (p.Nf + 1);
-    return al(sizeof(Tabs)) + (gen || ktf ? al(sizeof(TabsG)) : 0) + al(nrf * 4) + al(g.rows.size() * 5 * 4) + al(npos * 2) +
+    return al(sizeof(Tabs)) + (gen || ktf ? al(sizeof(TabsG)) : 0) + al(nrf * 4) + al(g.rows.size() * 5 * 4) + (gen ? al(npos * 2) : 0) +
            al(nbox * sizeof(int4)) + slots * ((size_t)C * p.N * p.k * p.k * p.kt + p.N + 1 + C + mpos_words) * 4 + 4096;
 }
 
@@ -1490,7 +1481,7 @@ void vbm3d_destroy(vbm3d_ctx* c) {
     for (DevBuf* b : {&c->noisy, &c->basic, &c->den, &c->ff, &c->bf, &c->num_raw, &c->den_raw, &c->noisy_rt, &c->basic_rt,
                       &c->idx, &c->nsx, &c->nsim, &c->dist, &c->est, &c->wgt, &c->tabs,
                       &c->refxy, &c->meta, &c->gpos, &c->rlist, &c->scal, &c->stats, &c->counts,
-                      &c->b_idx, &c->b_nsx, &c->b_est, &c->b_wgt, &c->b_refxy, &c->b_meta, &c->b_gpos,
+                      &c->b_idx, &c->b_nsx, &c->b_est, &c->b_wgt, &c->b_refxy, &c->b_meta,
                       &c->b_tabs, &c->b_box, &c->b_plan, &c->b_cnt, &c->b_save, &c->tabsg, &c->mpos, &c->tv, &c->pyr, &c->msbuf,
                       &c->boxtab})
         if (b->p) (void)hipFree(b->p);

@@ -221,8 +221,10 @@ struct AArgs {
     int K, N, Nf, kt;
     unsigned nrf, ring, Fr;
     int ncrop;
-    const int* crop_meta;       // per crop: offset in frame list, nrows, ncols, rows_at, cols_at
-    const uint16_t* grid_pos;   // concatenated sorted row and column positions
+    // per crop: offset in frame list, nrows, ncols, and (k_aggregate_gen) where
+    // its rows and columns start in grid_pos
+    const int* crop_meta;
+    const uint16_t* grid_pos;   // k_aggregate_gen: concatenated sorted row and column positions
     const uint32_t* idx;
     const uint32_t* nsx;
     const float* est;
