@@ -276,3 +276,30 @@ def test_adjoint_chunked_equals_whole(monkeypatch, C, k, N, T_2D, T_3D):
         b = V.step2_adjoint(20.0, z, basic, g, p2, ctx=chunked)
     assert torch.equal(a, b)
     assert float(a.abs().max()) > 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("C,nb,flows", [(1, 4, False), (3, 2, False), (1, 1, True), (3, 4, True)])
+def test_adjoint_chunked_equals_whole_on_crops_and_with_flows(C, nb, flows):
+    """The same on tiled reference grids (several references at one position,
+    the noisy value kept where den == 0) and with flows."""
+    import torch
+    import vbm3d_amd as V
+    from vbm3d_amd import synth
+    W, H, F = 83, 70, 9
+    _, noisy = synth.noisy_clip(W, H, F, C, 20.0, 62)
+    p2 = V.initialize_parameters_2(20.0)
+    z = torch.from_numpy(noisy).to("cuda:0")
+    basic = torch.nn.functional.avg_pool2d(z, 3, 1, 1).contiguous()
+    g = torch.from_numpy(np.random.default_rng(8).standard_normal(noisy.shape).astype(np.float32)).to("cuda:0")
+    kw = dict(ref_grid_nb=nb)
+    if flows:
+        fl = np.random.default_rng(9).uniform(-2.5, 2.5, (F - 1, 2, H, W)).astype(np.float32)
+        kw.update(fflow_t=torch.from_numpy(fl).to("cuda:0"), bflow_t=torch.from_numpy(-fl).to("cuda:0"))
+    with V.Context(0) as whole:
+        a = V.step2_adjoint(20.0, z, basic, g, p2, ctx=whole, **kw)
+    with V.Context(0) as chunked:
+        chunked.set_chunk_frames(2)
+        b = V.step2_adjoint(20.0, z, basic, g, p2, ctx=chunked, **kw)
+    assert torch.equal(a, b)
+    assert float(a.abs().max()) > 0

@@ -174,3 +174,18 @@ def test_multiscale_frames_in_several_batches(gpu_ctx):
             np.testing.assert_allclose(g[t], o, rtol=0, atol=1e-3)
         np.testing.assert_allclose(out[t], V.pyr_recompose([d[t] for d in dlev], factor=0.7, ctx=gpu_ctx), rtol=0,
                                    atol=1e-3)
+
+
+@pytest.mark.parametrize("type_", [1, 2], ids=["gauss", "lanczos"])
+def test_convolution_pyramids_in_several_batches(gpu_ctx, type_):
+    """The Gaussian and Lanczos pyramids take several frames at once too: on
+    both sides of a batch's seam, bit for bit the single-image entries."""
+    import vbm3d_amd as V
+    from vbm3d_amd import synth
+    F, W, H = 21, 1023, 1024
+    _, noisy = synth.noisy_clip(W, H, F, 1, 20.0, 52)
+    out, nlev, dlev = V.multiscale_denoise(noisy, 20.0, levels=2, type_=type_, return_levels=True, ctx=gpu_ctx)
+    for t in (0, 1, 17, 18, 20):
+        for g, o in zip(nlev, V.pyr_decompose(noisy[t], 2, type_, ctx=gpu_ctx)):
+            assert bits_equal(g[t], o)
+        assert bits_equal(out[t], V.pyr_recompose([d[t] for d in dlev], type_, 0.7, ctx=gpu_ctx))
