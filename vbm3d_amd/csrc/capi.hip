@@ -294,7 +294,10 @@ bool fast_ok(const vbm3d_params& p, unsigned W, unsigned H) {
 // kt > 1 slices at one position (no motion-compensated trajectories), the
 // paired matching's shapes, and the filter's working set in LDS.  They take
 // every set they can: 8 RGB frames 320x240 at kt 2 run in 3.5 ms, on the
-// general kernels in 17.0.
+// general kernels in 17.0, and the filter, whose wavefronts on a CU the working
+// set decides, still wins at its largest sets (320x240x8, step 2: k 8 RGB kt 2
+// N 16, 44 KB a wavefront, 5.15 -> 3.09 ms; k 8 RGB kt 3 N 12, 50 KB, 7.20 ->
+// 3.53; k 8 grey kt 4 N 16, 52 KB, 4.88 -> 1.34).
 bool fast_kt_ok(const vbm3d_params& p, unsigned W, unsigned H, unsigned C) {
     if (p.kt < 2 || p.kt > (unsigned)kGenMaxKt || p.mc) return false;
     vbm3d_params q = p;
@@ -1633,10 +1636,12 @@ int vbm3d_run(vbm3d_ctx* ctx, float sigma, float* noisy, const float* fflow, con
     for (hipEvent_t& e : ctx->ready)
         if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     // Step 2 in chunks where copying the result takes a while (clips of 16 MB
-    // and more): six of them, of at least 8 frames, so that only the last
+    // and more): at most six, of at least 8 frames, so that only the last
     // one's frames are copied after the kernels.  (Against one chunk: 20 RGB
     // frames 960x540 35.5 -> 33.5 ms, 30 at 1920x1080 203 -> 190, 20 grey
-    // frames 640x360 6.5 -> 5.8.)
+    // frames 640x360 6.5 -> 5.8, into buffers the process has written before.
+    // Into fresh ones the copies, which then take the page faults, outlast the
+    // kernels either way: 38.6 and 38.6 ms for the first.)
     std::vector<std::pair<unsigned, hipEvent_t>> pieces;
     const EarlyOut eo{rt ? (float*)ctx->noisy_rt.p : nullptr, rt ? (float*)ctx->basic_rt.p : nullptr,
                       ctx->ready[0], ctx->ready[1], n * 4 >= ((size_t)16 << 20) ? std::max(8u, (F + 5) / 6) : 0u,

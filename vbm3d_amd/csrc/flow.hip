@@ -4,12 +4,12 @@
 //
 // The pyramid runs as element-wise and stencil kernels over [ny][nx] float
 // planes in HBM, one thread per pixel; the primal-dual iterations run
-// several per launch on regions held in registers and LDS.  Every kernel evaluates the reference's expressions in its order
-// and precision -- float where it stores float, double where its
-// expressions promote (Gaussian taps and sums, bicubic cells, the
-// normalisation, 1.0 + taut * |grad|) -- with no FMA contraction and
-// IEEE-correct division and square root, so each pixel's value is the
-// reference's sequential value.  The one reduction, the mean squared
+// several per launch on regions held in registers and LDS.  Every kernel
+// evaluates the reference's expressions in its order and precision -- float
+// where it stores float, double where its expressions promote (Gaussian taps
+// and sums, bicubic cells, the normalisation, 1.0 + taut * |grad|) -- with no
+// FMA contraction and IEEE-correct division and square root, so each pixel's
+// value is the reference's sequential value.  The one reduction, the mean squared
 // change that stops the iterations, is summed in double in a fixed order;
 // the reference sums it in float, which can only move the stopping
 // iteration when the two sums straddle epsilon^2.
@@ -204,8 +204,8 @@ __global__ void k_gauss_cols(const float* __restrict__ in, float* out, int nx, i
 }
 
 // ---- bicubic resampling of a level (zoom.c:44-117): output (j1, i1)
-// samples the input at (j1 / fx, i1 / fy); flows are then multiplied by
-// `scale` (the 1 / zfactor of tvl1flow_lib.c:453-457).
+// samples the input at (j1 / fx, i1 / fy); k_upsample then multiplies a flow
+// by the 1 / zfactor of tvl1flow_lib.c:453-457.
 __global__ void k_resample(const float* __restrict__ in, float* out, int nx, int ny, int nxx, int nyy, float fx,
                            float fy) {
     const int j1 = blockIdx.x * BX + threadIdx.x, i1 = blockIdx.y * BY + threadIdx.y;
@@ -216,8 +216,8 @@ __global__ void k_resample(const float* __restrict__ in, float* out, int nx, int
     out[(size_t)i1 * nxx + j1] = interp(in, nx, n);
 }
 
-// Both components of a flow: from `a` or, at a solved level (ctl not null),
-// from the state that holds it
+// Both components of a flow, multiplied by `scale`: from state s0 or, at a
+// solved level (ctl not null), from the state that holds it
 __global__ void k_upsample(const FlowCtl* __restrict__ ctl, FlowState s0, FlowState s1, float* o1, float* o2, int nx,
                            int ny, int nxx, int nyy, float fx, float fy, float scale) {
     const int j1 = blockIdx.x * BX + threadIdx.x, i1 = blockIdx.y * BY + threadIdx.y;

@@ -29,13 +29,13 @@ namespace {
 // reference patch, whose rows arrive in scalar registers, in the reference's
 // (c, y, x) order.
 //
-// What bounds it: vector instruction issue, 84 % busy at 3,690 instructions
-// per 7x7 RGB patch of which 2,360 are the distances' separately rounded
-// subtractions, multiplications and additions; then the chain of dependent
-// steps per frame pair (copies, slot list, passes, two selections), which
-// the wavefronts of a SIMD hide from each other.  30 RGB frames 960x540,
-// step 2: 13.2 ms at 4,318 instructions and four wavefronts per SIMD, 12.6
-// at 3,690, 11.4 with a fifth wavefront.
+// What bounds it: vector instruction issue, 95 % busy at 3,768 instructions
+// per 7x7 RGB patch (60 frames 1920x1080) of which 2,360 are the distances'
+// separately rounded subtractions, multiplications and additions; then the
+// chain of dependent steps per frame pair (copies, slot list, passes, two
+// selections), which the wavefronts of a SIMD hide from each other.  30 RGB
+// frames 960x540, step 2: 13.2 ms at 4,318 instructions and four wavefronts
+// per SIMD, 12.6 at 3,690 (84 % busy), 11.4 with a fifth wavefront.
 // ---------------------------------------------------------------------
 // KT: temporal patches (a.kt > 1 slices, at one position in consecutive
 // frames; the paired form only): each slice of the windows goes through the

@@ -326,26 +326,6 @@ __device__ __forceinline__ void dct_fwd_pass(const float* x, float* y, const TAB
     }
 }
 
-// Output v of dct_fwd_pass on x[0], x[stride], ... (the same folding and
-// the same order of operations, so the two agree bit for bit).
-template <int K, class TAB>
-__device__ __forceinline__ float dct_fwd_one(const float* x, int stride, int v, const TAB* F) {
-    constexpr int H = K / 2;
-    static_assert(H >= 1, "a pass of at least two samples");
-    float m;
-    if ((v & 1) == 0) {
-        m = (x[0] + x[(K - 1) * stride]) * F[v * K];
-#pragma unroll
-        for (int q = 1; q < H; q++) m = m + (x[q * stride] + x[(K - 1 - q) * stride]) * F[v * K + q];
-        if (K & 1) m = m + x[H * stride] * F[v * K + H];
-    } else {
-        m = (x[0] - x[(K - 1) * stride]) * F[v * K];
-#pragma unroll
-        for (int q = 1; q < H; q++) m = m + (x[q * stride] - x[(K - 1 - q) * stride]) * F[v * K + q];
-    }
-    return m;
-}
-
 // One 1D pass of REDFT01 (I[o][i] = table[o*K + i], K >= 2): rows o and
 // K-1-o differ only in the sign of the odd-i terms, so E (even i) and O
 // (odd i) give y[o] = E + O and y[K-1-o] = E - O; the centre row of odd K

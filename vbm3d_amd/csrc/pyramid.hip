@@ -233,8 +233,9 @@ PTaps down_taps(bool lanczos) {
             return ctx_fail(VBM3D_ERR_HIP, std::string(#expr) + ": " + rocblas_status_to_string(s_)); \
     } while (0)
 
-// The device work of the pyramid entries: a context's stream and BLAS
-// handle, a scratch arena, and the DCT matrices of the sizes in use.
+// The device work of the pyramid entries: a context, its stream, and an arena
+// in the context's workspace (planes, and the DCT matrices of the call at
+// hand, which every dct2 forms anew).
 struct Pyr {
     vbm3d_ctx* ctx;
     hipStream_t s;
