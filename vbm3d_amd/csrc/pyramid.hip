@@ -522,13 +522,18 @@ int multiscale_denoise(vbm3d_ctx* ctx, float sigma, const float* noisy, unsigned
     // frames that go through the pyramid together: as many as a workspace of
     // kPyrBatchBytes holds, or of 1/64 of the free memory (the denoiser's
     // rings come out of the same), and fewer if it cannot be had, down to one
-    // (planes are a grid dimension: at most 65535)
-    size_t room = 0, total = 0;
-    if (hipMemGetInfo(&room, &total) != hipSuccess) room = 0;
-    room = std::min(kPyrBatchBytes, std::max(room / 64, ctx_pyr_held(ctx)));
+    // (planes are a grid dimension: at most 65535).  The free memory is asked
+    // for only where the context's workspace is too small.
     const size_t frame_bytes = pyr_bytes((int)H, (int)W, (int)C);
-    int batch = (int)std::max<size_t>(
-        1, std::min<size_t>(std::min<size_t>(F, 65535 / C), room / std::max<size_t>(frame_bytes, 1)));
+    auto frames_in = [&](size_t room) {
+        return (int)std::max<size_t>(1, std::min<size_t>(std::min<size_t>(F, 65535 / C), room / frame_bytes));
+    };
+    int batch = frames_in(kPyrBatchBytes);
+    if (pyr_bytes((int)H, (int)W, (int)C * batch) > ctx_pyr_held(ctx)) {
+        size_t room = 0, total = 0;
+        if (hipMemGetInfo(&room, &total) != hipSuccess) room = 0;
+        batch = frames_in(std::min(kPyrBatchBytes, std::max(room / 64, ctx_pyr_held(ctx))));
+    }
     Pyr P;
     while ((rc = pyr_open(ctx, P, pyr_bytes((int)H, (int)W, (int)C * batch))) == VBM3D_ERR_NOMEM && batch > 1) {
         batch = (batch + 1) / 2;
