@@ -29,7 +29,7 @@ namespace {
 // reference patch, whose rows arrive in scalar registers, in the reference's
 // (c, y, x) order.
 //
-// What bounds it: vector instruction issue, 95 % busy at 3,768 instructions
+// What bounds it: vector instruction issue, 95 % busy at 3,782 instructions
 // per 7x7 RGB patch (60 frames 1920x1080) of which 2,360 are the distances'
 // separately rounded subtractions, multiplications and additions; then the
 // chain of dependent steps per frame pair (copies, slot list, passes, two
